@@ -224,13 +224,13 @@ GCG_API size_t gcg_bwd_workspace_bytes(int64_t bs, int64_t L, int32_t g, int32_t
     const int a = resolve_algo(algo, dtype, dm, true);
     size_t n = 0;
     switch (a) {
-    case GCG_ALGO_DIRECT: n = gcg::direct_bwd_workspace(dm); break;
+    case GCG_ALGO_DIRECT: n = gcg::direct_bwd_workspace(dtype, dm); break;
     case GCG_ALGO_WINDOW: n = gcg::window_bwd_workspace(dm); break;
     case GCG_ALGO_MFMA:   n = gcg::mfma_bwd_workspace(dtype, dm); break;
     default: return 0;
     }
     // under AUTO a misaligned tensor reroutes to the direct kernels: size for both
-    if (algo == GCG_ALGO_AUTO && gcg::direct_bwd_workspace(dm) > n) n = gcg::direct_bwd_workspace(dm);
+    if (algo == GCG_ALGO_AUTO && gcg::direct_bwd_workspace(dtype, dm) > n) n = gcg::direct_bwd_workspace(dtype, dm);
     return (n + 255) & ~(size_t)255;
 }
 

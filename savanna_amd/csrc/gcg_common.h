@@ -280,12 +280,12 @@ KernelTimer take_kernel_timer();
 // neither reported as this library's nor cleared from under its owner.
 template <typename... KArgs, size_t... I>
 inline int launch_packed(const void *fn, dim3 grid, dim3 block, hipStream_t st, const KernelTimer &t,
-                         std::tuple<KArgs...> &vals, std::index_sequence<I...>)
+                         std::tuple<KArgs...> &vals, std::index_sequence<I...>, size_t lds = 0)
 {
     void *ptrs[] = {(void *)&std::get<I>(vals)...};
     if (t.start && t.stop)
-        return (int)hipExtLaunchKernel(fn, grid, block, ptrs, 0, st, t.start, t.stop, 0);
-    return (int)hipLaunchKernel(fn, grid, block, ptrs, 0, st);
+        return (int)hipExtLaunchKernel(fn, grid, block, ptrs, lds, st, t.start, t.stop, 0);
+    return (int)hipLaunchKernel(fn, grid, block, ptrs, lds, st);
 }
 
 // a small kernel beside the main one (reductions, filter generation): never timed
@@ -306,12 +306,29 @@ inline int launch_main(void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStrea
                          std::index_sequence_for<KArgs...>{});
 }
 
+// the same with `lds` bytes of dynamic LDS
+template <typename... KArgs, typename... Args>
+inline int launch_main_lds(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds, hipStream_t st, Args... args)
+{
+    std::tuple<KArgs...> vals{static_cast<KArgs>(args)...};
+    return launch_packed((const void *)kernel, grid, block, st, take_kernel_timer(), vals,
+                         std::index_sequence_for<KArgs...>{}, lds);
+}
+
 int direct_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h,
                       void *y, void *y2, void *bx, const Dims &dm, hipStream_t st);
-size_t direct_bwd_workspace(const Dims &dm);
+size_t direct_bwd_workspace(int dtype, const Dims &dm);
 int direct_bwd_launch(int dtype, const void *dy, const void *x, const void *B, const void *C,
                       const void *h, void *dx, void *dB, void *dC, void *dh, void *ws,
                       const Dims &dm, hipStream_t st);
+
+// matrix-core kernels of the general family: filters of 9 to 256 taps, any group width and element alignment
+bool toep_supported(int dtype, const Dims &dm, bool backward);
+int toep_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
+                    const Dims &dm, hipStream_t st);
+size_t toep_bwd_workspace(int dtype, const Dims &dm);
+int toep_bwd_launch(int dtype, const void *dy, const void *x, const void *B, const void *C, const void *h, void *dx,
+                    void *dB, void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st);
 
 bool window_supported(const Dims &dm);
 int window_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h,

@@ -5,7 +5,8 @@
 // consecutive time rows and walks the taps in blocks of 16, holding 16 taps and a
 // 31-sample window in registers so that a block costs 47 LDS reads for 256 FMAs.
 // This is the fallback for shapes the MFMA and register-window kernels do not take (filters
-// longer than 128 taps, narrow or odd group widths, misaligned tensors).
+// longer than 128 taps, narrow or odd group widths, misaligned tensors); of those, 9 to 256 taps go to the
+// matrix-core kernels of gcg_toep.hip, so what runs here are odd shapes of at most 8 taps and filters beyond 256.
 #include "gcg_common.h"
 
 namespace gcg {
@@ -314,6 +315,7 @@ int bwd_t(const void *dy, const void *x, const void *B, const void *C, const voi
 int direct_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h, void *y,
                       void *y2, void *bx, const Dims &dm, hipStream_t st)
 {
+    if (toep_supported(dtype, dm, false)) return toep_fwd_launch(dtype, x, B, C, h, y, y2, bx, dm, st);
     switch (dtype) {
     case GCG_F32:  return fwd_t<float>(x, B, C, h, y, y2, bx, dm, st);
     case GCG_BF16: return fwd_t<bf16_t>(x, B, C, h, y, y2, bx, dm, st);
@@ -324,8 +326,9 @@ int direct_fwd_launch(int dtype, const void *x, const void *B, const void *C, co
     return (int)hipErrorInvalidValue;
 }
 
-size_t direct_bwd_workspace(const Dims &dm)
+size_t direct_bwd_workspace(int dtype, const Dims &dm)
 {
+    if (toep_supported(dtype, dm, true)) return toep_bwd_workspace(dtype, dm);
     const BwdPlan p = plan_bwd(dm);
     return (size_t)p.nwg * p.gpt * dm.hl * sizeof(float);
 }
@@ -333,6 +336,7 @@ size_t direct_bwd_workspace(const Dims &dm)
 int direct_bwd_launch(int dtype, const void *dy, const void *x, const void *B, const void *C, const void *h,
                       void *dx, void *dB, void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st)
 {
+    if (toep_supported(dtype, dm, true)) return toep_bwd_launch(dtype, dy, x, B, C, h, dx, dB, dC, dh, ws, dm, st);
     switch (dtype) {
     case GCG_F32:  return bwd_t<float>(dy, x, B, C, h, dx, dB, dC, dh, ws, dm, st);
     case GCG_BF16: return bwd_t<bf16_t>(dy, x, B, C, h, dx, dB, dC, dh, ws, dm, st);
