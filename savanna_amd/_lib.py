@@ -206,6 +206,18 @@ class _on_device:
         return False
 
 
+def _run(op, *args):
+    """A torch.ops.gcg forward operator that writes none of its arguments.  With gradient recording off -- inference,
+    and inside the autograd functions of the layers above -- the autograd formula these operators have, a Python
+    function each (_ops.py), would only hand the call on; it is passed by then.  1 x 2048 x 256 fp32 forward of 7 taps,
+    a call whose kernel takes 4.5 us: 19.0 us with it, 15.4 without.  Not under torch.compile or a function transform,
+    which have layers of their own; the backward operators have no formula and gain nothing (9.8 -> 10.5 us)."""
+    if torch.is_grad_enabled() or torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active():
+        return op(*args)
+    with torch._C._AutoDispatchBelowAutograd():
+        return op(*args)
+
+
 def _require_gpu(t: torch.Tensor) -> None:
     if not t.is_cuda:
         raise RuntimeError(
@@ -227,8 +239,8 @@ def fwd(x, B, C, h, return_bx=False, return_y2=False, algo=ALGO_AUTO, out=None):
             torch.ops.gcg.fwd_out(x, B, C, h, out, a)
             return None, None, out
         if not (return_bx or return_y2):
-            return None, None, torch.ops.gcg.fwd(x, B, C, h, a)
-        bx, y2, y = torch.ops.gcg.fwd_full(x, B, C, h, return_bx, return_y2, a)
+            return None, None, _run(torch.ops.gcg.fwd, x, B, C, h, a)
+        bx, y2, y = _run(torch.ops.gcg.fwd_full, x, B, C, h, return_bx, return_y2, a)
         if out is not None:
             y = out.copy_(y)
         return (bx if return_bx else None), (y2 if return_y2 else None), y
@@ -329,7 +341,7 @@ def fwd_interleaved(feat, h, algo=ALGO_AUTO, out=None):
     """y (bs, L, g, dg) for feat (bs, L, g, dg, 3) with feat[..., 0] = C, [..., 1] = B, [..., 2] = x."""
     _require_gpu(feat)
     if TORCH_OPS and out is None:
-        return torch.ops.gcg.fwd_interleaved(feat, h, algo_code(algo))
+        return _run(torch.ops.gcg.fwd_interleaved, feat, h, algo_code(algo))
     lib = load()
     _check_feat(feat, h)
     bs, L, g, dg, _ = feat.shape
@@ -397,7 +409,7 @@ def fwd_planar(feat, h, algo=ALGO_AUTO):
     the thirds of each row read in place (block.py:881-884, the split without interleaving)."""
     _require_gpu(feat)
     if TORCH_OPS:
-        return torch.ops.gcg.fwd_planar(feat, h, algo_code(algo))
+        return _run(torch.ops.gcg.fwd_planar, feat, h, algo_code(algo))
     lib = load()
     _check_planar(feat, h)
     bs, L, _, g, dg = feat.shape
@@ -452,7 +464,7 @@ def dwconv_fwd(x, w, keep_output=False):
     ``keep_output``: y goes to fwd_interleaved next, store it through the cache."""
     _require_gpu(x)
     if TORCH_OPS:
-        return torch.ops.gcg.dwconv_fwd(x, w, bool(keep_output))
+        return _run(torch.ops.gcg.dwconv_fwd, x, w, bool(keep_output))
     lib = load()
     _check_dwconv(x, w)
     bs, L, g, dg = x.shape
@@ -513,7 +525,7 @@ def mixer_se_fwd(raw, wf, h, planar=False):
     ``planar``: raw is (bs, L, 3, g, dg), the split without interleaving (block.py:881-884)."""
     _require_gpu(raw)
     if TORCH_OPS:
-        return torch.ops.gcg.mixer_se_fwd(raw, wf, h, bool(planar))
+        return _run(torch.ops.gcg.mixer_se_fwd, raw, wf, h, bool(planar))
     lib = load()
     _check_mixer_se(raw, wf, h, planar)
     bs, L = raw.shape[:2]
@@ -571,7 +583,7 @@ def filter_decay_fwd(w, decay, hl: int, dtype: torch.dtype):
     """h (g, 1, hl) in ``dtype`` = w[:, :hl] * decay[:, :hl]."""
     _require_gpu(w)
     if TORCH_OPS:
-        return torch.ops.gcg.filter_decay_fwd(w, decay, hl, dtype)
+        return _run(torch.ops.gcg.filter_decay_fwd, w, decay, hl, dtype)
     lib = load()
     _check_filter_params(w, decay)
     g, l_cache = w.shape
@@ -668,7 +680,7 @@ def mixer_mr_fwd(raw, wf, h, planar=False):
     ``planar``: raw is (bs, L, 3, g, dg), the split without interleaving (block.py:881-884); 16-bit arithmetic only."""
     _require_gpu(raw)
     if TORCH_OPS:
-        return torch.ops.gcg.mixer_mr_fwd(raw, wf, h, bool(planar))
+        return _run(torch.ops.gcg.mixer_mr_fwd, raw, wf, h, bool(planar))
     lib = load()
     _check_mixer_mr(raw, wf, h, planar)
     bs, L = raw.shape[:2]
@@ -726,7 +738,7 @@ def mixer_mr_fwd_decay(raw, wf, w, decay, hl: int, filt: torch.dtype, planar=Fal
     """mixer_mr_fwd with the filter F(w * decay)[:, :hl] formed inside the kernel (w, decay: (g, l_cache) fp32)."""
     _require_gpu(raw)
     if TORCH_OPS:
-        return torch.ops.gcg.mixer_mr_fwd_decay(raw, wf, w, decay, hl, filt, bool(planar))
+        return _run(torch.ops.gcg.mixer_mr_fwd_decay, raw, wf, w, decay, hl, filt, bool(planar))
     lib = load()
     _check_filter_params(w, decay)
     bs, L = raw.shape[:2]
@@ -795,7 +807,7 @@ def fwd_time_major(x, B, C, h):
     """y (bs, seqlen, g, dg) for x, B, C of shape (seqlen, bs, g, dg), read where they lie."""
     _require_gpu(x)
     if TORCH_OPS:
-        return torch.ops.gcg.fwd_time_major(x, B, C, h)
+        return _run(torch.ops.gcg.fwd_time_major, x, B, C, h)
     lib = load()
     L, bs, g, dg = x.shape
     y = torch.empty(bs, L, g, dg, dtype=x.dtype, device=x.device)
@@ -859,7 +871,7 @@ def fwd_decay(x, B, C, w, decay, hl: int, filt: torch.dtype):
     """gcg_fwd with h = filt(w[:, :hl] * decay[:, :hl]) formed inside the kernel; w, decay: (g, L_cache) fp32."""
     _require_gpu(x)
     if TORCH_OPS:
-        return torch.ops.gcg.fwd_decay(x, B, C, w, decay, hl, filt)
+        return _run(torch.ops.gcg.fwd_decay, x, B, C, w, decay, hl, filt)
     lib = load()
     _check_filter_params(w, decay)
     bs, L, g, dg = x.shape
@@ -900,7 +912,7 @@ def bwd_decay(dy, x, B, C, w, decay, hl: int, filt: torch.dtype):
 def fwd_interleaved_decay(feat, w, decay, hl: int, filt: torch.dtype):
     _require_gpu(feat)
     if TORCH_OPS:
-        return torch.ops.gcg.fwd_interleaved_decay(feat, w, decay, hl, filt)
+        return _run(torch.ops.gcg.fwd_interleaved_decay, feat, w, decay, hl, filt)
     lib = load()
     _check_filter_params(w, decay)
     bs, L, g, dg, _ = feat.shape
