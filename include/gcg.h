@@ -364,7 +364,8 @@ GCG_API int gcg_mixer_se_bwd_planar(const void *dy, const void *raw, const void 
  * the features are made again from raw, their gradient is handed from the operator's part to the featurizer's
  * part inside the workgroup and never stored: 7 N s of memory traffic (dy and raw in, draw out) instead of the two-call
  * chain's 16 N s.  draw and dh are the chain's bit for bit (bf16), dwf up to the order in which partial sums are added.
- * Other types (fp32 arithmetic): one kernel recomputes the features and writes their gradient into dfeat_scratch
+ * GCG_BF16_F32 does the same from 1024 steps of 32 rows on (64-channel columns times batch rows times steps).
+ * Other types and smaller problems: one kernel recomputes the features and writes their gradient into dfeat_scratch
  * ((bs, L, g, dg, 3), caller's memory, contents on return unspecified), then the featurizer's own backward turns
  * it into draw and dwf -- the chain's traffic, but nothing of size 3 N is kept between forward and backward.
  * gcg_mixer_mr_bwd_scratch_bytes(...) says how large dfeat_scratch has to be: 0 (it may then be NULL) where the

@@ -749,7 +749,7 @@ GCG_API size_t gcg_mixer_mr_bwd_workspace_bytes(int64_t bs, int64_t L, int32_t g
     if (!gcg::mfma_feat_supported(dtype, dm, kf)) return 0;
     if (make_dims(bs, L, 3 * g * dg, 1, kf, plain_tensor_code(dtype), &df) || !gcg::dwconv_supported(df)) return 0;
     const size_t chain = up256(gcg::mfma_feat_bwd_workspace(dtype, dm)) + up256(gcg::dwconv_bwd_workspace(df));
-    const size_t fused = gcg::mixer_mr_fused_supported(dtype, dm, kf) ? up256(gcg::mixer_mr_fused_workspace(dm, kf)) : 0;
+    const size_t fused = gcg::mixer_mr_fused_bwd_supported(dtype, dm, kf) ? up256(gcg::mixer_mr_fused_workspace(dm, kf)) : 0;
     return chain > fused ? chain : fused;
 }
 
@@ -758,7 +758,7 @@ GCG_API size_t gcg_mixer_mr_bwd_scratch_bytes(int64_t bs, int64_t L, int32_t g, 
 {
     gcg::Dims dm;
     if (kf <= 0 || make_dims(bs, L, g, dg, hl, dtype, &dm, true)) return 0;
-    if (gcg::mixer_mr_fused_supported(dtype, dm, kf)) return 0;
+    if (gcg::mixer_mr_fused_bwd_supported(dtype, dm, kf)) return 0;
     return (size_t)(3 * bs * L * dm.d) * (dtype == GCG_F32 ? 4 : 2);
 }
 
@@ -832,7 +832,7 @@ int mixer_mr_bwd_dims(const void *dy, const void *raw, const void *wf, const voi
     int rc = 0;
     dm.es = dm.planar ? 1 : 3;
     dm.keep_out = 1;
-    const bool fused = gcg::mixer_mr_fused_supported(dtype, dm, kf);
+    const bool fused = gcg::mixer_mr_fused_bwd_supported(dtype, dm, kf);
     if (dm.planar && !fused) return GCG_ERR_UNSUPPORTED;          // one-kernel path only
     if (!fused && !dfeat_scratch) return GCG_ERR_BAD_ARG;
     if (!all_aligned16({dy, raw, draw}) || (!fused && !all_aligned16({dfeat_scratch})) ||

@@ -246,7 +246,7 @@ template <typename T, bool PL>
 __device__ __forceinline__ void mixer_bwd_finish(const float *ws, const float *wsf, T *__restrict__ dh,
                                                  T *__restrict__ dwf, const Dims &dm, const MfmaPlan &pl, int cb, int kf)
 {
-    typedef MixGeo<T> G;
+    typedef MixGeo<bf16_t> G;                   // (the same for every element type)
     if (!pl.fuse_dh) return;
     const int tid = threadIdx.x;
     if (!dh_arrive_last(pl, cb, (unsigned int)(dm.bs * pl.nseg))) return;
@@ -714,6 +714,448 @@ __global__ __launch_bounds__(MixGeo<T>::NT) void mixer_mr_bwd_kernel(const T *__
     mixer_bwd_finish<T, PL>(ws, wsf, dh, dwf, dm, pl, cb, kf);
 }
 
+// ---------------------------------------------------------------------------- backward, fp32 arithmetic
+// The same in fp32 arithmetic on bf16 tensors (the layer's default precision), on the product waves and row waves of
+// the duo kernels (gcg_mfma_tile.h: operands of two bf16 planes, one barrier per step, y2 / du tiles of two parities):
+//   row waves (4..7)      iteration s: gradient of the features of step s-1 from its y2 / du tiles -> LDS, and its d wf;
+//                         u of step s+1 and g2 of step s+NK; the filter-gradient products of step s;
+//   product waves (0..3)  iteration s: y2, du of step s, and d raw of step s-2 from the gradient rows in LDS.
+// The operand planes take the LDS that holds the raw rows in the 16-bit kernel, so a raw row is requested three times
+// -- five steps ahead for C (8 of a piece's 12 bytes), one step ahead for x and B, and with its gradient for d wf --
+// and all but the first are answered by the caches: a step's rows are 12 KB per workgroup, and those of six steps of
+// the 32 workgroups of an XCD are 2.4 MB of its 4 MB L2.  dy waits for its step in a lane-private ring in LDS.
+// A run goes one step beyond its end for the gradient rows that its last two rows of d raw need, and two iterations
+// further for the hand-overs; what these compute beyond the run is dropped by the windows or not accumulated.
+//
+// What bounds it: instruction issue (87 matrix instructions per 16 channels and step, and the vector work of both
+// kernels it replaces: 59 % of the quad-cycles issue, and a matrix instruction takes four).  7B shape (2 x 8192 x 4096),
+// bf16: 319 - 347 us, against 233 - 264 us for the operator's backward with the features made in front (gradient of the
+// features to memory) and 217 - 222 + 9 us for the featurizer's backward on it; 7 instead of 16 values moved per
+// element (454 MB read, 404 MB written).  Measured and left: d wf on the product waves (351 us), d wf with fused
+// multiply-adds on unpacked values (351), straight-line bodies for the first, middle and last steps (spills, 590).
+struct WideGeo {
+    typedef bf16w_t T;
+    typedef DuoGeo<T> D;
+    typedef MixGeo<bf16_t> X;                    // the lane layout of rows and gradient rows is the 16-bit kernel's
+    static constexpr int NW = D::NW, NT = 128 * NW, CB = 16 * NW, ND = D::ND, RSLOTS = D::RSLOTS;
+    static constexpr int LPR = X::LPR, NR = X::NR, NG = X::NG, NH = X::NH, BLK = X::BLK, PRE = X::PRE, PRE_BYTES = X::PRE_BYTES;
+    static constexpr int DQ_VEC = 64 * NW * 16;                  // dy of one step: a row vector per row-wave lane
+    static constexpr int OFF_DQ = D::OFF_H;                      // over the filter tables, dead by then
+    static constexpr int OFF_DF = OFF_DQ + RSLOTS * DQ_VEC;      // gradient rows of two steps, then three sets of a step's last NH rows
+    static constexpr int OFF_DFP = OFF_DF + 2 * PRE;
+    static constexpr int LDS_BYTES = OFF_DFP + 3 * PRE_BYTES;
+    static constexpr int OFF_P = 0;                              // tail: gradient tiles, then the d wf accumulators
+    static constexpr int OFF_W = OFF_P + NW * ND * 1024;
+    static constexpr int NACC = MR_KF * 6;
+    static_assert(CB == X::CB && NT == X::NT && NW == X::XW, "the tail is shared with the 16-bit kernel");
+    static_assert(D::H_BYTES <= RSLOTS * DQ_VEC, "filter tables fit");
+    static_assert(OFF_W + NW * 64 * NACC * 4 <= LDS_BYTES, "tail fits");
+    static_assert(LDS_BYTES <= 160 * 1024 - 64, "workgroup exceeds the 160 KB of LDS");
+    static_assert(OFF_DF % 16 == 0 && OFF_DFP % 16 == 0, "16-byte LDS accesses");
+};
+
+__device__ __forceinline__ u32x2 ldw8_cached(win_t w, uint32_t off)
+{
+    return __builtin_amdgcn_raw_buffer_load_b64(w, (int)off, 0, 0);
+}
+
+__global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
+    const bf16w_t *__restrict__ dy, const bf16w_t *__restrict__ raw, const bf16w_t *__restrict__ h,
+    const bf16w_t *__restrict__ wfeat, int kf, bf16w_t *__restrict__ draw, bf16w_t *__restrict__ dh,
+    bf16w_t *__restrict__ dwf, float *__restrict__ ws, float *__restrict__ wsf, Dims dm, MfmaPlan pl)
+{
+    typedef bf16w_t T;
+    typedef WideGeo G;
+    typedef G::D D;
+    typedef MT<T> M;
+    typedef M::op_t op_t;
+    constexpr int NK = D::NK, NW = G::NW, ND = G::ND, CB = G::CB, RSLOTS = G::RSLOTS;
+    constexpr int UROW = D::UROW, YROW = D::YROW, USZ = D::USZ, YSZ = D::YSZ;
+    constexpr int LPR = G::LPR, NR = G::NR, NH = G::NH, KF = MR_KF, NV = 6;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[G::LDS_BYTES];
+    unsigned char *const ring = smem + D::OFF_R;
+
+    const uint32_t wg_id = xcd_contiguous_u32(blockIdx.x, gridDim.x);
+    int cb, seg, bi;
+    wg_place(wg_id, pl, cb, seg, bi);
+    const int64_t b = bi;
+    const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
+    const bool row_wave = wv >= NW;
+    const int w = wv & (NW - 1);
+    const int64_t d = dm.d, L = dm.L;
+    const int64_t c0 = (int64_t)cb * CB;
+    const bool wave_valid = c0 + 16 * w < d;
+    const int64_t s_lo = (int64_t)seg * pl.steps_per_seg;
+    const int64_t s_hi = (s_lo + pl.steps_per_seg < pl.nsteps) ? s_lo + pl.steps_per_seg : pl.nsteps;
+    const int n_steps = (int)(s_hi - s_lo), n_it = n_steps + 3;      // iterations, counted from the run's first step
+
+    // Row layout, in both kinds of waves: lane (rr, a) owns rows NR*rr .. NR*rr+3 of a step and channels c0 + 2a, 2a+1.
+    const int vt = tid & (64 * NW - 1), rr = vt / LPR, a = vt % LPR;
+    const bool cvalid = c0 + 2 * a < d;
+    const uint32_t rb = (uint32_t)(d * 2), bad = cvalid ? 0u : WIN_OFF;
+    const uint32_t rb3 = __builtin_amdgcn_readfirstlane(3u * rb);
+    const uint32_t step_b3 = __builtin_amdgcn_readfirstlane((uint32_t)STEP * 3u * rb);
+    const int64_t row_bytes = d * 2;
+    const int64_t T0 = s_lo * STEP, T1 = s_hi * STEP < L ? s_hi * STEP : L;
+    const uint32_t lane_raw = 3u * ((uint32_t)(NR * rr - NH) * rb + (uint32_t)((c0 + 2 * a) * 2)) + bad;  // row NR*rr-NH of a step
+    float tap[KF][NV];
+    load_feat_taps<T, KF, NV>(wfeat, cvalid ? 3 * (c0 + 2 * a) : 0, kf, tap);
+    const int own_off = vt * G::BLK;
+    const int j = l & 15, q = l >> 4;
+
+    if (!row_wave) {
+        // -------------------------------------------------------------- product waves
+        M::hraw_t *htab = (M::hraw_t *)(smem + D::OFF_H);
+        M::hraw_t hv[HTAB / 64];
+        load_taps<T>(dm, h, wave_valid ? fdiv((uint32_t)(cb * NW + w), pl.q_dg16) : 0, l, hv);
+        op_t Au[NK], Ag[NK];
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            Au[i] = M::zero_op();
+            Ag[i] = M::zero_op();
+        }
+        const int y_wr = j * YROW + (16 * w + 4 * q) * 4;
+        const int d_wr = (15 - j) * YROW + (16 * w + 4 * q) * 4;      // columns come out reversed
+        store_taps(htab + w * HTAB, l, hv);
+        __syncthreads();                                              // (A)
+        M::wop_t W0[NK], W1[NK];
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            W0[i] = M::toeplitz(htab + w * HTAB, 32 * i, j, q);
+            W1[i] = M::toeplitz(htab + w * HTAB, 32 * i + 16, j, q);
+        }
+        __syncthreads();                                              // (A2)
+#pragma unroll
+        for (int i = 1; i < NK; ++i) {
+            __syncthreads();                                          // (B_i) lead-in tiles written
+            Au[NK - i] = M::load_operand(smem + D::OFF_U, UROW, w, j, q, false);
+            Ag[NK - 1 - i] = M::load_operand(smem + D::OFF_R + (NK - 1 - i) * USZ, UROW, w, j, q, true);
+            __syncthreads();                                          // (C_i) and read
+        }
+        __syncthreads();                                              // (D) the run's first step is prepared
+
+        const win_t wdr = make_window(draw + 3 * (b * L + T0) * d, 3 * (T1 - T0) * row_bytes);
+        uint32_t dr_b = 0u - 2u * step_b3;                            // of step s-2
+        const unsigned char *const df_own = smem + G::OFF_DF + own_off;
+        // the NH rows before the lane's own: its neighbour's last, or the last of the step before (three sets in turn)
+        const unsigned char *const df_halo = rr ? smem + G::OFF_DF + own_off - LPR * G::BLK + (NR - NH) * 12 : smem + G::OFF_DFP + a * 24;
+        uint32_t u_off = D::OFF_U, y_off = D::OFF_Y, df_off = 0;      // tiles of the step's parity
+        int g_new = NK - 1, df_last = 0;                              // ring slot of step s+NK-1; set of the rows before step s-2
+        u32x3 dro[NR];                                                // the rows of d raw stored last
+#pragma unroll
+        for (int r = 0; r < NR; ++r) dro[r] = u32x3{0u, 0u, 0u};
+        auto product_step = [&](int ph, bool live) __attribute__((always_inline)) {
+            const int slot_new = (ph + NK - 1) % NK;
+            Au[ph] = M::load_operand(smem + u_off, UROW, w, j, q, false);
+            Ag[slot_new] = M::load_operand(ring + g_new * USZ, UROW, w, j, q, true);
+            u32x3 pg[NH + NR];
+            halo_pieces(lds_load_halo(df_halo + (rr ? (int)df_off : df_last * G::PRE_BYTES)), pg);
+            blk_pieces(lds_load_blk(df_own + df_off), pg + NH);
+            f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+            f32x4 dac0 = {0.f, 0.f, 0.f, 0.f}, dac1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NK; ++i) {
+                acc0 = M::mfma(Au[(ph - i + NK) % NK], W0[i], acc0);
+                acc1 = M::mfma(Au[(ph - i + NK) % NK], W1[i], acc1);
+                dac0 = M::mfma(Ag[(ph + i) % NK], W1[i], dac0);   // output rows 0..15
+                dac1 = M::mfma(Ag[(ph + i) % NK], W0[i], dac1);   // output rows 16..31
+            }
+            unsigned char *const y_cur = smem + y_off, *const d_cur = y_cur + (D::OFF_D - D::OFF_Y);
+            *(f32x4 *)(y_cur + y_wr) = acc0;
+            *(f32x4 *)(y_cur + y_wr + 16 * YROW) = acc1;
+            *(f32x4 *)(d_cur + d_wr) = dac0;
+            *(f32x4 *)(d_cur + d_wr + 16 * YROW) = dac1;
+            // d raw of rows NR*rr-NH .. NR*rr+NR-NH-1 of step s-2: each needs the gradient rows from its own on.  (The
+            // rows stored last keep registers of their own until here: see the 16-bit kernel.)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) asm volatile("" ::"v"(dro[i][0]), "v"(dro[i][1]), "v"(dro[i][2]));
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                float lo[NH + NR], hi[NH + NR];
+#pragma unroll
+                for (int i = 0; i < NH + NR; ++i) M::unpack2(pg[i][c], lo[i], hi[i]);
+#pragma unroll
+                for (int i = 0; i < NR; ++i) {
+                    float s0 = 0.f, s1 = 0.f;                    // the featurizer backward's order: nearest row first
+#pragma unroll
+                    for (int m = KF - 1; m >= 0; --m) {
+                        s0 = fmaf(tap[m][2 * c], lo[i + KF - 1 - m], s0);
+                        s1 = fmaf(tap[m][2 * c + 1], hi[i + KF - 1 - m], s1);
+                    }
+                    dro[i][c] = M::pack2(s0, s1);
+                }
+            }
+            const uint32_t o = live ? lane_raw + dr_b : WIN_OFF;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) stw12(wdr, o + (uint32_t)i * rb3, dro[i]);
+            dr_b += step_b3;
+            u_off ^= (uint32_t)(D::OFF_U ^ (D::OFF_U + USZ));
+            y_off = y_off == D::OFF_Y ? D::OFF_Y + YSZ : D::OFF_Y;
+            df_off ^= G::PRE;
+            g_new = g_new + 1 == RSLOTS ? 0 : g_new + 1;
+            df_last = df_last == 2 ? 0 : df_last + 1;
+            __syncthreads();
+        };
+        int s = 0;
+        while (s < n_it) {
+#pragma unroll
+            for (int ph = 0; ph < NK; ++ph) {
+                if (s < n_it) {
+                    product_step(ph, s >= 2);
+                    ++s;
+                }
+            }
+        }
+        __syncthreads();                                              // (E) tiles and gradient rows are no longer in use
+        __syncthreads();                                              // (F) tail tiles written
+        // d wf: the row groups' sums, one partial row per run
+        const float *wacc = (const float *)(smem + G::OFF_W);
+        const int64_t prow = b * pl.nseg + seg, nprow = dm.bs * pl.nseg;
+        for (int idx = tid; idx < KF * LPR * NV; idx += 64 * NW) {
+            const int m = idx / (LPR * NV), col = idx % (LPR * NV);
+            const int kk = m - (KF - kf);                             // index into the kf taps of the filter
+            if (kk < 0 || 3 * c0 + col >= 3 * d) continue;
+            float sum = 0.f;
+#pragma unroll
+            for (int r = 0; r < G::NG; ++r) sum += wacc[(m * G::NG + r) * (LPR * NV) + col];
+            __hip_atomic_store(wsf + ((size_t)kk * nprow + prow) * (3 * d) + 3 * c0 + col, sum, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+    } else {
+        // -------------------------------------------------------------- row waves
+        f32x4 P[ND];
+#pragma unroll
+        for (int i = 0; i < ND; ++i) P[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // the rows read: from the NK-1 steps before the run (and the NH rows before those) to the NK-1 steps after the
+        // last step worked on, s_hi; what lies outside reads as zero
+        const int64_t t0 = (s_lo - (NK - 1)) * STEP > 0 ? (s_lo - (NK - 1)) * STEP : 0;
+        const int64_t tf = t0 - NH > 0 ? t0 - NH : 0;
+        const int64_t t2 = (s_hi + NK) * STEP < L ? (s_hi + NK) * STEP : L;
+        const win_t wraw = make_window(raw + 3 * (b * L + tf) * d, 3 * (t2 - tf) * row_bytes);
+        const win_t wdy = make_window(dy + (b * L + t0) * d, (t2 - t0) * row_bytes);
+        const uint32_t lane_dy = (uint32_t)(NR * rr) * rb + (uint32_t)((c0 + 2 * a) * 2) + bad;
+        const uint32_t step_b = __builtin_amdgcn_readfirstlane((uint32_t)STEP * rb);
+        const uint32_t lane_feat = lane_raw;
+        // offsets of a step from the run's first, step s_lo (uniform)
+        const uint32_t raw_0 = __builtin_amdgcn_readfirstlane(3u * (uint32_t)((T0 - tf) * row_bytes));
+        const uint32_t dy_0 = __builtin_amdgcn_readfirstlane((uint32_t)((T0 - t0) * row_bytes));
+
+        struct CRows { u32x2 p[NH + NR]; uint32_t dy[NR]; };      // the words of the pieces that hold C, and dy
+        struct Raw { u32x3 p[NH + NR]; };
+        auto fetch_c = [&](uint32_t raw_b, uint32_t dy_b, CRows &r) {
+#pragma unroll
+            for (int i = 0; i < NH + NR; ++i) r.p[i] = ldw8_cached(wraw, lane_feat + (raw_b + (uint32_t)i * rb3));
+#pragma unroll
+            for (int i = 0; i < NR; ++i) r.dy[i] = ldw4_cached(wdy, lane_dy + (dy_b + (uint32_t)i * rb));
+        };
+        auto fetch_raw = [&](uint32_t raw_b, Raw &r) {
+#pragma unroll
+            for (int i = 0; i < NH + NR; ++i) r.p[i] = ldw12_cached(wraw, lane_feat + (raw_b + (uint32_t)i * rb3));
+        };
+        auto store_units = [&](unsigned char *tile, const float (&f)[8]) {
+#pragma unroll
+            for (int k = 0; k < NR; ++k) store_operand_unit<T>(tile + (NR * rr + k) * UROW + 4 * a, UROW, &f[2 * k]);
+        };
+        // x, B of a step from its raw rows (rounded like the featurizer's output), and u
+        auto make_u = [&](const Raw &r, Row<T> &xr, Row<T> &Br, unsigned char *u_t) {
+            uint32_t xw[NR], Bw[NR];
+            float lo[3][NH + NR], hi[3][NH + NR], pf[8];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int i = 0; i < NH + NR; ++i) M::unpack2(r.p[i][c], lo[c][i], hi[c][i]);
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                float B0 = 0.f, x0 = 0.f, B1 = 0.f, x1 = 0.f;
+#pragma unroll
+                for (int m = 0; m < KF; ++m) {
+                    B0 = fmaf(tap[m][1], hi[0][k + m], B0);
+                    x0 = fmaf(tap[m][2], lo[1][k + m], x0);
+                    B1 = fmaf(tap[m][4], lo[2][k + m], B1);
+                    x1 = fmaf(tap[m][5], hi[2][k + m], x1);
+                }
+                xw[k] = M::pack2(x0, x1);
+                Bw[k] = M::pack2(B0, B1);
+                float xf[2], Bf[2];
+                M::unpack2(xw[k], xf[0], xf[1]);
+                M::unpack2(Bw[k], Bf[0], Bf[1]);
+                pf[2 * k] = xf[0] * Bf[0];
+                pf[2 * k + 1] = xf[1] * Bf[1];
+            }
+            xr.w[0] = make_uint4(xw[0], xw[1], xw[2], xw[3]);
+            Br.w[0] = make_uint4(Bw[0], Bw[1], Bw[2], Bw[3]);
+            store_units(u_t, pf);
+        };
+        // C of a step from its words of the raw rows, g2 = dy * C into its ring slot, dy into its own ring
+        unsigned char *const dq_own = smem + G::OFF_DQ + vt * 16;
+        auto make_g2 = [&](const CRows &r, int slot) {
+            float c0v[NH + NR], c1v[NH + NR], pf[8], skip;
+#pragma unroll
+            for (int i = 0; i < NH + NR; ++i) {
+                M::unpack2(r.p[i][0], c0v[i], skip);
+                M::unpack2(r.p[i][1], skip, c1v[i]);
+            }
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                float C0 = 0.f, C1 = 0.f, d0, d1;
+#pragma unroll
+                for (int m = 0; m < KF; ++m) {
+                    C0 = fmaf(tap[m][0], c0v[k + m], C0);
+                    C1 = fmaf(tap[m][3], c1v[k + m], C1);
+                }
+                M::unpack2(M::pack2(C0, C1), C0, C1);
+                M::unpack2(r.dy[k], d0, d1);
+                pf[2 * k] = d0 * C0;
+                pf[2 * k + 1] = d1 * C1;
+            }
+            store_units(ring + slot * USZ, pf);
+            *(uint4 *)(dq_own + slot * G::DQ_VEC) = make_uint4(r.dy[0], r.dy[1], r.dy[2], r.dy[3]);
+        };
+
+        float dwa[KF][NV];                // d wf of the lane's 6 feature channels
+#pragma unroll
+        for (int m = 0; m < KF; ++m)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) dwa[m][v] = 0.f;
+        Row<T> xh[3], Bh[3];              // x, B of steps s-1, s, s+1, indexed by step modulo 3
+#pragma unroll
+        for (int i = 0; i < 3; ++i) xh[i] = Bh[i] = zero_row<T>();
+        CRows st[2];
+        Raw rn, rg;                       // raw rows of the step prepared next, and of the step whose gradient is formed next
+        {
+            // Lead-in: raw rows of the NK-1 steps before the run (for u), C and dy of its first NK steps, requested together
+            Raw past[NK - 1], first;
+            CRows lead[NK];
+#pragma unroll
+            for (int i = 1; i < NK; ++i) fetch_raw(raw_0 - (uint32_t)i * step_b3, past[i - 1]);
+#pragma unroll
+            for (int jj = NK - 2; jj >= 0; --jj) fetch_c(raw_0 + (uint32_t)jj * step_b3, dy_0 + (uint32_t)jj * step_b, lead[jj]);
+            fetch_c(raw_0 + (uint32_t)(NK - 1) * step_b3, dy_0 + (uint32_t)(NK - 1) * step_b, lead[NK - 1]);
+            fetch_raw(raw_0, first);
+            fetch_c(raw_0 + (uint32_t)NK * step_b3, dy_0 + (uint32_t)NK * step_b, st[1]);
+            __syncthreads();                                          // (A)
+            __syncthreads();                                          // (A2): the filter tables' place is free
+#pragma unroll
+            for (int i = 1; i < NK; ++i) {
+                // iteration s_lo-i carries u of step s_lo-i and g2 / dy of step s_lo+NK-1-i
+                Row<T> x_, B_;
+                make_u(past[i - 1], x_, B_, smem + D::OFF_U);
+                make_g2(lead[NK - 1 - i], NK - 1 - i);
+                __syncthreads();                                      // (B_i)
+                __syncthreads();                                      // (C_i)
+            }
+            make_u(first, xh[0], Bh[0], smem + D::OFF_U);
+            make_g2(lead[NK - 1], NK - 1);
+            rg = first;                   // (not used: step s_lo-1 is outside the run)
+            fetch_raw(raw_0 + step_b3, rn);
+            __syncthreads();                                          // (D)
+        }
+
+        const int rows_left = (int)(L - T0 < (int64_t)(n_steps + 4) * STEP ? L - T0 : (int64_t)(n_steps + 4) * STEP);
+        __builtin_amdgcn_s_setprio(2);            // these waves are the longer ones: 372 -> 355 us
+        uint32_t raw_b = raw_0, dy_b = dy_0;      // of step s
+        int s = 0;                                // counted from the run's first step
+        unsigned char *const df_own = smem + G::OFF_DF + own_off, *const df_last = smem + G::OFF_DFP + a * 24;
+        auto row_step = [&](int pu) __attribute__((always_inline)) {
+            const int par = pu & 1, prev = (pu + RSLOTS - 1) % RSLOTS;
+            const unsigned char *const u_cur = smem + D::OFF_U + par * USZ;
+            unsigned char *const u_nx = smem + D::OFF_U + (par ^ 1) * USZ;
+            const unsigned char *const y_old = smem + D::OFF_Y + (par ^ 1) * YSZ + NR * rr * YROW + 8 * a;
+            const unsigned char *const d_old = y_old + (D::OFF_D - D::OFF_Y);
+            fetch_c(raw_b + (uint32_t)(NK + 1) * step_b3, dy_b + (uint32_t)(NK + 1) * step_b, st[par]);
+            // gradient of the features of step s-1 -> LDS, where the product waves turn it into d raw
+            u32x3 po[NR];
+            {
+                const uint4 dyq = *(const uint4 *)(dq_own + prev * G::DQ_VEC);
+                const uint32_t dyw[NR] = {dyq.x, dyq.y, dyq.z, dyq.w};
+                const uint4 xq = xh[(pu + 2) % 3].w[0], Bq = Bh[(pu + 2) % 3].w[0];
+                const uint32_t xw[NR] = {xq.x, xq.y, xq.z, xq.w}, Bw[NR] = {Bq.x, Bq.y, Bq.z, Bq.w};
+#pragma unroll
+                for (int i = 0; i < NR; ++i) {
+                    const float2 y2v = *(const float2 *)(y_old + i * YROW), duv = *(const float2 *)(d_old + i * YROW);
+                    float d0, d1, x0, x1, B0, B1;
+                    M::unpack2(dyw[i], d0, d1);
+                    M::unpack2(xw[i], x0, x1);
+                    M::unpack2(Bw[i], B0, B1);
+                    po[i] = u32x3{M::pack2(d0 * y2v.x, duv.x * x0), M::pack2(duv.x * B0, d1 * y2v.y), M::pack2(duv.y * x1, duv.y * B1)};
+                }
+                if (s * STEP > rows_left) {
+                    // rows past the sequence: zero whatever their features are
+#pragma unroll
+                    for (int i = 0; i < NR; ++i)
+                        if ((s - 1) * STEP + NR * rr + i >= rows_left) po[i] = u32x3{0u, 0u, 0u};
+                }
+                lds_store_blk(df_own + (par ^ 1) * G::PRE, pieces_blk(po));
+                if (rr == G::NG - 1) lds_store_halo(df_last + ((pu + 2) % 3) * G::PRE_BYTES, pieces_halo(po + NR - NH));
+            }
+            if (s > 0 && s <= n_steps) {
+                // d wf of step s-1, two rows per product: value v of rows (i, i+1) of the gradient with value v of rows
+                // (i+m, i+m+1) of raw
+                uint32_t rp[NH + NR - 1][NV], gp[NR / 2][NV];
+#pragma unroll
+                for (int i = 0; i < NH + NR - 1; ++i)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        rp[i][2 * c] = pair_lo(rg.p[i][c], rg.p[i + 1][c]);
+                        rp[i][2 * c + 1] = pair_hi(rg.p[i][c], rg.p[i + 1][c]);
+                    }
+#pragma unroll
+                for (int i = 0; i < NR / 2; ++i)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        gp[i][2 * c] = pair_lo(po[2 * i][c], po[2 * i + 1][c]);
+                        gp[i][2 * c + 1] = pair_hi(po[2 * i][c], po[2 * i + 1][c]);
+                    }
+#pragma unroll
+                for (int i = 0; i < NR / 2; ++i)
+#pragma unroll
+                    for (int m = 0; m < KF; ++m)
+#pragma unroll
+                        for (int v = 0; v < NV; ++v) dwa[m][v] = dot2<bf16_t>(gp[i][v], rp[2 * i + m][v], dwa[m][v]);
+            }
+            fetch_raw(raw_b, rg);
+            // step s+1: x, B, u; C and dy of step s+NK, g2
+            make_u(rn, xh[(pu + 1) % 3], Bh[(pu + 1) % 3], u_nx);
+            fetch_raw(raw_b + 2u * step_b3, rn);
+            make_g2(st[par ^ 1], prev);
+            if (s < n_steps) duo_filter_gradient<T>(P, u_cur, ring, pu, w, l);    // filter-gradient tiles of step s
+            __syncthreads();
+            ++s;
+            raw_b += step_b3;
+            dy_b += step_b;
+        };
+        // (each kind of iteration is a straight-line body of its own, so that its LDS reads can be requested early)
+        while (s < n_it) {
+#pragma unroll
+            for (int pu = 0; pu < RSLOTS; ++pu)
+                if (s < n_it) row_step(pu);
+        }
+        __syncthreads();                                              // (E)
+        float *pt = (float *)(smem + G::OFF_P) + w * ND * 256;
+#pragma unroll
+        for (int dl = 0; dl < ND; ++dl)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) pt[dl * 256 + (4 * q + v) * 16 + j] = P[dl][v];
+        float *wacc = (float *)(smem + G::OFF_W);
+#pragma unroll
+        for (int m = 0; m < KF; ++m)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) wacc[(m * G::NG + rr) * (LPR * NV) + a * NV + v] = dwa[m][v];
+        __syncthreads();                                              // (F)
+        if (wave_valid) {
+            float *out = ws + ((size_t)wg_id * NW + w) * 128;
+            for (int lag = l; lag < 128; lag += 64) {
+                const int dl = lag >> 4, r = lag & 15;
+                float sum = 0.f;
+                for (int jj = 0; jj + r < 16; ++jj) sum += pt[dl * 256 + (jj + r) * 16 + jj];
+                for (int ii = 0; ii < r; ++ii) sum += pt[(dl + 1) * 256 + ii * 16 + ii + 16 - r];
+                __hip_atomic_store(out + lag, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    mixer_bwd_finish<T, false>(ws, wsf, dh, dwf, dm, pl, cb, kf);
+}
+
 // ---------------------------------------------------------------------------- forward
 // The same division of labour for y = C * (T u), u = x * B, with the features made from the projection output on
 // the way.  The forward has no ring to keep and few registers per wave, so a workgroup takes sixteen waves and 128
@@ -954,6 +1396,25 @@ int bwd_t(const void *dy, const void *raw, const void *wfeat, int kf, const void
     return launch_colsum_reduce<T>(ws_f, (T *)dwf, dm.bs * p.nseg, 3 * dm.d, 1, (int)(3 * dm.d), kf, st);
 }
 
+int bwd_wide(const void *dy, const void *raw, const void *wfeat, int kf, const void *h, void *draw, void *dwf, void *dh,
+             void *ws, const Dims &dm, hipStream_t st)
+{
+    typedef bf16w_t T;
+    MfmaPlan p = mixer_plan(dm);
+    if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
+    if (p.fuse_dh && (p.slot = dh_slot_for_stream(st)) < 0) p.fuse_dh = p.slot = 0;   // no ticket set: second launches
+    float *ws_dh = (float *)ws;
+    float *ws_f = ws_dh + (size_t)p.nwg * WideGeo::NW * 128;
+    int e = launch_main(mixer_mr_bwd_wide_kernel, dim3((unsigned)p.nwg), dim3(WideGeo::NT), st, (const T *)dy, (const T *)raw,
+                        (const T *)h, (const T *)wfeat, kf, (T *)draw, (T *)dh, (T *)dwf, ws_dh, ws_f, dm, p);
+    if (e || p.fuse_dh) return e;
+    const int64_t n = (int64_t)dm.g * (dm.fw ? dm.lc : dm.hl);
+    e = launch_plain(mfma_dh_reduce_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), st, (const float *)ws_dh,
+                     (T *)dh, dm, p);
+    if (e) return e;
+    return launch_colsum_reduce<bf16_t>(ws_f, (bf16_t *)dwf, dm.bs * p.nseg, 3 * dm.d, 1, (int)(3 * dm.d), kf, st);
+}
+
 } // namespace
 
 namespace {
@@ -991,6 +1452,20 @@ bool mixer_mr_fused_supported(int dtype, const Dims &dm, int kf)
     return windows_fit(dm, mixer_plan(dm)) && windows_fit(dm, mixer_fwd_plan(dm));
 }
 
+// The backward alone: also bf16 tensors in fp32 arithmetic (interleaved features; f16's operands take three planes,
+// whose rings do not fit the registers of the product waves).  Not where the columns hold fewer than 1024 steps of 32
+// rows, 64 runs at most: with three quarters of the chip idle the featurizer's backward is better a kernel of its own,
+// which spreads over all of it, than three more iterations of each run (one kernel against two, 16-channel groups:
+// 64 steps 51.5 / 46.0 us, 256 steps 52.0 / 48.8, 516 steps 65.4 / 66.1, 1024 steps 57.4 / 62.2 and 63.4 / 70.0,
+// 4096 steps 72 / 87, 32768 steps 332 / 458).
+bool mixer_mr_fused_bwd_supported(int dtype, const Dims &dm, int kf)
+{
+    if (dtype != GCG_BF16_F32) return mixer_mr_fused_supported(dtype, dm, kf);
+    const MfmaPlan p = mixer_plan(dm);
+    return !dm.planar && mfma_feat_supported(dtype, dm, kf) && 3 * dm.d <= 0x7fffffffLL && windows_fit(dm, p) &&
+           dm.bs * p.ncb * p.nsteps >= 1024;
+}
+
 size_t mixer_mr_fused_workspace(const Dims &dm, int kf)
 {
     const MfmaPlan p = mixer_plan(dm);
@@ -1002,6 +1477,7 @@ int mixer_mr_fused_bwd_launch(int dtype, const void *dy, const void *raw, const 
 {
     if (dtype == GCG_BF16) return bwd_t<bf16_t>(dy, raw, wfeat, kf, h, draw, dwf, dh, ws, dm, st);
     if (dtype == GCG_F16) return bwd_t<f16_t>(dy, raw, wfeat, kf, h, draw, dwf, dh, ws, dm, st);
+    if (dtype == GCG_BF16_F32 && !dm.planar) return bwd_wide(dy, raw, wfeat, kf, h, draw, dwf, dh, ws, dm, st);
     return (int)hipErrorInvalidValue;
 }
 
