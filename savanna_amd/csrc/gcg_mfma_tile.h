@@ -905,6 +905,19 @@ int nk_for(int hl) { const int n = (hl + 30) / 32 + 1; return n > 5 ? 5 : n; }
 // request keeps a CU to one.  The 8-wave form is no longer instantiated.
 constexpr int BWD_NW = 4;
 
+// Shortest runs.  A launch that leaves CUs idle is as long as one run -- its steps and the NK-1 steps of lead-in -- so a
+// run is cut as far as that shortens it, down to where the lead-in, the tables and the arrival at the sums outweigh
+// the steps saved.
+// Backward: 4 steps.  16 (before), 8, 4, 2 at 1 x 701 x 1024: bf16 28.5, 19.1, 14.3, 12.4 us, fp32 64, 42, 27, 21,
+// mixer 48, 38, 30, 35; 1 x 701 x 4096: bf16 31, 22, 22, 20, fp32 74, 46, 38, 37, mixer 52, 42, 45, 45; 1 x 300 x
+// 4096: mixer 35, 35, 33, 40.  From runs of 16 steps on (1 x 8192 x 1024) nothing changes.
+constexpr int BWD_MIN_STEPS = 4;
+// Forward: 3 steps with 16-bit operands, where two workgroups share a CU and more of them slow each other down (4 steps
+// before, 3, 2: 1 x 2000 x 4096 17.7, 15.7, 15.3 us, 1 x 701 x 4096 10.0, 9.1, 10.9, 1 x 4000 x 1024 9.7, 9.3, 10.9),
+// 2 with operands of several planes (bf16 tensors in fp32 arithmetic, 1 x 300 x 4096: 10.6 and 8.0 us; fp32 tensors
+// 18.8 and 16.7, 1 x 701 x 4096 23.4 and 19.1).
+template <typename T> constexpr int fwd_min_steps() { return MT<T>::SPLIT ? 2 : 3; }
+
 // one workgroup per CU in either geometry (fp32: one wave per SIMD by its registers alone)
 MfmaPlan plan_bwd_nw(const Dims &dm, int nw, int elem_bytes);
 MfmaPlan plan_bwd(const Dims &dm, bool split, int elem_bytes)
@@ -922,7 +935,7 @@ int choose_nw_bwd_feat(bool split)
 }
 MfmaPlan plan_bwd_nw(const Dims &dm, int nw, int elem_bytes)
 {
-    MfmaPlan p = plan(dm, nw, 16, nw, elem_bytes);
+    MfmaPlan p = plan(dm, nw, BWD_MIN_STEPS, nw, elem_bytes);
     // the kernel adds the partials itself when a filter group lies within one channel block (and the launch gets a
     // ticket set, dh_slot_for_stream); otherwise a second launch does
     p.fuse_dh = (16 * nw) % dm.dg == 0 && p.ncb <= DH_UNITS;

@@ -262,12 +262,20 @@ __device__ __forceinline__ void mixer_bwd_finish(const float *ws, const float *w
                 ((float *)dh)[grp * row + k] = 0.f;
                 continue;
             }
-            const int lag = dm.hl - 1 - k;
+            // p-major, as the second launch adds them; eight reads in flight together
+            const float *src = ws + ((int64_t)cb * G::XW + gl * bpg) * 128 + (dm.hl - 1 - k);
+            const int64_t n = np * bpg;
             float sum = 0.f;
-            for (int64_t p = 0; p < np; ++p)
-                for (int kk = 0; kk < bpg; ++kk)
-                    sum += __hip_atomic_load(ws + ((p * pl.ncb + cb) * G::XW + gl * bpg + kk) * 128 + lag, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
+            for (int64_t i0 = 0; i0 < n; i0 += 8) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int64_t i = i0 + u < n ? i0 + u : 0, p = bpg == 1 ? i : bpg == 2 ? i >> 1 : i >> 2;
+                    v[u] = __hip_atomic_load(src + (p * pl.ncb * G::XW + (i - p * bpg)) * 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) sum = i0 + u < n ? sum + v[u] : sum;
+            }
             store_dh<T>(dh, dm, grp, k, sum);
         }
     }
@@ -277,10 +285,18 @@ __device__ __forceinline__ void mixer_bwd_finish(const float *ws, const float *w
         // the block's feature channels: 3 * CB consecutive ones, or CB of each plane
         const int64_t f = PL ? (int64_t)(col / G::CB) * dm.d + (int64_t)cb * G::CB + col % G::CB : (int64_t)cb * 3 * G::CB + col;
         if (PL ? (int64_t)cb * G::CB + col % G::CB >= dm.d : f >= nf) continue;
-        float sum = 0.f;
-        for (int64_t p = 0; p < np; ++p)
-            sum += __hip_atomic_load(wsf + ((size_t)kk * np + p) * nf + f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        Elem<T>::store(dwf + f * kf + kk, sum);
+        // every fourth run, then the four sums: as the second launch (colsum_reduce_block) adds them
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int64_t p0 = 0; p0 < np; p0 += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                v[u] = __hip_atomic_load(wsf + ((size_t)kk * np + (p0 + u < np ? p0 + u : 0)) * nf + f, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) sum[u & 3] = p0 + u < np ? sum[u & 3] + v[u] : sum[u & 3];
+        }
+        Elem<T>::store(dwf + f * kf + kk, sum[0] + sum[1] + sum[2] + sum[3]);
     }
 }
 
@@ -1358,7 +1374,7 @@ namespace {
 
 MfmaPlan mixer_plan(const Dims &dm)
 {
-    MfmaPlan p = plan(dm, MixGeo<bf16_t>::XW, 16, MixGeo<bf16_t>::XW, 2);
+    MfmaPlan p = plan(dm, MixGeo<bf16_t>::XW, BWD_MIN_STEPS, MixGeo<bf16_t>::XW, 2);
     // the kernel adds the partials itself when a filter group lies within one channel block
     p.fuse_dh = MixGeo<bf16_t>::CB % dm.dg == 0 && p.ncb <= DH_UNITS;
     return p;
@@ -1420,7 +1436,8 @@ int bwd_wide(const void *dy, const void *raw, const void *wfeat, int kf, const v
 namespace {
 MfmaPlan mixer_fwd_plan(const Dims &dm)
 {
-    return plan(dm, MixFwdGeo<bf16_t>::XW, 4, MixFwdGeo<bf16_t>::XW, 2);
+    // runs of 2 steps at least: 1 x 701 x 4096, 20.0 us with 4 and 17.9 with 2; 1 x 701 x 1024, 17.8 and 15.1
+    return plan(dm, MixFwdGeo<bf16_t>::XW, 2, MixFwdGeo<bf16_t>::XW, 2);
 }
 template <typename T>
 int fwd_t(const void *raw, const void *wfeat, int kf, const void *h, void *y, const Dims &dm, hipStream_t st)
@@ -1453,11 +1470,10 @@ bool mixer_mr_fused_supported(int dtype, const Dims &dm, int kf)
 }
 
 // The backward alone: also bf16 tensors in fp32 arithmetic (interleaved features; f16's operands take three planes,
-// whose rings do not fit the registers of the product waves).  Not where the columns hold fewer than 1024 steps of 32
-// rows, 64 runs at most: with three quarters of the chip idle the featurizer's backward is better a kernel of its own,
-// which spreads over all of it, than three more iterations of each run (one kernel against two, 16-channel groups:
-// 64 steps 51.5 / 46.0 us, 256 steps 52.0 / 48.8, 516 steps 65.4 / 66.1, 1024 steps 57.4 / 62.2 and 63.4 / 70.0,
-// 4096 steps 72 / 87, 32768 steps 332 / 458).
+// whose rings do not fit the registers of the product waves).  From 1024 steps of 32 rows on, all columns together:
+// smaller problems keep the two kernels and with them the order of the sums of d wf (its bits are the two-call chain's);
+// what that costs there is mostly the second launch (one kernel against two, from graph replays: 64 steps 28.8 / 29.0 us,
+// 256 steps 30 / 35, 560 steps 34 / 42, 1024 steps 39 / 52, 4096 steps 64 / 91).
 bool mixer_mr_fused_bwd_supported(int dtype, const Dims &dm, int kf)
 {
     if (dtype != GCG_BF16_F32) return mixer_mr_fused_supported(dtype, dm, kf);

@@ -107,8 +107,5 @@ def test_graph_replays_match_eager(gcg_lib):
         dy.normal_()
         graph.replay()
         torch.cuda.synchronize()
-        draw, dwf, dh = _lib.mixer_mr_bwd(dy, raw, wf, h)
-        assert torch.equal(recorded[0], draw) and torch.equal(recorded[2], dh), it
-        # (a recorded launch adds the runs' sums of d wf with a second kernel, in another order: one unit of bf16)
-        a, b = recorded[1].double(), dwf.double()
-        assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-5 * b.abs().max()).all(), it
+        for a, b in zip(recorded, _lib.mixer_mr_bwd(dy, raw, wf, h)):
+            assert torch.equal(a, b), it
