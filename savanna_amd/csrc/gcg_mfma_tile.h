@@ -911,7 +911,14 @@ constexpr int BWD_NW = 4;
 // Backward: 4 steps.  16 (before), 8, 4, 2 at 1 x 701 x 1024: bf16 28.5, 19.1, 14.3, 12.4 us, fp32 64, 42, 27, 21,
 // mixer 48, 38, 30, 35; 1 x 701 x 4096: bf16 31, 22, 22, 20, fp32 74, 46, 38, 37, mixer 52, 42, 45, 45; 1 x 300 x
 // 4096: mixer 35, 35, 33, 40.  From runs of 16 steps on (1 x 8192 x 1024) nothing changes.
-constexpr int BWD_MIN_STEPS = 4;
+// Only where runs of 16 steps leave CUs idle: a launch that fills the chip keeps its runs, and the sums of its filter
+// gradient their scratch (at most 2304 workgroups otherwise, a little over half of the static scratch array).
+constexpr int BWD_MIN_STEPS = 4, BWD_FULL_STEPS = 16;
+MfmaPlan plan_bwd_runs(const Dims &dm, int nw, int elem_bytes)
+{
+    const MfmaPlan p = plan(dm, nw, BWD_FULL_STEPS, nw, elem_bytes);
+    return p.nwg >= cu_count() ? p : plan(dm, nw, BWD_MIN_STEPS, nw, elem_bytes);
+}
 // Forward: 3 steps with 16-bit operands, where two workgroups share a CU and more of them slow each other down (4 steps
 // before, 3, 2: 1 x 2000 x 4096 17.7, 15.7, 15.3 us, 1 x 701 x 4096 10.0, 9.1, 10.9, 1 x 4000 x 1024 9.7, 9.3, 10.9),
 // 2 with operands of several planes (bf16 tensors in fp32 arithmetic, 1 x 300 x 4096: 10.6 and 8.0 us; fp32 tensors
@@ -935,7 +942,7 @@ int choose_nw_bwd_feat(bool split)
 }
 MfmaPlan plan_bwd_nw(const Dims &dm, int nw, int elem_bytes)
 {
-    MfmaPlan p = plan(dm, nw, BWD_MIN_STEPS, nw, elem_bytes);
+    MfmaPlan p = plan_bwd_runs(dm, nw, elem_bytes);
     // the kernel adds the partials itself when a filter group lies within one channel block (and the launch gets a
     // ticket set, dh_slot_for_stream); otherwise a second launch does
     p.fuse_dh = (16 * nw) % dm.dg == 0 && p.ncb <= DH_UNITS;

@@ -1374,7 +1374,7 @@ namespace {
 
 MfmaPlan mixer_plan(const Dims &dm)
 {
-    MfmaPlan p = plan(dm, MixGeo<bf16_t>::XW, BWD_MIN_STEPS, MixGeo<bf16_t>::XW, 2);
+    MfmaPlan p = plan_bwd_runs(dm, MixGeo<bf16_t>::XW, 2);
     // the kernel adds the partials itself when a filter group lies within one channel block
     p.fuse_dh = MixGeo<bf16_t>::CB % dm.dg == 0 && p.ncb <= DH_UNITS;
     return p;
