@@ -738,16 +738,17 @@ __global__ __launch_bounds__(MixGeo<T>::NT) void mixer_mr_bwd_kernel(const T *__
 //   product waves (0..3)  iteration s: y2, du of step s, and d raw of step s-2 from the gradient rows in LDS.
 // The operand planes take the LDS that holds the raw rows in the 16-bit kernel, so a raw row is requested three times
 // -- five steps ahead for C (8 of a piece's 12 bytes), one step ahead for x and B, and with its gradient for d wf --
-// and all but the first are answered by the caches: a step's rows are 12 KB per workgroup, and those of six steps of
-// the 32 workgroups of an XCD are 2.4 MB of its 4 MB L2.  dy waits for its step in a lane-private ring in LDS.
+// and nearly all but the first are answered by the L2: a step's rows are 12 KB per workgroup, and those of six steps of
+// the 32 workgroups of an XCD are 2.4 MB of its 4 MB, which dy and the last reading therefore pass with the streaming
+// hint (907 MB read from beyond the L2 without it, 625 with it, 537 at least).  dy waits for its step in a lane-private ring in LDS.
 // A run goes one step beyond its end for the gradient rows that its last two rows of d raw need, and two iterations
 // further for the hand-overs; what these compute beyond the run is dropped by the windows or not accumulated.
 //
 // What bounds it: instruction issue (87 matrix instructions per 16 channels and step, and the vector work of both
 // kernels it replaces: 59 % of the quad-cycles issue, and a matrix instruction takes four).  7B shape (2 x 8192 x 4096),
-// bf16: 319 - 347 us, against 233 - 264 us for the operator's backward with the features made in front (gradient of the
+// bf16: 319 - 343 us, against 233 - 264 us for the operator's backward with the features made in front (gradient of the
 // features to memory) and 217 - 222 + 9 us for the featurizer's backward on it; 7 instead of 16 values moved per
-// element (454 MB read, 404 MB written).  Measured and left: d wf on the product waves (351 us), d wf with fused
+// element.  Measured and left: d wf on the product waves (351 us), d wf with fused
 // multiply-adds on unpacked values (351), straight-line bodies for the first, middle and last steps (spills, 590).
 struct WideGeo {
     typedef bf16w_t T;
@@ -962,7 +963,12 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
 #pragma unroll
             for (int i = 0; i < NH + NR; ++i) r.p[i] = ldw8_cached(wraw, lane_feat + (raw_b + (uint32_t)i * rb3));
 #pragma unroll
-            for (int i = 0; i < NR; ++i) r.dy[i] = ldw4_cached(wdy, lane_dy + (dy_b + (uint32_t)i * rb));
+            for (int i = 0; i < NR; ++i) r.dy[i] = ldw4(wdy, lane_dy + (dy_b + (uint32_t)i * rb));
+        };
+        // (dy, and the raw rows when they are read for the last time, with the streaming hint: 350 -> 343 us)
+        auto fetch_raw_last = [&](uint32_t raw_b, Raw &r) {
+#pragma unroll
+            for (int i = 0; i < NH + NR; ++i) r.p[i] = ldw12(wraw, lane_feat + (raw_b + (uint32_t)i * rb3));
         };
         auto fetch_raw = [&](uint32_t raw_b, Raw &r) {
 #pragma unroll
@@ -1129,7 +1135,7 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
 #pragma unroll
                         for (int v = 0; v < NV; ++v) dwa[m][v] = dot2<bf16_t>(gp[i][v], rp[2 * i + m][v], dwa[m][v]);
             }
-            fetch_raw(raw_b, rg);
+            fetch_raw_last(raw_b, rg);
             // step s+1: x, B, u; C and dy of step s+NK, g2
             make_u(rn, xh[(pu + 1) % 3], Bh[(pu + 1) % 3], u_nx);
             fetch_raw(raw_b + 2u * step_b3, rn);
