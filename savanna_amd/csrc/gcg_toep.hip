@@ -15,6 +15,12 @@
 // Precision is that of the fp32 vector kernels of gcg_direct.hip: every operand enters as a sum of bf16 planes that
 // hold it exactly (the product of two bf16 values has 16 significant bits: two planes; of two f16 values 22: three;
 // fp32: three), and of the plane products those with m + n <= 2 are formed; the ones left out are below 2^-24.
+// A matrix instruction rounds its sum towards minus infinity, not to the nearest value: in a product of 32 NK terms
+// that is below the vector kernels' own error, but in the filter gradient, a sum over all rows, it adds up to a bias
+// (dh 2.5 to 6 times as far from 64 bits as the vector kernels'; 1 x 16384 x (16 groups of 32), 256 taps: 1.8e-6 of the
+// 2-norm against 3.2e-7).  There each instruction's chain is 32 rows long, a tile and a run are summed on the vector
+// ALUs, and half of a tile's products enter negated, so that the bias of one half is taken off by the other's: 1.4e-7,
+// and below the vector kernels' error at every shape compared, for 4 % of the backward's time.
 //
 // A workgroup owns CB adjacent channels and a run of 256-row tiles of one batch row; u (and g2) of a tile and of the
 // filter's reach stay in LDS as rings, so each row is read once (dy twice in the backward: for g2 OFF rows ahead, and
@@ -111,6 +117,15 @@ __device__ __forceinline__ bf16x8 lds_any8(const uint16_t *row, int idx)
     bf16x8 r;
     __builtin_memcpy(&r, o, 16);
     return r;
+}
+__device__ __forceinline__ bf16x8 negated(bf16x8 v)
+{
+    uint32_t o[4];
+    __builtin_memcpy(o, &v, 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] ^= 0x80008000u;
+    __builtin_memcpy(&v, o, 16);
+    return v;
 }
 // plane products a_m b_n with m + n <= 2, smallest first
 template <int NA, int NB>
@@ -405,21 +420,31 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         *(f32x4 *)(v + 4) = *(const f32x4 *)(yr + 4);
 #pragma unroll
         for (int e = 0; e < 8; ++e) st_elem<T>(wdC, (row + e) * ri + ci, raw_float<T>(rd[e]) * v[e]);
-        band_product<T, NK, CB>(acc, rg, tb, nf, fa, fb, cw, front, lane);
+        // filter gradient: 32 rows' products by themselves, added to the tile's sum and that to the run's; half of the
+        // products with a negated operand (see the head of this file)
+        f32x4 dt[2];
+        dt[0] = dt[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int neg = 0; neg < 2; ++neg)
 #pragma unroll 1
-        for (int s = 0; s < TT / 32; ++s) {
-            const int pg = wrap<G::R>(front + 32 * s + 8 * q + ga), pu = wrap<G::R>(oldest + G::OFF + 32 * s + 8 * q - n);
+            for (int s = neg * (TT / 64); s < (neg + 1) * (TT / 64); ++s) {
+                const int pg = wrap<G::R>(front + 32 * s + 8 * q + ga), pu = wrap<G::R>(oldest + G::OFF + 32 * s + 8 * q - n);
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                bf16x8 a[NPA], b[NPA];
+                for (int c = 0; c < 2; ++c) {
+                    bf16x8 a[NPA], b[NPA];
 #pragma unroll
-                for (int m = 0; m < NPA; ++m) {
-                    a[m] = lds_aligned8(rg + (m * CB + cw + c) * G::RP + pg);
-                    b[m] = lds_any8(ru + (m * CB + cw + c) * G::RP, pu);
+                    for (int m = 0; m < NPA; ++m) {
+                        a[m] = lds_aligned8(rg + (m * CB + cw + c) * G::RP + pg);
+                        if (neg) a[m] = negated(a[m]);
+                        b[m] = lds_any8(ru + (m * CB + cw + c) * G::RP, pu);
+                    }
+                    const f32x4 t = mfma_planes(a, b, (f32x4){0.f, 0.f, 0.f, 0.f});
+                    dt[c] = neg ? dt[c] - t : dt[c] + t;
                 }
-                dh[c] = mfma_planes(a, b, dh[c]);
             }
-        }
+        dh[0] += dt[0];
+        dh[1] += dt[1];
+        band_product<T, NK, CB>(acc, rg, tb, nf, fa, fb, cw, front, lane);
         __syncthreads();
         *(f32x4 *)yw = acc[0];
         *(f32x4 *)(yw + YP) = acc[1];

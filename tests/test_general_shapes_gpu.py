@@ -68,3 +68,19 @@ def test_feature_layouts_give_the_same_bits(gcg_lib, bs, L, g, dg, hl, layout):
     for a, b in zip(dfeat.unbind(dim), (dC, dB, dx)):
         assert torch.equal(a, b)
     assert torch.equal(dh, dh_s)
+
+
+@pytest.mark.parametrize("types", ["f32", "bf16w", "f16w"])
+@pytest.mark.parametrize("bs,L,g,dg,hl", [(1, 4096, 64, 8, 128), (4, 16384, 9, 14, 30), (1, 8192, 16, 32, 256), (2, 3000, 7, 5, 17)])
+def test_filter_gradient_has_no_bias(gcg_lib, bs, L, g, dg, hl, types):
+    """dh (kept in fp32) against its 64-bit sum.  A sum of P terms of random sign, added one after the other with rounding
+    to nearest, is off by 2^-24 sqrt(P / 6) of its size; the bar is that for the vector kernels' P = 64-row partial sums,
+    and 1.5 units for the roundings within them.  A rounding that always goes one way adds up like P instead."""
+    dtype, filt = TYPES[types]
+    gen = torch.Generator(device=DEV).manual_seed(hl)
+    x, B, C, dy = (torch.randn(bs, L, g, dg, generator=gen, device=DEV).to(dtype) for _ in range(4))
+    h = torch.randn(g, 1, hl, generator=gen, device=DEV).to(filt or dtype)
+    dh = _lib.bwd(dy, x, B, C, h)[3][:, 0].double()
+    u, g2 = x.double() * B.double(), dy.double() * C.double()
+    exact = torch.stack([(g2[:, lag:] * u[:, :L - lag]).sum((0, 1, 3)) for lag in reversed(range(hl))], dim=1)
+    assert (dh - exact).norm() <= 2.0 ** -24 * (1.5 + (bs * L / 64 / 6) ** 0.5) * exact.norm()
