@@ -749,7 +749,7 @@ GCG_API size_t gcg_mixer_mr_bwd_workspace_bytes(int64_t bs, int64_t L, int32_t g
     if (!gcg::mfma_feat_supported(dtype, dm, kf)) return 0;
     if (make_dims(bs, L, 3 * g * dg, 1, kf, plain_tensor_code(dtype), &df) || !gcg::dwconv_supported(df)) return 0;
     const size_t chain = up256(gcg::mfma_feat_bwd_workspace(dtype, dm)) + up256(gcg::dwconv_bwd_workspace(df));
-    const size_t fused = gcg::mixer_mr_fused_bwd_supported(dtype, dm, kf) ? up256(gcg::mixer_mr_fused_workspace(dm, kf)) : 0;
+    const size_t fused = gcg::mixer_mr_fused_bwd_supported(dtype, dm, kf) ? up256(gcg::mixer_mr_fused_workspace(dtype, dm, kf)) : 0;
     return chain > fused ? chain : fused;
 }
 

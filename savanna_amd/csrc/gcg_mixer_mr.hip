@@ -776,10 +776,28 @@ __device__ __forceinline__ u32x2 ldw8_cached(win_t w, uint32_t off)
     return __builtin_amdgcn_raw_buffer_load_b64(w, (int)off, 0, 0);
 }
 
+// A lane's sums of d wf are put aside in memory every `every` steps and start again at zero (a step is 4 rows of a lane,
+// two an addition), so that their chains of additions are not longer than in the featurizer's own backward, whose lanes
+// sum 64 rows of small problems and 128 of large ones; the row groups' sums are added as a tree.  Distance from the
+// 64-bit sums, in 2^-24 of the 2-norm of the terms: 16236 x 4096 1.8 (one chain for a run of 128 steps 3.2, the
+// featurizer's backward 2.2), 3948 x 4096 1.3 (1.6, 1.5), 32620 x 4096 2.0 (4.8, 2.7), 1900 x 8192 1.2 (1.4, 1.2).
+// Costs 1 - 2 % of the kernel (291 -> 294 us at the 7B shape).  A run has at most 16 such sums: longer ones where it has
+// more than 512 steps.
+struct WideSums {
+    static constexpr int VEC = 5;                // 16-byte vectors of a lane: 18 values
+    int every, n;                                // steps of a sum, and how many of a run are put aside
+};
+WideSums wide_sums(const MfmaPlan &p)
+{
+    const int64_t steps = p.steps_per_seg, every = steps <= 32 ? 8 : steps <= 64 ? 16 : steps <= 512 ? 32 : (steps + 15) / 16;
+    return {(int)every, (int)((steps - 1) / every)};
+}
+
 __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
     const bf16w_t *__restrict__ dy, const bf16w_t *__restrict__ raw, const bf16w_t *__restrict__ h,
     const bf16w_t *__restrict__ wfeat, int kf, bf16w_t *__restrict__ draw, bf16w_t *__restrict__ dh,
-    bf16w_t *__restrict__ dwf, float *__restrict__ ws, float *__restrict__ wsf, Dims dm, MfmaPlan pl)
+    bf16w_t *__restrict__ dwf, float *__restrict__ ws, float *__restrict__ wsf, f32x4 *__restrict__ wsx, WideSums sums,
+    Dims dm, MfmaPlan pl)
 {
     typedef bf16w_t T;
     typedef WideGeo G;
@@ -932,10 +950,14 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
             const int m = idx / (LPR * NV), col = idx % (LPR * NV);
             const int kk = m - (KF - kf);                             // index into the kf taps of the filter
             if (kk < 0 || 3 * c0 + col >= 3 * d) continue;
-            float sum = 0.f;
+            float sum[G::NG];
 #pragma unroll
-            for (int r = 0; r < G::NG; ++r) sum += wacc[(m * G::NG + r) * (LPR * NV) + col];
-            __hip_atomic_store(wsf + ((size_t)kk * nprow + prow) * (3 * d) + 3 * c0 + col, sum, __ATOMIC_RELAXED,
+            for (int r = 0; r < G::NG; ++r) sum[r] = wacc[(m * G::NG + r) * (LPR * NV) + col];
+#pragma unroll
+            for (int n = G::NG / 2; n > 0; n /= 2)
+#pragma unroll
+                for (int r = 0; r < n; ++r) sum[r] += sum[r + n];
+            __hip_atomic_store(wsf + ((size_t)kk * nprow + prow) * (3 * d) + 3 * c0 + col, sum[0], __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
         }
     } else {
@@ -1039,6 +1061,7 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
         for (int m = 0; m < KF; ++m)
 #pragma unroll
             for (int v = 0; v < NV; ++v) dwa[m][v] = 0.f;
+        f32x4 *const aside = wsx + (size_t)wg_id * sums.n * (WideSums::VEC * 64 * NW) + vt;
         Row<T> xh[3], Bh[3];              // x, B of steps s-1, s, s+1, indexed by step modulo 3
 #pragma unroll
         for (int i = 0; i < 3; ++i) xh[i] = Bh[i] = zero_row<T>();
@@ -1077,6 +1100,7 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
         __builtin_amdgcn_s_setprio(2);            // these waves are the longer ones: 372 -> 355 us
         uint32_t raw_b = raw_0, dy_b = dy_0;      // of step s
         int s = 0;                                // counted from the run's first step
+        int sum_left = sums.every, n_aside = 0;
         unsigned char *const df_own = smem + G::OFF_DF + own_off, *const df_last = smem + G::OFF_DFP + a * 24;
         auto row_step = [&](int pu) __attribute__((always_inline)) {
             const int par = pu & 1, prev = (pu + RSLOTS - 1) % RSLOTS;
@@ -1134,6 +1158,21 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
                     for (int m = 0; m < KF; ++m)
 #pragma unroll
                         for (int v = 0; v < NV; ++v) dwa[m][v] = dot2<bf16_t>(gp[i][v], rp[2 * i + m][v], dwa[m][v]);
+                if (--sum_left == 0 && s < n_steps) {
+                    float *const f = &dwa[0][0];
+#pragma unroll
+                    for (int i = 0; i < WideSums::VEC; ++i) {
+                        f32x4 t;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            t[k] = 4 * i + k < G::NACC ? f[4 * i + k] : 0.f;
+                            if (4 * i + k < G::NACC) f[4 * i + k] = 0.f;
+                        }
+                        aside[(n_aside * WideSums::VEC + i) * (64 * NW)] = t;
+                    }
+                    ++n_aside;
+                    sum_left = sums.every;
+                }
             }
             fetch_raw_last(raw_b, rg);
             // step s+1: x, B, u; C and dy of step s+NK, g2
@@ -1158,6 +1197,14 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
         for (int dl = 0; dl < ND; ++dl)
 #pragma unroll
             for (int v = 0; v < 4; ++v) pt[dl * 256 + (4 * q + v) * 16 + j] = P[dl][v];
+        for (int k = 0; k < n_aside; ++k) {
+            float *const f = &dwa[0][0];
+            f32x4 t[WideSums::VEC];
+#pragma unroll
+            for (int i = 0; i < WideSums::VEC; ++i) t[i] = aside[(k * WideSums::VEC + i) * (64 * NW)];
+#pragma unroll
+            for (int i = 0; i < G::NACC; ++i) f[i] += t[i / 4][i % 4];
+        }
         float *wacc = (float *)(smem + G::OFF_W);
 #pragma unroll
         for (int m = 0; m < KF; ++m)
@@ -1427,8 +1474,10 @@ int bwd_wide(const void *dy, const void *raw, const void *wfeat, int kf, const v
     if (p.fuse_dh && (p.slot = dh_slot_for_stream(st)) < 0) p.fuse_dh = p.slot = 0;   // no ticket set: second launches
     float *ws_dh = (float *)ws;
     float *ws_f = ws_dh + (size_t)p.nwg * WideGeo::NW * 128;
+    float *ws_x = ws_f + (size_t)kf * dm.bs * p.nseg * 3 * dm.d;      // (16-byte aligned: d is a multiple of 16)
     int e = launch_main(mixer_mr_bwd_wide_kernel, dim3((unsigned)p.nwg), dim3(WideGeo::NT), st, (const T *)dy, (const T *)raw,
-                        (const T *)h, (const T *)wfeat, kf, (T *)draw, (T *)dh, (T *)dwf, ws_dh, ws_f, dm, p);
+                        (const T *)h, (const T *)wfeat, kf, (T *)draw, (T *)dh, (T *)dwf, ws_dh, ws_f, (f32x4 *)ws_x,
+                        wide_sums(p), dm, p);
     if (e || p.fuse_dh) return e;
     const int64_t n = (int64_t)dm.g * (dm.fw ? dm.lc : dm.hl);
     e = launch_plain(mfma_dh_reduce_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), st, (const float *)ws_dh,
@@ -1488,10 +1537,11 @@ bool mixer_mr_fused_bwd_supported(int dtype, const Dims &dm, int kf)
            dm.bs * p.ncb * p.nsteps >= 1024;
 }
 
-size_t mixer_mr_fused_workspace(const Dims &dm, int kf)
+size_t mixer_mr_fused_workspace(int dtype, const Dims &dm, int kf)
 {
     const MfmaPlan p = mixer_plan(dm);
-    return ((size_t)p.nwg * MixGeo<bf16_t>::XW * 128 + (size_t)kf * dm.bs * p.nseg * 3 * dm.d) * sizeof(float);
+    const size_t aside = dtype == GCG_BF16_F32 ? (size_t)wide_sums(p).n * WideSums::VEC * 64 * WideGeo::NW * sizeof(f32x4) : 0;
+    return ((size_t)p.nwg * MixGeo<bf16_t>::XW * 128 + (size_t)kf * dm.bs * p.nseg * 3 * dm.d) * sizeof(float) + (size_t)p.nwg * aside;
 }
 
 int mixer_mr_fused_bwd_launch(int dtype, const void *dy, const void *raw, const void *wfeat, int kf, const void *h,

@@ -62,6 +62,37 @@ def test_against_chain(gcg_lib, bs, L, g, dg, hl, kf):
     check(run(*args), *args)
 
 
+@pytest.mark.parametrize("L,g", [(16236, 256), (3948, 256), (16236, 512)])
+def test_chains_of_the_featurizer_gradient(gcg_lib, L, g):
+    """d wf of two halves of a sequence that take each other off: dy of the second is the first's with its sign turned,
+    and zero at the ends, so what is left of the sum is small and the error of its fp32 additions shows beside the
+    rounding to bf16.  (The halves are no multiple of a lane's rows, or the errors would take each other off as well.)
+    An addition rounded to nearest is off by 0.4 2^-24 of its result (rms over the mantissas), so a chain of m additions of
+    random sign is off by 0.4 2^-24 sqrt(m / 2) of the 2-norm of its terms; the bar is that of chains of 64 rows, and of 16
+    terms in the sums above them.  Chains of a run's rows, 512 and 1024 at the first and the last shape, are beyond it."""
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    half, dg, d = L // 2, 16, 16 * g
+    raw = torch.randn(1, half, g, dg, 3, generator=gen, device=DEV).to(BF).repeat(1, 2, 1, 1, 1)
+    dy = torch.randn(1, half, g, dg, generator=gen, device=DEV).to(BF)
+    dy[:, :256] = 0
+    dy[:, -256:] = 0
+    dy = torch.cat([dy, -dy], dim=1)
+    wf = (torch.randn(3 * d, 1, 3, generator=gen, device=DEV) / 2).to(BF)
+    h = torch.randn(g, 1, 128, generator=gen, device=DEV) / 11
+    assert one_kernel(1, L, g, dg, 128, 3)
+    got = _lib.mixer_mr_bwd(dy, raw, wf, h)[1][:, 0].double()
+    f = _lib.dwconv_fwd(raw.reshape(1, L, 3 * d, 1), wf)
+    df, r = _lib.bwd_interleaved(dy, f.reshape(raw.shape), h)[0].reshape(L, 3 * d), raw.reshape(L, 3 * d)
+    err = terms2 = 0.
+    for lo in range(0, 3 * d, 2048):
+        for k in range(3):
+            terms = df[2 - k:, lo:lo + 2048].double() * r[:L - 2 + k, lo:lo + 2048].double()
+            exact = terms.sum(0)
+            err += (got[lo:lo + 2048, k] - exact).square().sum().item() - (2.0 ** -9 * exact).square().sum().item() / 3
+            terms2 += terms.square().sum().item()
+    assert err <= terms2 * (0.4 * 2.0 ** -24) ** 2 * (64 + 16) / 2
+
+
 def test_where_it_starts(gcg_lib):
     assert not one_kernel(1, 1023 * 32, 4, 16, 128, 3) and one_kernel(1, 1023 * 32 + 1, 4, 16, 128, 3)
     lib = _lib.load()
