@@ -22,6 +22,12 @@
 // ALUs, and half of a tile's products enter negated, so that the bias of one half is taken off by the other's: 1.4e-7,
 // and below the vector kernels' error at every shape compared, for 4 % of the backward's time.
 //
+// Infinities, NaN and values that round to an infinite bf16: the products multiply samples with the zeros around the
+// band, and a plane of such a value is infinite or NaN.  Whatever the sample, some y2 or du of the run is then not finite;
+// a workgroup that met one does its run once more on the vector ALUs, tap by tap in fp32 and with the sums of the filter
+// gradient cut the same way: a sample then reaches the rows its taps reach and no other.  Looking at the results costs
+// 1 % of the kernels' time, at the samples (their largest magnitude) 4 %.
+//
 // A workgroup owns CB adjacent channels and a run of 256-row tiles of one batch row; u (and g2) of a tile and of the
 // filter's reach stay in LDS as rings, so each row is read once (dy twice in the backward: for g2 OFF rows ahead, and
 // for dC).  What bounds it: the LDS reads of the operands and the transposition between the tensors' channel-fastest
@@ -52,7 +58,7 @@ template <int NK> struct Reach {
 // LDS bytes of a workgroup of cb channels touching nf filters; dirs = 1 (forward) or 2 (backward: two rings, two tables)
 constexpr int lds_bytes(int npa, int npw, int nk, int cb, int nf, int dirs)
 {
-    return dirs * npa * cb * (TT + 32 * nk - 16 + 8) * 2 + cb * YP * 4 + dirs * npw * nf * (32 * nk + 24) * 2;
+    return 16 + dirs * npa * cb * (TT + 32 * nk - 16 + 8) * 2 + cb * YP * 4 + dirs * npw * nf * (32 * nk + 24) * 2;
 }
 constexpr int LDS_MAX = 160 * 1024;
 // 32 channels (64-byte rows at 16 bits, 16 waves) where the rings and one filter per channel fit, else 16
@@ -216,6 +222,28 @@ __device__ __forceinline__ void band_product(f32x4 (&acc)[2], const uint16_t *ri
     }
 }
 
+__device__ __forceinline__ bool all_finite(const float (&v)[8])
+{
+    float z = 0.f;                               // NaN from the first value on that is not
+#pragma unroll
+    for (int e = 0; e < 8; ++e) z = fmaf(v[e], 0.f, z);
+    return z == 0.f;
+}
+// a[t] b[t] of one channel (rows ra, rb elements apart), zero outside the sequence
+template <typename T>
+__device__ __forceinline__ float product_at(const T *a, const T *b, int64_t ra, int64_t rb, int64_t t, int64_t L)
+{
+    return t >= 0 && t < L ? Elem<T>::load(a + t * ra) * Elem<T>::load(b + t * rb) : 0.f;
+}
+// one row of a channel: sum over lags of h[lag] times the sample DIR * lag rows on
+template <typename FT, int CB, int DIR> __device__ __forceinline__ float row_by_tap(const float *at, const FT *taps, int hl)
+{
+    float v = 0.f;
+#pragma unroll 1
+    for (int lag = 0; lag < hl; ++lag) v = fmaf(Elem<FT>::load(taps + (hl - 1 - lag)), at[DIR * lag * CB], v);
+    return v;
+}
+
 struct Plan {
     int nct, ntile, nseg, tps, nf;               // channel blocks, tiles of a row, runs, tiles per run, filters per block
     int64_t nwg;
@@ -244,7 +272,8 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
     typedef typename Filt<T>::type FT;
     constexpr int NPA = GT<T>::NPA, NT = 32 * CB;
     extern __shared__ __align__(16) unsigned char smem[];
-    uint16_t *ring = (uint16_t *)smem;
+    int *const flag = (int *)smem;                                        // the run has to be done again by taps
+    uint16_t *ring = (uint16_t *)(smem + 16);
     float *yt = (float *)(ring + NPA * CB * G::RP);
     uint16_t *tab = (uint16_t *)(yt + CB * YP);
 
@@ -271,6 +300,7 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
     const int64_t clast = min(c0 + CB, d) - 1;
     const int nf = (int)(clast / dm.dg - f0) + 1;
     const int fa = (int)(min(c0 + cw, clast) / dm.dg - f0), fb = (int)(min(c0 + cw + 1, clast) / dm.dg - f0);
+    if (tid == 0) *flag = 0;
     fill_taps<T, NK, false>(tab, (const FT *)h, f0, nf, dm.hl, tid, NT);
 
     int oldest = 0;                                                       // ring position of row t0 - OFF
@@ -312,6 +342,7 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
         float v[8];
         *(f32x4 *)v = *(const f32x4 *)(yt + cl * YP + 8 * tg);
         *(f32x4 *)(v + 4) = *(const f32x4 *)(yt + cl * YP + 8 * tg + 4);
+        if (!all_finite(v)) *flag = 1;
         if (y2)
 #pragma unroll
             for (int e = 0; e < 8; ++e) st_elem<T>(wy2, (row + e) * ro + co, v[e]);
@@ -322,6 +353,29 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
             st_elem<T>(wy, (row + e) * ro + co, cv * v[e]);
         }
         oldest = wrap<G::R>(oldest + TT);
+    }
+    __syncthreads();
+    if (*flag == 0) return;
+    // the run again by taps, each row by the thread that stored it: u of a tile and its reach as fp32, rows of CB
+    // (the index is hidden from the compiler: what follows from it shall not take registers of the loop above)
+    int again = tid;
+    asm volatile("" : "+v"(again));
+    const int cr = again % CB, tr = again / CB;
+    float *const us = (float *)ring;
+    const int64_t c = min(c0 + cr, clast), in0 = pl.b * dm.L * rowi + c * dm.es, out0 = pl.b * dm.L * d + c;
+    const FT *const taps = (const FT *)h + (c / dm.dg) * dm.hl;
+    for (int64_t t0 = T0; t0 < T1; t0 += TT) {
+        __syncthreads();
+        for (int r = tr; r < G::R; r += 32) us[r * CB + cr] = product_at<T>(x + in0, B + in0, rowi, rowi, t0 - G::OFF + r, dm.L);
+        __syncthreads();
+#pragma unroll 1
+        for (int r = 8 * tr; r < 8 * tr + 8; ++r) {
+            const int64_t t = t0 + r;
+            if (t >= T1 || c0 + cr >= d) break;
+            const float v = row_by_tap<FT, CB, -1>(us + (G::OFF + r) * CB + cr, taps, dm.hl);
+            if (y2) Elem<T>::store(y2 + out0 + t * d, v);
+            Elem<T>::store(y + out0 + t * d, Elem<T>::load(C + in0 + t * rowi) * v);
+        }
     }
 }
 
@@ -336,7 +390,8 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
     typedef typename Filt<T>::type FT;
     constexpr int NPA = GT<T>::NPA, NPW = GT<T>::NPW, NT = 32 * CB;
     extern __shared__ __align__(16) unsigned char smem[];
-    uint16_t *ru = (uint16_t *)smem, *rg = ru + NPA * CB * G::RP;
+    int *const flag = (int *)smem;
+    uint16_t *ru = (uint16_t *)(smem + 16), *rg = ru + NPA * CB * G::RP;
     float *yt = (float *)(rg + NPA * CB * G::RP);
     uint16_t *ta = (uint16_t *)(yt + CB * YP);
 
@@ -363,6 +418,7 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
     const int nf = (int)(clast / dm.dg - f0) + 1;
     const int fa = (int)(min(c0 + cw, clast) / dm.dg - f0), fb = (int)(min(c0 + cw + 1, clast) / dm.dg - f0);
     uint16_t *tb = ta + NPW * nf * G::HP;
+    if (tid == 0) *flag = 0;
     fill_taps<T, NK, false>(ta, (const FT *)h, f0, nf, dm.hl, tid, NT);
     fill_taps<T, NK, true>(tb, (const FT *)h, f0, nf, dm.hl, tid, NT);
 
@@ -420,6 +476,7 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         *(f32x4 *)(v + 4) = *(const f32x4 *)(yr + 4);
 #pragma unroll
         for (int e = 0; e < 8; ++e) st_elem<T>(wdC, (row + e) * ri + ci, raw_float<T>(rd[e]) * v[e]);
+        if (!all_finite(v)) *flag = 1;
         // filter gradient: 32 rows' products by themselves, added to the tile's sum and that to the run's; half of the
         // products with a negated operand (see the head of this file)
         f32x4 dt[2];
@@ -459,15 +516,55 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
             st_elem<T>(wdx, o, v[e] * bv);
             st_elem<T>(wdB, o, v[e] * xv);
         }
+        if (!all_finite(v)) *flag = 1;
         oldest = wrap<G::R>(oldest + TT);
         front = wrap<G::R>(front + TT);
     }
     // this run's filter gradient by lag: the channels of a filter added in their order
     __syncthreads();
+    if (*flag == 0) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) yt[(cw + c) * TT + (4 * q + r) * 16 + n] = dh[c][r];
+            for (int r = 0; r < 4; ++r) yt[(cw + c) * TT + (4 * q + r) * 16 + n] = dh[c][r];
+    } else {
+        // the run again by taps, each row by the thread that stored it and lags tr, tr + 32, ... of its channel: u and g2
+        // of a tile and their reach as fp32, rows of CB
+        int again = tid;
+        asm volatile("" : "+v"(again));
+        const int cr = again % CB, tr = again / CB;
+        float *const us = (float *)ru, *const gs = (float *)rg;
+        const int64_t c = min(c0 + cr, clast), in0 = pl.b * dm.L * rowi + c * dm.es, out0 = pl.b * dm.L * d + c;
+        const FT *const taps = (const FT *)h + (c / dm.dg) * dm.hl;
+        for (int lag = tr; lag < dm.hl; lag += 32) yt[cr * TT + lag] = 0.f;
+        for (int64_t t0 = T0; t0 < T1; t0 += TT) {
+            __syncthreads();
+            for (int r = tr; r < G::R; r += 32) {
+                us[r * CB + cr] = product_at<T>(x + in0, B + in0, rowi, rowi, t0 - G::OFF + r, dm.L);
+                gs[r * CB + cr] = product_at<T>(dy + out0, C + in0, d, rowi, t0 + r, dm.L);
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (int r = 8 * tr; r < 8 * tr + 8; ++r) {
+                const int64_t t = t0 + r, o = in0 + t * rowi;
+                if (t >= T1 || c0 + cr >= d) break;
+                Elem<T>::store(dC + o, Elem<T>::load(dy + out0 + t * d) *
+                                           row_by_tap<FT, CB, -1>(us + (G::OFF + r) * CB + cr, taps, dm.hl));
+                const float du = row_by_tap<FT, CB, 1>(gs + r * CB + cr, taps, dm.hl);
+                Elem<T>::store(dx + o, du * Elem<T>::load(B + o));
+                Elem<T>::store(dB + o, du * Elem<T>::load(x + o));
+            }
+#pragma unroll 1
+            for (int lag = tr; lag < dm.hl; lag += 32) {
+                const int a = lag & ~15, b = lag & 15;                     // as the products cut it: g2[s + a] u[s - b]
+                float s = yt[cr * TT + lag];
+#pragma unroll 1
+                for (int r = 0; r < TT; ++r)
+                    if (t0 + r + a < dm.L && t0 + r - b >= 0) s = fmaf(gs[(r + a) * CB + cr], us[(G::OFF + r - b) * CB + cr], s);
+                yt[cr * TT + lag] = s;
+            }
+        }
+    }
     __syncthreads();
     float *const slot = ws + (size_t)((pl.b * p.nseg + pl.seg) * p.nct + pl.ct) * p.nf * dm.hl;
     for (int i = tid; i < nf * dm.hl; i += NT) {

@@ -84,3 +84,67 @@ def test_filter_gradient_has_no_bias(gcg_lib, bs, L, g, dg, hl, types):
     u, g2 = x.double() * B.double(), dy.double() * C.double()
     exact = torch.stack([(g2[:, lag:] * u[:, :L - lag]).sum((0, 1, 3)) for lag in reversed(range(hl))], dim=1)
     assert (dh - exact).norm() <= 2.0 ** -24 * (1.5 + (bs * L / 64 / 6) ** 0.5) * exact.norm()
+
+
+def _taps_form(u, taps, step):
+    """Sum over lags of taps[lag] * u[t - step * lag] in 64 bits, zero outside the sequence: where a term is infinite or NaN
+    the sum is, and nowhere else."""
+    out, L = torch.zeros_like(u), u.shape[1]
+    for lag in range(taps.shape[1]):
+        past = torch.zeros_like(u)
+        if step > 0:
+            past[:, lag:] = u[:, :max(L - lag, 0)]
+        else:
+            past[:, :max(L - lag, 0)] = u[:, lag:]
+        out += past * taps[:, lag].view(1, 1, -1, 1)
+    return out
+
+
+@pytest.mark.parametrize("types", list(TYPES))
+@pytest.mark.parametrize("where", ["x", "dy", "h"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), "large"])
+@pytest.mark.parametrize("bs,L,g,dg,hl", [(2, 300, 5, 3, 17), (1, 1500, 3, 10, 100), (1, 700, 20, 2, 256)])
+def test_values_beyond_the_finite_range(gcg_lib, bs, L, g, dg, hl, value, where, types):
+    """An infinity or NaN reaches the rows its taps reach and no other, as the kind it is in the tap-by-tap sum, and what
+    stays finite is as exact as ever; the largest finite values give finite products."""
+    dtype, filt = TYPES[types]
+    gen = torch.Generator().manual_seed(hl)
+    x, B, C, dy = (torch.randn(bs, L, g, dg, generator=gen).to(dtype) for _ in range(4))
+    h = (torch.rand(g, 1, hl, generator=gen) / hl + 0.1 / hl).to(filt or dtype)
+    if value == "large":
+        value = torch.finfo((filt or dtype) if where == "h" else dtype).max
+        B[:, L // 2], C[:, L // 2], C[:, L - 1] = 1, 1, 1            # (the sample itself is the large value)
+        if where == "h":
+            x, dy = x / 16, dy / 16
+    t = {"x": x, "dy": dy, "h": h}[where]
+    if where == "h":
+        t[g // 2, 0, hl // 2] = value
+    else:
+        for b, row, c in ((0, L // 2, 1), (bs - 1, L - 1, 0)):
+            t[b, row, g // 2, c] = value
+    dev = [v.to(DEV) for v in (x, B, C, h)]
+    bx, y2, y = _lib.fwd(*dev, return_bx=True, return_y2=True)
+    dx, dB, dC, dh = _lib.bwd(dy.to(DEV), *dev)
+    # the gated products are fp32 in the kernels: an infinite one may be a finite 64-bit value
+    u, g2 = (x.float() * B.float()).double(), (dy.float() * C.float()).double()
+    taps = h[:, 0].double().flip(-1)                                 # by lag
+    ry2, rdu = _taps_form(u, taps, 1), _taps_form(g2, taps, -1)
+    terms = [g2[:, lag:] * u[:, :max(L - lag, 0)] for lag in reversed(range(hl))]
+    rdh = torch.stack([t.sum((0, 1, 3)) for t in terms], dim=1)
+    most = torch.stack([t.abs().sum((0, 1, 3)) for t in terms], dim=1)    # (partial sums of dh may pass the limit where it does not)
+    big = torch.finfo(torch.float32).max
+    for name, got, ref in (("y2", y2, ry2), ("y", y, C.double() * ry2), ("dx", dx, B.double() * rdu), ("dB", dB, x.double() * rdu),
+                           ("dC", dC, dy.double() * ry2), ("dh", dh[:, 0], rdh)):
+        got, limit = got.cpu(), torch.finfo(got.dtype).max
+        sure = ~((ref.abs() > limit / 4) & (ref.abs() < 4 * big))        # (around the type's limit either is right)
+        if name == "dh":
+            sure &= ~(most.isfinite() & (most > big / 4))
+        ref = torch.where(ref.abs() > limit, ref * float("inf"), ref)
+        fin = ref.isfinite()
+        assert torch.equal(got.isfinite()[sure], fin[sure]), name
+        if name != "dh":                                                 # (its order of summation decides between inf and NaN)
+            kind = sure & ~fin
+            assert torch.equal(got[kind].isnan(), ref[kind].isnan()), name
+            assert torch.equal(got[kind].double().nan_to_num(0, 1, -1), ref[kind].nan_to_num(0, 1, -1)), name
+        small = fin & (ref.abs() < 1e4) & got.isfinite()
+        assert_close(got[small], ref[small], BAR[got.dtype], name)
