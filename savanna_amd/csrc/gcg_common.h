@@ -283,7 +283,7 @@ inline int launch_packed(const void *fn, dim3 grid, dim3 block, hipStream_t st, 
                          std::tuple<KArgs...> &vals, std::index_sequence<I...>, size_t lds = 0)
 {
     void *ptrs[] = {(void *)&std::get<I>(vals)...};
-    if (t.start && t.stop)
+    if (t.start || t.stop)
         return (int)hipExtLaunchKernel(fn, grid, block, ptrs, lds, st, t.start, t.stop, 0);
     return (int)hipLaunchKernel(fn, grid, block, ptrs, lds, st);
 }
@@ -306,13 +306,14 @@ inline int launch_main(void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStrea
                          std::index_sequence_for<KArgs...>{});
 }
 
-// the same with `lds` bytes of dynamic LDS
+// the same with `lds` bytes of dynamic LDS; t: the caller's event pair, or one event of it at the first and the last of
+// several launches
 template <typename... KArgs, typename... Args>
-inline int launch_main_lds(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds, hipStream_t st, Args... args)
+inline int launch_main_lds(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds, hipStream_t st, const KernelTimer &t,
+                           Args... args)
 {
     std::tuple<KArgs...> vals{static_cast<KArgs>(args)...};
-    return launch_packed((const void *)kernel, grid, block, st, take_kernel_timer(), vals,
-                         std::index_sequence_for<KArgs...>{}, lds);
+    return launch_packed((const void *)kernel, grid, block, st, t, vals, std::index_sequence_for<KArgs...>{}, lds);
 }
 
 int direct_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h,
@@ -322,13 +323,14 @@ int direct_bwd_launch(int dtype, const void *dy, const void *x, const void *B, c
                       const void *h, void *dx, void *dB, void *dC, void *dh, void *ws,
                       const Dims &dm, hipStream_t st);
 
-// matrix-core kernels of the general family: filters of 9 to 256 taps, any group width and element alignment
-bool toep_supported(int dtype, const Dims &dm, bool backward);
+// Matrix-core kernels of the general family: filters of 9 to 256 taps, any group width and element alignment.  Sizes they
+// do not take are answered with TOEP_NOT_TAKEN and a workspace of 0; vector_bytes is the workspace of the vector kernels.
+constexpr int TOEP_NOT_TAKEN = -1;
 int toep_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
                     const Dims &dm, hipStream_t st);
-size_t toep_bwd_workspace(int dtype, const Dims &dm);
+size_t toep_bwd_workspace(int dtype, const Dims &dm, size_t vector_bytes);
 int toep_bwd_launch(int dtype, const void *dy, const void *x, const void *B, const void *C, const void *h, void *dx,
-                    void *dB, void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st);
+                    void *dB, void *dC, void *dh, void *ws, const Dims &dm, size_t vector_bytes, hipStream_t st);
 
 bool window_supported(const Dims &dm);
 int window_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h,

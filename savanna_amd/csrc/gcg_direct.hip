@@ -280,6 +280,8 @@ BwdPlan plan_bwd(const Dims &dm)
     return p;
 }
 
+size_t workspace_bytes(const BwdPlan &p, const Dims &dm) { return (size_t)p.nwg * p.gpt * dm.hl * sizeof(float); }
+
 template <typename T>
 int fwd_t(const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
           const Dims &dm, hipStream_t st)
@@ -315,7 +317,8 @@ int bwd_t(const void *dy, const void *x, const void *B, const void *C, const voi
 int direct_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h, void *y,
                       void *y2, void *bx, const Dims &dm, hipStream_t st)
 {
-    if (toep_supported(dtype, dm, false)) return toep_fwd_launch(dtype, x, B, C, h, y, y2, bx, dm, st);
+    const int e = toep_fwd_launch(dtype, x, B, C, h, y, y2, bx, dm, st);
+    if (e != TOEP_NOT_TAKEN) return e;
     switch (dtype) {
     case GCG_F32:  return fwd_t<float>(x, B, C, h, y, y2, bx, dm, st);
     case GCG_BF16: return fwd_t<bf16_t>(x, B, C, h, y, y2, bx, dm, st);
@@ -328,15 +331,15 @@ int direct_fwd_launch(int dtype, const void *x, const void *B, const void *C, co
 
 size_t direct_bwd_workspace(int dtype, const Dims &dm)
 {
-    if (toep_supported(dtype, dm, true)) return toep_bwd_workspace(dtype, dm);
-    const BwdPlan p = plan_bwd(dm);
-    return (size_t)p.nwg * p.gpt * dm.hl * sizeof(float);
+    const size_t vector = workspace_bytes(plan_bwd(dm), dm), n = toep_bwd_workspace(dtype, dm, vector);
+    return n ? n : vector;
 }
 
 int direct_bwd_launch(int dtype, const void *dy, const void *x, const void *B, const void *C, const void *h,
                       void *dx, void *dB, void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st)
 {
-    if (toep_supported(dtype, dm, true)) return toep_bwd_launch(dtype, dy, x, B, C, h, dx, dB, dC, dh, ws, dm, st);
+    const int e = toep_bwd_launch(dtype, dy, x, B, C, h, dx, dB, dC, dh, ws, dm, workspace_bytes(plan_bwd(dm), dm), st);
+    if (e != TOEP_NOT_TAKEN) return e;
     switch (dtype) {
     case GCG_F32:  return bwd_t<float>(dy, x, B, C, h, dx, dB, dC, dh, ws, dm, st);
     case GCG_BF16: return bwd_t<bf16_t>(dy, x, B, C, h, dx, dB, dC, dh, ws, dm, st);

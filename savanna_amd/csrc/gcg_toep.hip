@@ -246,7 +246,8 @@ template <typename FT, int CB, int DIR> __device__ __forceinline__ float row_by_
 
 struct Plan {
     int nct, ntile, nseg, tps, nf;               // channel blocks, tiles of a row, runs, tiles per run, filters per block
-    int64_t nwg;
+    int64_t rows, b0;                            // batch rows of a launch, and its first
+    int64_t nwg;                                 // workgroups of a launch
 };
 
 // where a workgroup is: channel block fastest, then run, then batch row, contiguous per XCD so that the
@@ -258,7 +259,7 @@ __device__ __forceinline__ Place place(const Plan &p)
     Place r;
     r.ct = (int)(id % (uint32_t)p.nct); id /= (uint32_t)p.nct;
     r.seg = (int)(id % (uint32_t)p.nseg);
-    r.b = id / (uint32_t)p.nseg;
+    r.b = p.b0 + id / (uint32_t)p.nseg;
     return r;
 }
 
@@ -566,18 +567,18 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         }
     }
     __syncthreads();
-    float *const slot = ws + (size_t)((pl.b * p.nseg + pl.seg) * p.nct + pl.ct) * p.nf * dm.hl;
+    float *const slot = ws + (size_t)(((pl.b - p.b0) * p.nseg + pl.seg) * p.nct + pl.ct) * p.nf * dm.hl;
     for (int i = tid; i < nf * dm.hl; i += NT) {
         const int f = i / dm.hl, k = i - f * dm.hl;
         const int64_t lo = (f0 + f) * dm.dg - c0, hi = lo + dm.dg;
         const int a = (int)max((int64_t)0, lo), b = (int)min(hi, clast + 1 - c0);
         float s = 0.f;
         for (int c = a; c < b; ++c) s += yt[c * TT + dm.hl - 1 - k];
-        slot[i] = s;
+        slot[i] = p.b0 ? slot[i] + s : s;
     }
 }
 
-// dh[grp, k] = sum over batch rows, runs and the channel blocks that touch the group, in that order
+// dh[grp, k] = sum over the batch rows of a launch, runs and the channel blocks that touch the group, in that order
 template <typename FT>
 __global__ __launch_bounds__(64) void toep_dh_kernel(const float *__restrict__ ws, FT *__restrict__ dh, Dims dm, Plan p,
                                                      int cb)
@@ -590,7 +591,7 @@ __global__ __launch_bounds__(64) void toep_dh_kernel(const float *__restrict__ w
     for (int64_t ct = lo; ct <= hi; ++ct) {
         const int64_t f = grp - ct * cb / dm.dg;
         const float *w = ws + (ct * p.nf + f) * dm.hl + k;
-        const int64_t step = (int64_t)p.nct * p.nf * dm.hl, n = dm.bs * p.nseg;
+        const int64_t step = (int64_t)p.nct * p.nf * dm.hl, n = p.rows * p.nseg;
         int64_t r = 0;
         for (; r + 8 <= n; r += 8) {
             float v[8];
@@ -608,18 +609,24 @@ int pick_nk(int hl) { return hl <= 17 ? 1 : hl <= 81 ? 3 : hl <= 145 ? 5 : 9; }
 int npa_of(int dtype) { return dtype == GCG_BF16 || dtype == GCG_BF16_F32 ? 2 : 3; }
 int npw_of(int dtype) { return dtype == GCG_BF16 ? 1 : dtype == GCG_F16 ? 2 : 3; }
 
-Plan make_plan(int dtype, const Dims &dm, int dirs)
+// vector_bytes: what the vector kernels' backward of these sizes keeps partial sums in.  False: sizes for those kernels.
+bool make_plan(int dtype, const Dims &dm, int dirs, size_t vector_bytes, Plan &p)
 {
-    const int nk = pick_nk(dm.hl), cb = pick_cb(npa_of(dtype), npw_of(dtype), nk, dirs);
-    Plan p;
+    if (dm.hl < 9 || dm.hl > 256 || dm.tmajor) return false;
+    const int npa = npa_of(dtype), npw = npw_of(dtype), nk = pick_nk(dm.hl), cb = pick_cb(npa, npw, nk, dirs);
     p.nct = (int)((dm.d + cb - 1) / cb);
     p.ntile = (int)((dm.L + TT - 1) / TT);
+    p.nf = (int)((cb - 1) / dm.dg + 2 < cb ? (cb - 1) / dm.dg + 2 : cb);
+    if (cb % dm.dg == 0) p.nf = cb / dm.dg;
+    else if (dm.dg % cb == 0) p.nf = 1;
+    if (lds_bytes(npa, npw, nk, cb, p.nf, dirs) > LDS_MAX) return false;
     const int64_t cols = dm.bs * p.nct;
     // rows of a run: what a window spans (with the reach on both sides; the workspace query does not know the layout,
     // so always that of a features tensor), and no more tiles than there are
     const int64_t esz = dtype == GCG_F32 ? 4 : 2, rowb = 3 * dm.d * esz;
     int64_t cap = (WIN_MAX_BYTES / rowb - 2 * (32 * nk - 16)) / TT;
     if (cap > p.ntile) cap = p.ntile;
+    if (cap <= 0) return false;
     // as many runs as make rounds of 256 workgroups x (tiles of a run + the reach it loads first) smallest
     int64_t best = -1;
     p.tps = 0;
@@ -630,12 +637,22 @@ Plan make_plan(int dtype, const Dims &dm, int dirs)
         if (best < 0 || cost <= best) { best = cost; p.tps = (int)tps; }
         if (tps >= 64) tps += tps / 16;
     }
-    p.nseg = p.tps ? (p.ntile + p.tps - 1) / p.tps : 0;
-    p.nf = (int)((cb - 1) / dm.dg + 2 < cb ? (cb - 1) / dm.dg + 2 : cb);
-    if (cb % dm.dg == 0) p.nf = cb / dm.dg;
-    else if (dm.dg % cb == 0) p.nf = 1;
-    p.nwg = cols * p.nseg;
-    return p;
+    p.nseg = (p.ntile + p.tps - 1) / p.tps;
+    p.rows = dm.bs;
+    p.b0 = 0;
+    // A backward whose partial sums the static scratch held with the vector kernels' blocks of 64 channels and does not
+    // with these of 16 or 32 is launched for a part of the batch rows at a time, each launch adding to the sums of the
+    // one before, here and with a workspace alike (21 x 160 x (256 groups of 32), 256 taps, bf16: 10.5 MB and 537 us in
+    // one launch, 5.5 MB in two and 1 % more time).
+    const size_t row_bytes = (size_t)p.nct * p.nseg * p.nf * dm.hl * sizeof(float);
+    if (dirs == 2 && vector_bytes <= GCG_BWD_STATIC_SCRATCH_BYTES && dm.bs * row_bytes > GCG_BWD_STATIC_SCRATCH_BYTES) {
+        const int64_t rows = (int64_t)(GCG_BWD_STATIC_SCRATCH_BYTES / row_bytes);
+        if (rows == 0) return false;
+        const int64_t launches = (dm.bs + rows - 1) / rows;
+        p.rows = (dm.bs + launches - 1) / launches;
+    }
+    p.nwg = p.rows * p.nct * p.nseg;
+    return p.nwg <= 0x7fffffffLL;
 }
 
 template <typename T, int NK>
@@ -644,8 +661,8 @@ int fwd_nk(const void *x, const void *B, const void *C, const void *h, void *y, 
 {
     constexpr int CB = pick_cb(GT<T>::NPA, GT<T>::NPW, NK, 1);
     return launch_main_lds(toep_fwd_kernel<T, NK, CB>, dim3((unsigned)p.nwg), dim3(32 * CB),
-                           lds_bytes(GT<T>::NPA, GT<T>::NPW, NK, CB, p.nf, 1), st, (const T *)x, (const T *)B, (const T *)C,
-                           h, (T *)y, (T *)y2, (T *)bx, dm, p);
+                           lds_bytes(GT<T>::NPA, GT<T>::NPW, NK, CB, p.nf, 1), st, take_kernel_timer(), (const T *)x,
+                           (const T *)B, (const T *)C, h, (T *)y, (T *)y2, (T *)bx, dm, p);
 }
 
 template <typename T, int NK>
@@ -654,10 +671,15 @@ int bwd_nk(const void *dy, const void *x, const void *B, const void *C, const vo
 {
     constexpr int CB = pick_cb(GT<T>::NPA, GT<T>::NPW, NK, 2);
     typedef typename Filt<T>::type FT;
-    const int e = launch_main_lds(toep_bwd_kernel<T, NK, CB>, dim3((unsigned)p.nwg), dim3(32 * CB),
-                                  lds_bytes(GT<T>::NPA, GT<T>::NPW, NK, CB, p.nf, 2), st, (const T *)dy, (const T *)x,
-                                  (const T *)B, (const T *)C, h, (T *)dx, (T *)dB, (T *)dC, (float *)ws, dm, p);
-    if (e) return e;
+    const KernelTimer timer = take_kernel_timer();
+    for (Plan q = p; q.b0 < dm.bs; q.b0 += q.rows) {
+        const int64_t nwg = p.nwg / p.rows * min(p.rows, dm.bs - q.b0);
+        const KernelTimer t = {q.b0 ? nullptr : timer.start, q.b0 + q.rows < dm.bs ? nullptr : timer.stop};
+        const int e = launch_main_lds(toep_bwd_kernel<T, NK, CB>, dim3((unsigned)nwg), dim3(32 * CB),
+                                      lds_bytes(GT<T>::NPA, GT<T>::NPW, NK, CB, p.nf, 2), st, t, (const T *)dy, (const T *)x,
+                                      (const T *)B, (const T *)C, h, (T *)dx, (T *)dB, (T *)dC, (float *)ws, dm, q);
+        if (e) return e;
+    }
     const int64_t n = (int64_t)dm.g * dm.hl;
     return launch_plain(toep_dh_kernel<FT>, dim3((unsigned)((n + 63) / 64)), dim3(64), st, (const float *)ws, (FT *)dh, dm, p,
                         CB);
@@ -684,19 +706,11 @@ template <typename T, typename... A> int bwd_t(int hl, A... a)
 
 } // namespace
 
-bool toep_supported(int dtype, const Dims &dm, bool backward)
-{
-    if (dm.hl < 9 || dm.hl > 256 || dm.tmajor) return false;
-    const int nk = pick_nk(dm.hl), dirs = backward ? 2 : 1;
-    const int cb = pick_cb(npa_of(dtype), npw_of(dtype), nk, dirs);
-    const Plan p = make_plan(dtype, dm, dirs);
-    return p.tps > 0 && p.nwg <= 0x7fffffffLL && lds_bytes(npa_of(dtype), npw_of(dtype), nk, cb, p.nf, dirs) <= LDS_MAX;
-}
-
 int toep_fwd_launch(int dtype, const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
                     const Dims &dm, hipStream_t st)
 {
-    const Plan p = make_plan(dtype, dm, 1);
+    Plan p;
+    if (!make_plan(dtype, dm, 1, 0, p)) return TOEP_NOT_TAKEN;
     switch (dtype) {
     case GCG_F32:  return fwd_t<float>(dm.hl, x, B, C, h, y, y2, bx, dm, p, st);
     case GCG_BF16: return fwd_t<bf16_t>(dm.hl, x, B, C, h, y, y2, bx, dm, p, st);
@@ -707,16 +721,17 @@ int toep_fwd_launch(int dtype, const void *x, const void *B, const void *C, cons
     return (int)hipErrorInvalidValue;
 }
 
-size_t toep_bwd_workspace(int dtype, const Dims &dm)
+size_t toep_bwd_workspace(int dtype, const Dims &dm, size_t vector_bytes)
 {
-    const Plan p = make_plan(dtype, dm, 2);
-    return (size_t)p.nwg * p.nf * dm.hl * sizeof(float);
+    Plan p;
+    return make_plan(dtype, dm, 2, vector_bytes, p) ? (size_t)p.nwg * p.nf * dm.hl * sizeof(float) : 0;
 }
 
 int toep_bwd_launch(int dtype, const void *dy, const void *x, const void *B, const void *C, const void *h, void *dx,
-                    void *dB, void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st)
+                    void *dB, void *dC, void *dh, void *ws, const Dims &dm, size_t vector_bytes, hipStream_t st)
 {
-    const Plan p = make_plan(dtype, dm, 2);
+    Plan p;
+    if (!make_plan(dtype, dm, 2, vector_bytes, p)) return TOEP_NOT_TAKEN;
     switch (dtype) {
     case GCG_F32:  return bwd_t<float>(dm.hl, dy, x, B, C, h, dx, dB, dC, dh, ws, dm, p, st);
     case GCG_BF16: return bwd_t<bf16_t>(dm.hl, dy, x, B, C, h, dx, dB, dC, dh, ws, dm, p, st);

@@ -148,3 +148,28 @@ def test_values_beyond_the_finite_range(gcg_lib, bs, L, g, dg, hl, value, where,
             assert torch.equal(got[kind].double().nan_to_num(0, 1, -1), ref[kind].nan_to_num(0, 1, -1)), name
         small = fin & (ref.abs() < 1e4) & got.isfinite()
         assert_close(got[small], ref[small], BAR[got.dtype], name)
+
+
+@pytest.mark.parametrize("types", ["f32", "bf16"])
+@pytest.mark.parametrize("bs,L,g,dg,hl", [(36, 4, 52, 54, 246), (6, 5, 653, 12, 255), (84, 20, 64, 32, 256)])
+def test_backward_in_several_launches(gcg_lib, bs, L, g, dg, hl, types):
+    """Batches launched in parts so that the sums of dh fit the static scratch: as exact as in one launch, with the same
+    bits from the static scratch and from a workspace, and timed from the first launch to the end of the last."""
+    dtype, filt = TYPES[types]
+    gen = torch.Generator().manual_seed(hl)
+    x, B, C, dy = (torch.randn(bs, L, g, dg, generator=gen).to(dtype) for _ in range(4))
+    h = (torch.randn(g, 1, hl, generator=gen) / hl ** 0.5).to(filt or dtype)
+    dev = [t.to(DEV) for t in (dy, x, B, C, h)]
+    start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    start.record(), stop.record()                    # (creates them)
+    got = _lib.bwd(*dev)
+    torch.cuda.synchronize()
+    _lib.time_next_kernel(start.cuda_event, stop.cuda_event)
+    again = [torch.full_like(t, float("nan")) for t in got]
+    _lib.bwd_static(*dev, *again)
+    torch.cuda.synchronize()
+    assert 0 < start.elapsed_time(stop) < 1000
+    for a, b in zip(got, again):
+        assert torch.equal(a, b)
+    for o, r, n in zip(got, oracle_bwd(dy, x, B, C, h), ("dx", "dB", "dC", "dh")):
+        assert_close(o, r, TOL_DH[dtype] if n == "dh" else BAR[dtype], n)

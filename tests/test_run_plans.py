@@ -1,4 +1,4 @@
-"""How the matrix-core backward cuts a sequence into runs, seen through the scratch its partial sums need."""
+"""How the matrix-core backwards cut their work into runs and launches, seen through the scratch their partial sums need."""
 import pytest
 
 from savanna_amd import _lib
@@ -6,8 +6,19 @@ from savanna_amd import _lib
 STATIC = _lib.STATIC_SCRATCH_BYTES
 
 
+CODES = [_lib.GCG_F32, _lib.GCG_BF16, _lib.GCG_F16, _lib.GCG_BF16_F32, _lib.GCG_F16_F32]
+
+
 def scratch(bs, L, g, hl):
     return _lib.load().gcg_bwd_workspace_bytes(bs, L, g, 16, hl, _lib.GCG_BF16, _lib.ALGO_MFMA)
+
+
+def vector_scratch(bs, L, g, dg, hl):
+    """The vector kernels': one slot of a filter for each that a block of 64 channels touches, runs of 64 rows or more."""
+    blocks, tiles = (g * dg + 63) // 64, (L + 63) // 64
+    tps = -(-tiles // min(max(4096 // (bs * blocks), 1), tiles))
+    filters = 64 // dg if 64 % dg == 0 else min(63 // dg + 2, 64)
+    return -(-bs * -(-tiles // tps) * blocks * filters * hl * 4 // 256) * 256
 
 
 @pytest.mark.parametrize("bs,nsteps,hl", [(854, 75, 9), (858, 75, 9), (1023, 31, 9), (257, 63, 128), (769, 63, 33),
@@ -22,3 +33,14 @@ def test_static_scratch_holds_what_it_held(bs, nsteps, hl):
 def test_small_launches_stay_far_below_it(cols, hl):
     for nsteps in (1, 7, 16, 31, 75, 200):
         assert 0 < scratch(cols, 32 * nsteps, 4, hl) <= 2304 * 2048 + 4096
+
+
+@pytest.mark.parametrize("code", CODES)
+@pytest.mark.parametrize("bs,L,g,dg,hl", [(21, 160, 256, 32, 256), (49, 1, 64, 24, 256), (6, 5, 653, 12, 255), (47, 189, 124, 63, 111),
+                                          (22, 215, 147, 43, 226), (127, 1634, 839, 6, 15), (36, 4, 52, 54, 246),
+                                          (1, 100, 8000, 64, 255), (3, 7, 2730, 64, 250)])
+def test_general_family_stays_in_static_scratch(code, bs, L, g, dg, hl):
+    """Where the vector kernels' sums fit it, those of the matrix-core kernels with their narrower blocks do too."""
+    assert vector_scratch(bs, L, g, dg, hl) <= STATIC
+    for algo in (_lib.ALGO_NAMES["direct"], _lib.ALGO_AUTO):
+        assert 0 < _lib.load().gcg_bwd_workspace_bytes(bs, L, g, dg, hl, code, algo) <= STATIC
