@@ -652,7 +652,7 @@ bool make_plan(int dtype, const Dims &dm, int dirs, size_t vector_bytes, Plan &p
         p.rows = (dm.bs + launches - 1) / launches;
     }
     p.nwg = p.rows * p.nct * p.nseg;
-    return p.nwg <= 0x7fffffffLL;
+    return p.nwg * 32 * cb <= 0xffffffffLL;      // work-items of a launch
 }
 
 template <typename T, int NK>

@@ -44,3 +44,11 @@ def test_general_family_stays_in_static_scratch(code, bs, L, g, dg, hl):
     assert vector_scratch(bs, L, g, dg, hl) <= STATIC
     for algo in (_lib.ALGO_NAMES["direct"], _lib.ALGO_AUTO):
         assert 0 < _lib.load().gcg_bwd_workspace_bytes(bs, L, g, dg, hl, code, algo) <= STATIC
+
+
+def test_launches_beyond_the_grid_stay_with_the_vector_kernels():
+    """A launch holds 2^32 - 1 work-items.  65536 rows of 65 blocks in workgroups of 1024 are more: the vector kernels' 33
+    blocks in workgroups of 256 are not."""
+    size = lambda *s: _lib.load().gcg_bwd_workspace_bytes(*s, _lib.GCG_BF16, _lib.ALGO_NAMES["direct"])
+    assert size(65536, 16, 86, 24, 64) == vector_scratch(65536, 16, 86, 24, 64)
+    assert size(63000, 16, 86, 24, 64) != vector_scratch(63000, 16, 86, 24, 64)
