@@ -1,6 +1,7 @@
 // C ABI (include/gcg.h): argument checks, kernel-family selection, launch.
 #include "gcg_common.h"
 
+#include <algorithm>
 #include <initializer_list>
 #include <mutex>
 
@@ -222,15 +223,11 @@ GCG_API size_t gcg_bwd_workspace_bytes(int64_t bs, int64_t L, int32_t g, int32_t
     gcg::Dims dm;
     if (make_dims(bs, L, g, dg, hl, dtype, &dm, true)) return 0;
     const int a = resolve_algo(algo, dtype, dm, true);
-    size_t n = 0;
-    switch (a) {
-    case GCG_ALGO_DIRECT: n = gcg::direct_bwd_workspace(dtype, dm); break;
-    case GCG_ALGO_WINDOW: n = gcg::window_bwd_workspace(dm); break;
-    case GCG_ALGO_MFMA:   n = gcg::mfma_bwd_workspace(dtype, dm); break;
-    default: return 0;
-    }
+    if (a < 0) return 0;
     // under AUTO a misaligned tensor reroutes to the direct kernels: size for both
-    if (algo == GCG_ALGO_AUTO && gcg::direct_bwd_workspace(dtype, dm) > n) n = gcg::direct_bwd_workspace(dtype, dm);
+    size_t n = a == GCG_ALGO_DIRECT || algo == GCG_ALGO_AUTO ? gcg::direct_bwd_workspace(dtype, dm) : 0;
+    if (a == GCG_ALGO_WINDOW) n = std::max(n, gcg::window_bwd_workspace(dm));
+    if (a == GCG_ALGO_MFMA) n = std::max(n, gcg::mfma_bwd_workspace(dtype, dm));
     return (n + 255) & ~(size_t)255;
 }
 

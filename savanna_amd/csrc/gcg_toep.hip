@@ -609,6 +609,23 @@ int pick_nk(int hl) { return hl <= 17 ? 1 : hl <= 81 ? 3 : hl <= 145 ? 5 : 9; }
 int npa_of(int dtype) { return dtype == GCG_BF16 || dtype == GCG_BF16_F32 ? 2 : 3; }
 int npw_of(int dtype) { return dtype == GCG_BF16 ? 1 : dtype == GCG_F16 ? 2 : 3; }
 
+// Tiles per run, at most cap: as many runs as make rounds of one workgroup per CU x (tiles of a run + the reach it loads
+// first) smallest.  For a number of rounds the best run is the shortest that needs no more; no more rounds are tried once
+// their leads alone, on top of the work spread evenly, cost what the best cut does (two or three as a rule: the query that
+// sizes a backward's workspace comes through here on every call).
+int pick_tps(int64_t cols, int64_t ntile, int64_t cap, int64_t cus, int lead)
+{
+    const int64_t fewest = (ntile + cap - 1) / cap, least = cols * ntile * TT / cus;
+    int64_t rounds = (cols * fewest + cus - 1) / cus, best = INT64_MAX, tps = cap;
+    for (int64_t tries = 0; tries < 64 && least + rounds * lead < best; ++tries, ++rounds) {
+        int64_t runs = rounds * cus / cols;
+        if (runs > ntile) runs = ntile;
+        const int64_t n = (ntile + runs - 1) / runs, cost = rounds * (n * TT + lead);
+        if (cost < best) { best = cost; tps = n; }
+    }
+    return (int)tps;
+}
+
 // vector_bytes: what the vector kernels' backward of these sizes keeps partial sums in.  False: sizes for those kernels.
 bool make_plan(int dtype, const Dims &dm, int dirs, size_t vector_bytes, Plan &p)
 {
@@ -622,21 +639,15 @@ bool make_plan(int dtype, const Dims &dm, int dirs, size_t vector_bytes, Plan &p
     if (lds_bytes(npa, npw, nk, cb, p.nf, dirs) > LDS_MAX) return false;
     const int64_t cols = dm.bs * p.nct;
     // rows of a run: what a window spans (with the reach on both sides; the workspace query does not know the layout,
-    // so always that of a features tensor), and no more tiles than there are
+    // so always that of a features tensor), no more tiles than there are, and 256: the tiles' sums of the filter gradient
+    // are added one after the other (a run's lead is 0.3 % of that)
     const int64_t esz = dtype == GCG_F32 ? 4 : 2, rowb = 3 * dm.d * esz;
     int64_t cap = (WIN_MAX_BYTES / rowb - 2 * (32 * nk - 16)) / TT;
     if (cap > p.ntile) cap = p.ntile;
+    if (cap > 256) cap = 256;
     if (cap <= 0) return false;
-    // as many runs as make rounds of 256 workgroups x (tiles of a run + the reach it loads first) smallest
-    int64_t best = -1;
-    p.tps = 0;
-    for (int64_t tps = 1; tps <= cap; ++tps) {
-        const int64_t nseg = (p.ntile + tps - 1) / tps;
-        const int64_t rounds = (cols * nseg + 255) / 256;
-        const int64_t cost = rounds * (tps * TT + dirs * (32 * nk - 16) / 2 + 64);
-        if (best < 0 || cost <= best) { best = cost; p.tps = (int)tps; }
-        if (tps >= 64) tps += tps / 16;
-    }
+    const int lead = dirs * (32 * nk - 16) / 2 + 64;
+    p.tps = pick_tps(cols, p.ntile, cap, cu_count(), lead);
     p.nseg = (p.ntile + p.tps - 1) / p.tps;
     p.rows = dm.bs;
     p.b0 = 0;

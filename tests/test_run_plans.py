@@ -1,4 +1,6 @@
 """How the matrix-core backwards cut their work into runs and launches, seen through the scratch their partial sums need."""
+import time
+
 import pytest
 
 from savanna_amd import _lib
@@ -52,3 +54,21 @@ def test_launches_beyond_the_grid_stay_with_the_vector_kernels():
     size = lambda *s: _lib.load().gcg_bwd_workspace_bytes(*s, _lib.GCG_BF16, _lib.ALGO_NAMES["direct"])
     assert size(65536, 16, 86, 24, 64) == vector_scratch(65536, 16, 86, 24, 64)
     assert size(63000, 16, 86, 24, 64) != vector_scratch(63000, 16, 86, 24, 64)
+
+
+def test_query_for_either_alignment_costs_no_search():
+    """Under AUTO the query that every backward call makes also sizes for misaligned tensors; that takes a fraction of the
+    call (0.16 us against 0.12 of its own at a million rows, where a search over all run lengths took 1.3)."""
+    query = _lib.load().gcg_bwd_workspace_bytes
+
+    def best(*args):
+        times = []
+        for _ in range(40):
+            t = time.perf_counter()
+            for _ in range(500):
+                query(*args)
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    shape = (1, 1 << 20, 256, 16, 128, _lib.GCG_BF16)
+    assert best(*shape, _lib.ALGO_AUTO) < 1.6 * best(*shape, _lib.ALGO_MFMA)
