@@ -22,8 +22,8 @@
 // ALUs, and half of a tile's products enter negated, so that the bias of one half is taken off by the other's: 1.4e-7,
 // and below the vector kernels' error at every shape compared, for 4 % of the backward's time.
 //
-// Infinities, NaN and values that round to an infinite bf16: the products multiply samples with the zeros around the
-// band, and a plane of such a value is infinite or NaN.  Whatever the sample, some y2 or du of the run is then not finite;
+// Infinities, NaN and samples from 2^104 on (LIFT): the products multiply samples with the zeros around the band, and a
+// plane of such a value is infinite or NaN.  Whatever the sample, some y2 or du of the run is then not finite;
 // a workgroup that met one does its run once more on the vector ALUs, tap by tap in fp32 and with the sums of the filter
 // gradient cut the same way: a sample then reaches the rows its taps reach and no other.  Looking at the results costs
 // 1 % of the kernels' time, at the samples (their largest magnitude) 4 %.
@@ -34,6 +34,8 @@
 // rows and the channel-major rings, then memory.  Measured at 1 x 4096 x (256 groups of 8), 128 taps, bf16, against
 // gcg_direct.hip: forward 124 -> 21 us, backward 333 -> 57 us, its filter-gradient sum 27 -> 4 us.
 #include "gcg_mfma_tile.h"
+
+#include <type_traits>
 
 namespace gcg {
 namespace {
@@ -47,6 +49,10 @@ template <> struct GT<bf16_t> { static constexpr int NPA = 2, NPW = 1; };
 template <> struct GT<f16_t> { static constexpr int NPA = 3, NPW = 2; };
 template <> struct GT<bf16w_t> { static constexpr int NPA = 2, NPW = 3; };
 template <> struct GT<f16w_t> { static constexpr int NPA = 3, NPW = 3; };
+
+// Samples enter the rings times 2^24 and taps the tables times 2^-24: the last planes of a sample below 2^-110 would be
+// bf16 subnormals, and bits of it lost (f16's smallest product is 2^-48: no need)
+template <typename T> constexpr float LIFT = std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t> ? 1.f : 0x1p24f;
 
 template <int NK> struct Reach {
     static constexpr int OFF = 32 * NK - 16;     // rows of history (u) and look-ahead (g2) held beside a tile
@@ -151,15 +157,16 @@ template <int R> __device__ __forceinline__ int wrap(int pos)      // pos in [0,
 }
 
 // 8 samples of channel cl into every plane of a ring at position pos (a multiple of 8)
-template <int NPA, int NK, int CB>
+template <typename T, int NK, int CB>
 __device__ __forceinline__ void ring_store(uint16_t *ring, int cl, int pos, const float (&f)[8])
 {
     typedef Reach<NK> G;
+    constexpr int NPA = GT<T>::NPA;
     uint16_t v[NPA][8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         uint16_t o[NPA];
-        split_planes<NPA>(f[e], o);
+        split_planes<NPA>(f[e] * LIFT<T>, o);
 #pragma unroll
         for (int m = 0; m < NPA; ++m) v[m][e] = o[m];
     }
@@ -188,7 +195,7 @@ __device__ __forceinline__ void fill_taps(uint16_t *tab, const typename Filt<T>:
         float v = 0.f;
         if (lag >= 0 && lag < hl) v = Elem<FT>::load(h + (f0 + f) * hl + (hl - 1 - lag));
         uint16_t o[NPW];
-        split_planes<NPW>(v, o);
+        split_planes<NPW>(v * (1.f / LIFT<T>), o);
 #pragma unroll
         for (int m = 0; m < NPW; ++m) tab[(m * nf + f) * G::HP + z + 16] = o[m];
     }
@@ -312,7 +319,7 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
             const uint32_t off = (uint32_t)(int32_t)(T0 - G::OFF - tw + 8 * g + e) * ri + ci;
             u[e] = raw_float<T>(ld_raw<T>(wx, off)) * raw_float<T>(ld_raw<T>(wB, off));
         }
-        ring_store<NPA, NK, CB>(ring, cl, 8 * g, u);
+        ring_store<T, NK, CB>(ring, cl, 8 * g, u);
     }
     uint32_t rx[8], rB[8], rC[8];
     uint32_t row = (uint32_t)(T0 - tw) + 8 * tg;                          // first row of the thread, from tw
@@ -325,7 +332,7 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
         float u[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) u[e] = raw_float<T>(rx[e]) * raw_float<T>(rB[e]);
-        ring_store<NPA, NK, CB>(ring, cl, wrap<G::R>(oldest + G::OFF + 8 * tg), u);
+        ring_store<T, NK, CB>(ring, cl, wrap<G::R>(oldest + G::OFF + 8 * tg), u);
         if (bx)
 #pragma unroll
             for (int e = 0; e < 8; ++e) st_elem<T>(wbx, (row + e) * ro + co, u[e]);
@@ -431,13 +438,13 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
             const uint32_t off = (uint32_t)(int32_t)(T0 - G::OFF - tw + 8 * g + e) * ri + ci;
             u[e] = raw_float<T>(ld_raw<T>(wx, off)) * raw_float<T>(ld_raw<T>(wB, off));
         }
-        ring_store<NPA, NK, CB>(ru, cl, 8 * g, u);
+        ring_store<T, NK, CB>(ru, cl, 8 * g, u);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const uint32_t r = (uint32_t)(T0 - tw) + 8 * g + e;
             v[e] = raw_float<T>(ld_raw<T>(wdy, r * ro + co)) * raw_float<T>(ld_raw<T>(wC, r * ri + ci));
         }
-        ring_store<NPA, NK, CB>(rg, cl, 8 * g, v);
+        ring_store<T, NK, CB>(rg, cl, 8 * g, v);
     }
     uint32_t rx[8], rB[8], rl[8], rC[8], rd[8];                           // rl, rC: dy and C of the look-ahead; rd: dy of the tile
     uint32_t row = (uint32_t)(T0 - tw) + 8 * tg;
@@ -455,10 +462,10 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         float u[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) u[e] = raw_float<T>(rx[e]) * raw_float<T>(rB[e]);
-        ring_store<NPA, NK, CB>(ru, cl, wrap<G::R>(oldest + G::OFF + 8 * tg), u);
+        ring_store<T, NK, CB>(ru, cl, wrap<G::R>(oldest + G::OFF + 8 * tg), u);
 #pragma unroll
         for (int e = 0; e < 8; ++e) u[e] = raw_float<T>(rl[e]) * raw_float<T>(rC[e]);
-        ring_store<NPA, NK, CB>(rg, cl, wrap<G::R>(front + G::OFF + 8 * tg), u);
+        ring_store<T, NK, CB>(rg, cl, wrap<G::R>(front + G::OFF + 8 * tg), u);
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -522,12 +529,17 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         front = wrap<G::R>(front + TT);
     }
     // this run's filter gradient by lag: the channels of a filter added in their order
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (!(dh[c][r] * 0.f == 0.f)) *flag = 1;                      // (2^48 times the sum: past the range earlier)
     __syncthreads();
     if (*flag == 0) {
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) yt[(cw + c) * TT + (4 * q + r) * 16 + n] = dh[c][r];
+            for (int r = 0; r < 4; ++r) yt[(cw + c) * TT + (4 * q + r) * 16 + n] = dh[c][r] * (1.f / (LIFT<T> * LIFT<T>));
     } else {
         // the run again by taps, each row by the thread that stored it and lags tr, tr + 32, ... of its channel: u and g2
         // of a tile and their reach as fp32, rows of CB

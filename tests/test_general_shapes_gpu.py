@@ -173,3 +173,23 @@ def test_backward_in_several_launches(gcg_lib, bs, L, g, dg, hl, types):
         assert torch.equal(a, b)
     for o, r, n in zip(got, oracle_bwd(dy, x, B, C, h), ("dx", "dB", "dC", "dh")):
         assert_close(o, r, TOL_DH[dtype] if n == "dh" else BAR[dtype], n)
+
+
+@pytest.mark.parametrize("types", ["f32", "bf16w"])
+def test_products_near_the_smallest_normal_value(gcg_lib, types):
+    """Gated products around 2^-122 keep the bits that larger ones have, through all planes of the split."""
+    bs, L, g, dg, hl = 1, 1000, 8, 6, 64
+    dtype, filt = TYPES[types]
+    gen = torch.Generator().manual_seed(8)
+    x, B, C, dy = (torch.randn(bs, L, g, dg, generator=gen).to(dtype) for _ in range(4))
+    x, h = x * 2.0 ** -122, torch.randn(g, 1, hl, generator=gen)
+    _, y2, y = _lib.fwd(*(t.to(DEV) for t in (x, B, C, h)), return_y2=True)
+    dh = _lib.bwd(*(t.to(DEV) for t in (dy, x, B, C, h)))[3]
+    u, taps = (x.float() * B.float()).double(), h[:, 0].double().flip(-1)
+    ref = _taps_form(u, taps, 1)
+    g2 = (dy.float() * C.float()).double()
+    rdh = torch.stack([(g2[:, lag:] * u[:, :L - lag]).sum((0, 1, 3)) for lag in reversed(range(hl))], dim=1)
+    up = 2.0 ** 122
+    assert_close(y2.cpu().double() * up, ref * up, BAR[dtype], "y2")
+    assert_close(y.cpu().double() * up, C.double() * ref * up, BAR[dtype], "y")
+    assert_close(dh[:, 0].cpu().double() * up, rdh * up, TOL_DH[torch.float32], "dh")
