@@ -66,7 +66,7 @@ def test_algo_selection(gcg_lib):
     assert _lib.select_algo(1, 32768, 512, 16, 7, bf) == "window"         # Hyena-SE
     assert _lib.select_algo(1, 2048, 16, 16, 7, f32) == "window"          # fp32 SE config
     assert _lib.select_algo(2, 8192, 256, 16, 128, f32) == "mfma"         # fp32 MFMA keeps fp32 accuracy
-    assert _lib.select_algo(2, 8192, 256, 4, 128, f32) == "direct"        # narrow groups stay on the vector ALUs
+    assert _lib.select_algo(2, 8192, 256, 4, 128, f32) == "direct"        # narrow groups: the general family
     assert _lib.select_algo(1, 512, 4, 16, 300, bf) == "direct"           # filter longer than a chunk
     assert _lib.select_algo(1, 512, 64, 1, 64, bf) == "direct"            # one channel per filter
 

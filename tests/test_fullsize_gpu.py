@@ -74,7 +74,7 @@ def test_more_workgroups_than_fit_at_once(gcg_lib, bs, L):
     assert torch.equal(dfeat[..., 2], grads[0]) and torch.equal(dfeat[..., 1], grads[1]) and torch.equal(dfeat[..., 0], grads[2])
     assert_close(dh_i, grads[3], TOL_DH[dtype], "dh interleaved")
     direct = _lib.bwd(inp["dy"], inp["k"], inp["q"], inp["v"], inp["h"], algo="direct")
-    assert_close(grads[0], direct[0], TOL[dtype], "dx, matrix cores against vector ALUs")
+    assert_close(grads[0], direct[0], TOL[dtype], "dx, tile family against the general one")
 
 
 # ---- the benchmark configurations ------------------------------------------------------------------

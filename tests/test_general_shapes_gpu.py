@@ -26,7 +26,8 @@ SHAPES = [                    # bs, L, g, dg, hl
     (2, 513, 5, 7, 146),
     (1, 1111, 1, 40, 241),
     (1, 900, 17, 2, 256),
-    (1, 300, 40, 1, 256),     # the deepest product with one filter per channel (fp32 and f16: vector kernels)
+    (1, 300, 40, 1, 256),     # the deepest product with one filter per channel (backward in fp32 arithmetic on fp32 and f16
+                              # tensors: vector kernels)
 ]
 
 

@@ -31,7 +31,7 @@ SHAPES = [
     (1, 200, 17, 16, 64),
     (2, 5, 2, 16, 128),
     (3, 2500, 10, 16, 128),   # several runs per column
-    (1, 700, 2, 16, 200),     # direct kernels only
+    (1, 700, 2, 16, 200),     # general family only
 ]
 
 

@@ -93,6 +93,24 @@ def test_chains_of_the_featurizer_gradient(gcg_lib, L, g):
     assert err <= terms2 * (0.4 * 2.0 ** -24) ** 2 * (64 + 16) / 2
 
 
+@pytest.mark.parametrize("bs,L,g,dg,hl,lc,kf", [
+    (2, 4097, 16, 16, 128, 128, 3),
+    (1, 8190, 11, 48, 100, 128, 3),     # sums in second launches; a cut filter
+    (600, 40, 3, 32, 40, 64, 2),        # runs of two steps, the filter as long as the sequence
+    (1, 16384, 16, 16, 9, 128, 1),
+])
+def test_decayed_filter(gcg_lib, bs, L, g, dg, hl, lc, kf):
+    """The filter formed in the kernel, as the module has it: the bits of the explicit filter's, and dw those of its dh."""
+    assert one_kernel(bs, L, g, dg, hl, kf)
+    raw, wf, _, dy = (t.to(DEV) for t in make(bs, L, g, dg, hl, kf, BF, F32, seed=6))
+    w = torch.randn(g, lc, generator=torch.Generator().manual_seed(6)).to(DEV)
+    decay = torch.exp(-torch.logspace(0, 2, g)[:, None] * torch.linspace(0, 1, lc)[None]).to(DEV)
+    draw, dwf, dw = _lib.mixer_mr_bwd_decay(dy, raw, wf, w, decay, hl, F32)
+    want = _lib.mixer_mr_bwd(dy, raw, wf, _lib.filter_decay_fwd(w, decay, hl, F32))
+    assert torch.equal(draw, want[0]) and torch.equal(dwf, want[1])
+    assert torch.equal(dw, _lib.filter_decay_bwd(want[2], decay))
+
+
 def test_where_it_starts(gcg_lib):
     assert not one_kernel(1, 1023 * 32, 4, 16, 128, 3) and one_kernel(1, 1023 * 32 + 1, 4, 16, 128, 3)
     lib = _lib.load()

@@ -40,7 +40,7 @@ SMALL = [
     (1, 64, 6, 1, 5),        # one channel per filter
     (1, 70, 2, 24, 1),       # single tap
     (1, 400, 1, 64, 8),
-    (1, 700, 2, 16, 200),    # filter longer than a chunk (direct kernel only)
+    (1, 700, 2, 16, 200),    # filter longer than a chunk (general family only)
     (1, 200, 17, 16, 64),    # d = 272: a 256-channel workgroup plus a block with one live wave
     (1, 100, 9, 16, 128),    # d = 144: partial 128-channel block
     (2, 5, 2, 16, 128),      # sequence shorter than one step and than the filter
