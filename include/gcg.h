@@ -48,7 +48,9 @@ enum { GCG_F32 = 0, GCG_BF16 = 1, GCG_F16 = 2, GCG_BF16_F32 = 3, GCG_F16_F32 = 4
  * family and fail with GCG_ERR_UNSUPPORTED when the shape does not fit it. */
 enum {
     GCG_ALGO_AUTO   = 0,
-    GCG_ALGO_DIRECT = 1, /* LDS-tiled sliding window on the vector ALUs, any hl/dg/dtype */
+    GCG_ALGO_DIRECT = 1, /* the general family, any hl/dg/dtype and element alignment: filters of 9 to 256
+                            taps as products of time blocks on MFMA, all others (and the few sizes whose
+                            tables or scratch do not fit) as an LDS-tiled sliding window on the vector ALUs */
     GCG_ALGO_WINDOW = 2, /* register sliding window, hl <= 8 (Hyena-SE)                   */
     GCG_ALGO_MFMA   = 3  /* banded Toeplitz GEMM on MFMA, any dtype, hl <= 128, dg % 16 == 0 (Hyena-MR) */
 };
@@ -86,7 +88,7 @@ GCG_API int gcg_last_hip_error(void);
  * or matrix-core kernels has the runtime stamp the two events at the start and at the end of
  * its main kernel -- not of the small filter-gradient reduction that follows a backward -- so
  * that hipEventElapsedTime(start, stop) is that kernel's own duration, as a profiler reports
- * it.  The arming lasts for one call: every entry point that launches kernels clears it on
+ * it (from the first to the last where a batch is launched in parts).  The arming lasts for one call: every entry point that launches kernels clears it on
  * return, whatever it returns and whether its launcher used the events or not.  Two null
  * pointers disarm; one null pointer is GCG_ERR_BAD_ARG.  Not for a stream that is being
  * captured into a graph: a timed launch is not a plain kernel node.
@@ -118,6 +120,10 @@ GCG_API int gcg_route_supported(int32_t route, int64_t bs, int64_t L, int32_t g,
  * Replaces two_pass_fwd_grouped(x, B, C, h, return_bx=, return_y2=)
  * (savanna/kernels/triton_src/cgcg/src/fwd.py:13-233), which launches
  * _two_pass_fwd_refactor_kernel (src/fwd_kernels.py:585-750).
+ *
+ * Infinities and NaN: at 9 to 256 taps the general family keeps them to the rows their taps reach.  The other
+ * kernels also form products with zeros beyond the filter, within the block of taps or rows they work in, as the
+ * reference's chunked products do: rows near such a value may be NaN there.
  *
  *   y            out, required
  *   y2_or_null   out, optional: the convolution before the post-gate (fwd.py `return_y2`)
@@ -175,7 +181,8 @@ GCG_API int gcg_bwd(const void *dy, const void *x, const void *B, const void *C,
  * hand over.  The per-workgroup partial sums of dh go to a device array that is part of the
  * library image (GCG_BWD_STATIC_SCRATCH_BYTES per GPU, held from the first call on that GPU until
  * the process ends); the call itself allocates and frees nothing.  Same kernels, same order of
- * summation, hence the same bits as gcg_bwd.
+ * summation, hence the same bits as gcg_bwd.  (The general family launches a batch whose partial
+ * sums would not fit this array in parts, with a workspace too.)
  *
  * Sizes whose gcg_bwd_workspace_bytes(...) exceeds GCG_BWD_STATIC_SCRATCH_BYTES are rejected with
  * GCG_ERR_STATIC_SCRATCH (the Evo2-7B and 40B layer shapes need 0.5 MB on the matrix-core kernels and
@@ -364,7 +371,9 @@ GCG_API int gcg_mixer_se_bwd_planar(const void *dy, const void *raw, const void 
  * the features are made again from raw, their gradient is handed from the operator's part to the featurizer's
  * part inside the workgroup and never stored: 7 N s of memory traffic (dy and raw in, draw out) instead of the two-call
  * chain's 16 N s.  draw and dh are the chain's bit for bit (bf16), dwf up to the order in which partial sums are added.
- * GCG_BF16_F32 does the same from 1024 steps of 32 rows on (64-channel columns times batch rows times steps).
+ * GCG_BF16_F32 does the same from 1024 steps of 32 rows on (64-channel columns times batch rows times steps):
+ * draw is the chain's bit for bit; dh and dwf are the chain's terms summed in fp32 in another order and cut, dwf in
+ * pairs of rows (v_dot2_f32_bf16), in chains short enough that neither ends further from its 64-bit sum than the chain's.
  * Other types and smaller problems: one kernel recomputes the features and writes their gradient into dfeat_scratch
  * ((bs, L, g, dg, 3), caller's memory, contents on return unspecified), then the featurizer's own backward turns
  * it into draw and dwf -- the chain's traffic, but nothing of size 3 N is kept between forward and backward.

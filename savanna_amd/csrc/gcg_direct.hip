@@ -6,7 +6,8 @@
 // 31-sample window in registers so that a block costs 47 LDS reads for 256 FMAs.
 // This is the fallback for shapes the MFMA and register-window kernels do not take (filters
 // longer than 128 taps, narrow or odd group widths, misaligned tensors); of those, 9 to 256 taps go to the
-// matrix-core kernels of gcg_toep.hip, so what runs here are odd shapes of at most 8 taps and filters beyond 256.
+// matrix-core kernels of gcg_toep.hip, so what runs here are odd shapes of at most 8 taps, filters beyond 256, and the
+// few sizes in between whose tap tables, launch or scratch those kernels cannot hold.
 #include "gcg_common.h"
 
 namespace gcg {

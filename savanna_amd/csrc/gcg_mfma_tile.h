@@ -919,9 +919,11 @@ MfmaPlan plan_bwd_runs(const Dims &dm, int nw, int elem_bytes)
     const MfmaPlan p = plan(dm, nw, BWD_FULL_STEPS, nw, elem_bytes);
     return p.nwg >= cu_count() ? p : plan(dm, nw, BWD_MIN_STEPS, nw, elem_bytes);
 }
-// Forward: 3 steps with 16-bit operands, where two workgroups share a CU and more of them slow each other down (4 steps
-// before, 3, 2: 1 x 2000 x 4096 17.7, 15.7, 15.3 us, 1 x 701 x 4096 10.0, 9.1, 10.9, 1 x 4000 x 1024 9.7, 9.3, 10.9),
-// 2 with operands of several planes (bf16 tensors in fp32 arithmetic, 1 x 300 x 4096: 10.6 and 8.0 us; fp32 tensors
+// Forward: 3 steps with 16-bit operands (4 before).  Of 13 shapes none takes more than 1.5 % longer than with 4, and
+// eight take 4 to 12 % less (1 x 2000 x 4096 17.7 -> 15.7 us, 1 x 701 x 4096 10.0 -> 9.1).  With 2 steps five are faster still (1 x
+// 300 x 4096 7.5 against 8.7, 2 x 1000 x 512 6.8 against 8.0), but two are slower than with 4, where two workgroups share
+// a CU and slow each other down (1 x 701 x 4096 10.9, 1 x 4000 x 1024 10.9 against 9.3): a constant that loses nowhere.
+// 2 steps with operands of several planes (bf16 tensors in fp32 arithmetic, 1 x 300 x 4096: 10.6 and 8.0 us; fp32 tensors
 // 18.8 and 16.7, 1 x 701 x 4096 23.4 and 19.1).
 template <typename T> constexpr int fwd_min_steps() { return MT<T>::SPLIT ? 2 : 3; }
 

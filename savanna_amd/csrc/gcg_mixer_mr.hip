@@ -740,13 +740,13 @@ __global__ __launch_bounds__(MixGeo<T>::NT) void mixer_mr_bwd_kernel(const T *__
 // -- five steps ahead for C (8 of a piece's 12 bytes), one step ahead for x and B, and with its gradient for d wf --
 // and nearly all but the first are answered by the L2: a step's rows are 12 KB per workgroup, and those of six steps of
 // the 32 workgroups of an XCD are 2.4 MB of its 4 MB, which dy and the last reading therefore pass with the streaming
-// hint (907 MB read from beyond the L2 without it, 625 with it, 537 at least).  dy waits for its step in a lane-private ring in LDS.
+// hint (907 MB read from beyond the L2 without it, 625 with it, 537 at least; now 661, with the sums put aside).  dy waits for its step in a lane-private ring in LDS.
 // A run goes one step beyond its end for the gradient rows that its last two rows of d raw need, and two iterations
 // further for the hand-overs; what these compute beyond the run is dropped by the windows or not accumulated.
 //
 // What bounds it: instruction issue (87 matrix instructions per 16 channels and step, and the vector work of both
-// kernels it replaces: 59 % of the quad-cycles issue, and a matrix instruction takes four).  7B shape (2 x 8192 x 4096),
-// bf16: 319 - 343 us, against 233 - 264 us for the operator's backward with the features made in front (gradient of the
+// kernels it replaces: 57 % of the quad-cycles issue, and a matrix instruction takes four).  7B shape (2 x 8192 x 4096),
+// bf16: 311 - 343 us, against 233 - 264 us for the operator's backward with the features made in front (gradient of the
 // features to memory) and 217 - 222 + 9 us for the featurizer's backward on it; 7 instead of 16 values moved per
 // element.  Measured and left: d wf on the product waves (351 us), d wf with fused
 // multiply-adds on unpacked values (351), straight-line bodies for the first, middle and last steps (spills, 590).
@@ -1185,7 +1185,6 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
             raw_b += step_b3;
             dy_b += step_b;
         };
-        // (each kind of iteration is a straight-line body of its own, so that its LDS reads can be requested early)
         while (s < n_it) {
 #pragma unroll
             for (int pu = 0; pu < RSLOTS; ++pu)
@@ -1526,9 +1525,9 @@ bool mixer_mr_fused_supported(int dtype, const Dims &dm, int kf)
 
 // The backward alone: also bf16 tensors in fp32 arithmetic (interleaved features; f16's operands take three planes,
 // whose rings do not fit the registers of the product waves).  From 1024 steps of 32 rows on, all columns together:
-// smaller problems keep the two kernels and with them the order of the sums of d wf (its bits are the two-call chain's);
-// what that costs there is mostly the second launch (one kernel against two, from graph replays: 64 steps 28.8 / 29.0 us,
-// 256 steps 30 / 35, 560 steps 34 / 42, 1024 steps 39 / 52, 4096 steps 64 / 91).
+// smaller problems keep the two kernels and with them the bits of d wf, which callers of the two-call chain have there.
+// One kernel would be faster from 64 steps on (one against two, from graph replays: 64 steps 28.8 / 29.0 us, 256 steps
+// 30 / 35, 560 steps 34 / 42, 1024 steps 39 / 52, 4096 steps 64 / 91): the line is not where the times cross.
 bool mixer_mr_fused_bwd_supported(int dtype, const Dims &dm, int kf)
 {
     if (dtype != GCG_BF16_F32) return mixer_mr_fused_supported(dtype, dm, kf);

@@ -30,9 +30,12 @@
 //
 // A workgroup owns CB adjacent channels and a run of 256-row tiles of one batch row; u (and g2) of a tile and of the
 // filter's reach stay in LDS as rings, so each row is read once (dy twice in the backward: for g2 OFF rows ahead, and
-// for dC).  What bounds it: the LDS reads of the operands and the transposition between the tensors' channel-fastest
-// rows and the channel-major rings, then memory.  Measured at 1 x 4096 x (256 groups of 8), 128 taps, bf16, against
-// gcg_direct.hip: forward 124 -> 21 us, backward 333 -> 57 us, its filter-gradient sum 27 -> 4 us.
+// for dC).  Measured at 1 x 4096 x (256 groups of 8), 128 taps, bf16, against gcg_direct.hip: forward 124 -> 22 us,
+// backward 333 -> 63 us, its filter-gradient sum 27 -> 4 us.  What bounds it (SQ counters there): vector instructions --
+// the split into planes, its transposition between the tensors' channel-fastest rows and the channel-major rings, one
+// access per element -- take 44 % of the SIMDs' issue cycles forward and 56 % backward, matrix instructions occupy 13 and
+// 22 %, and waves spend half of their time waiting, for rows and at the two or four barriers of a tile.  Memory is far off:
+// 71 MB in 22 us forward, 146 MB in 63 us backward.
 #include "gcg_mfma_tile.h"
 
 #include <type_traits>
@@ -665,8 +668,8 @@ bool make_plan(int dtype, const Dims &dm, int dirs, size_t vector_bytes, Plan &p
     p.b0 = 0;
     // A backward whose partial sums the static scratch held with the vector kernels' blocks of 64 channels and does not
     // with these of 16 or 32 is launched for a part of the batch rows at a time, each launch adding to the sums of the
-    // one before, here and with a workspace alike (21 x 160 x (256 groups of 32), 256 taps, bf16: 10.5 MB and 537 us in
-    // one launch, 5.5 MB in two and 1 % more time).
+    // one before, here and with a workspace alike (21 x 160 x (256 groups of 32), 256 taps, bf16: 10.5 MB and 587 us in
+    // one launch, 5.5 MB and 594 us in two).
     const size_t row_bytes = (size_t)p.nct * p.nseg * p.nf * dm.hl * sizeof(float);
     if (dirs == 2 && vector_bytes <= GCG_BWD_STATIC_SCRATCH_BYTES && dm.bs * row_bytes > GCG_BWD_STATIC_SCRATCH_BYTES) {
         const int64_t rows = (int64_t)(GCG_BWD_STATIC_SCRATCH_BYTES / row_bytes);
