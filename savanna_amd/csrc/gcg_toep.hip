@@ -22,8 +22,8 @@
 // ALUs, and half of a tile's products enter negated, so that the bias of one half is taken off by the other's: 1.4e-7,
 // and below the vector kernels' error at every shape compared, for 4 % of the backward's time.
 //
-// Infinities, NaN and samples from 2^104 on (LIFT): the products multiply samples with the zeros around the band, and a
-// plane of such a value is infinite or NaN.  Whatever the sample, some y2 or du of the run is then not finite;
+// Infinities, NaN, samples and taps from 2^104 on, results from 2^80 on (LIFT): the products multiply samples with the zeros
+// around the band, and a plane of such a value is infinite or NaN.  Whatever the sample, some y2 or du of the run is then not finite;
 // a workgroup that met one does its run once more on the vector ALUs, tap by tap in fp32 and with the sums of the filter
 // gradient cut the same way: a sample then reaches the rows its taps reach and no other.  Looking at the results costs
 // 1 % of the kernels' time, at the samples (their largest magnitude) 4 %.
@@ -53,9 +53,10 @@ template <> struct GT<f16_t> { static constexpr int NPA = 3, NPW = 2; };
 template <> struct GT<bf16w_t> { static constexpr int NPA = 2, NPW = 3; };
 template <> struct GT<f16w_t> { static constexpr int NPA = 3, NPW = 3; };
 
-// Samples enter the rings times 2^24 and taps the tables times 2^-24: the last planes of a sample below 2^-110 would be
-// bf16 subnormals, and bits of it lost (f16's smallest product is 2^-48: no need)
+// Samples enter the rings and taps the tables times 2^24, and results are divided by both: the last planes of a value below
+// 2^-110 would be bf16 subnormals, and bits of it lost (f16's smallest tap is 2^-24 and its smallest product 2^-48: no need)
 template <typename T> constexpr float LIFT = std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t> ? 1.f : 0x1p24f;
+template <typename T> constexpr float DROP = 1.f / (LIFT<T> * LIFT<typename Filt<T>::type>);       // of y2 and du
 
 template <int NK> struct Reach {
     static constexpr int OFF = 32 * NK - 16;     // rows of history (u) and look-ahead (g2) held beside a tile
@@ -198,7 +199,7 @@ __device__ __forceinline__ void fill_taps(uint16_t *tab, const typename Filt<T>:
         float v = 0.f;
         if (lag >= 0 && lag < hl) v = Elem<FT>::load(h + (f0 + f) * hl + (hl - 1 - lag));
         uint16_t o[NPW];
-        split_planes<NPW>(v * (1.f / LIFT<T>), o);
+        split_planes<NPW>(v * LIFT<FT>, o);
 #pragma unroll
         for (int m = 0; m < NPW; ++m) tab[(m * nf + f) * G::HP + z + 16] = o[m];
     }
@@ -347,8 +348,8 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
         }
         f32x4 acc[2];
         band_product<T, NK, CB>(acc, ring, tab, nf, fa, fb, cw, oldest, lane);
-        *(f32x4 *)(yt + cw * YP + 16 * (lane & 15) + 4 * (lane >> 4)) = acc[0];
-        *(f32x4 *)(yt + (cw + 1) * YP + 16 * (lane & 15) + 4 * (lane >> 4)) = acc[1];
+        *(f32x4 *)(yt + cw * YP + 16 * (lane & 15) + 4 * (lane >> 4)) = acc[0] * DROP<T>;
+        *(f32x4 *)(yt + (cw + 1) * YP + 16 * (lane & 15) + 4 * (lane >> 4)) = acc[1] * DROP<T>;
         __syncthreads();
         float v[8];
         *(f32x4 *)v = *(const f32x4 *)(yt + cl * YP + 8 * tg);
@@ -480,8 +481,8 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         float v[8];
         float *const yw = yt + cw * YP + 16 * n + 4 * q, *const yr = yt + cl * YP + 8 * tg;
         band_product<T, NK, CB>(acc, ru, ta, nf, fa, fb, cw, oldest, lane);
-        *(f32x4 *)yw = acc[0];
-        *(f32x4 *)(yw + YP) = acc[1];
+        *(f32x4 *)yw = acc[0] * DROP<T>;
+        *(f32x4 *)(yw + YP) = acc[1] * DROP<T>;
         __syncthreads();
         *(f32x4 *)v = *(const f32x4 *)yr;
         *(f32x4 *)(v + 4) = *(const f32x4 *)(yr + 4);
@@ -514,8 +515,8 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         dh[1] += dt[1];
         band_product<T, NK, CB>(acc, rg, tb, nf, fa, fb, cw, front, lane);
         __syncthreads();
-        *(f32x4 *)yw = acc[0];
-        *(f32x4 *)(yw + YP) = acc[1];
+        *(f32x4 *)yw = acc[0] * DROP<T>;
+        *(f32x4 *)(yw + YP) = acc[1] * DROP<T>;
         __syncthreads();
         *(f32x4 *)v = *(const f32x4 *)yr;
         *(f32x4 *)(v + 4) = *(const f32x4 *)(yr + 4);

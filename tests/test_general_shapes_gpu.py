@@ -176,21 +176,45 @@ def test_backward_in_several_launches(gcg_lib, bs, L, g, dg, hl, types):
         assert_close(o, r, TOL_DH[dtype] if n == "dh" else BAR[dtype], n)
 
 
-@pytest.mark.parametrize("types", ["f32", "bf16w"])
-def test_products_near_the_smallest_normal_value(gcg_lib, types):
-    """Gated products around 2^-122 keep the bits that larger ones have, through all planes of the split."""
+@pytest.mark.parametrize("types,which", [("f32", "x"), ("bf16w", "x"), ("f32", "h"), ("bf16w", "h")])
+def test_values_near_the_smallest_normal_one(gcg_lib, types, which):
+    """Gated products or taps around 2^-122 keep the bits that larger ones have, through all planes of the split."""
     bs, L, g, dg, hl = 1, 1000, 8, 6, 64
     dtype, filt = TYPES[types]
     gen = torch.Generator().manual_seed(8)
     x, B, C, dy = (torch.randn(bs, L, g, dg, generator=gen).to(dtype) for _ in range(4))
-    x, h = x * 2.0 ** -122, torch.randn(g, 1, hl, generator=gen)
+    h, up = torch.randn(g, 1, hl, generator=gen), 2.0 ** 122
+    if which == "x":
+        x = x / up
+    else:
+        h = h / up
     _, y2, y = _lib.fwd(*(t.to(DEV) for t in (x, B, C, h)), return_y2=True)
-    dh = _lib.bwd(*(t.to(DEV) for t in (dy, x, B, C, h)))[3]
+    dx, _, _, dh = _lib.bwd(*(t.to(DEV) for t in (dy, x, B, C, h)))
     u, taps = (x.float() * B.float()).double(), h[:, 0].double().flip(-1)
-    ref = _taps_form(u, taps, 1)
     g2 = (dy.float() * C.float()).double()
-    rdh = torch.stack([(g2[:, lag:] * u[:, :L - lag]).sum((0, 1, 3)) for lag in reversed(range(hl))], dim=1)
-    up = 2.0 ** 122
+    ref, rdx = _taps_form(u, taps, 1), B.double() * _taps_form(g2, taps, -1)
     assert_close(y2.cpu().double() * up, ref * up, BAR[dtype], "y2")
     assert_close(y.cpu().double() * up, C.double() * ref * up, BAR[dtype], "y")
-    assert_close(dh[:, 0].cpu().double() * up, rdh * up, TOL_DH[torch.float32], "dh")
+    if which == "h":
+        assert_close(dx.cpu().double() * up, rdx * up, BAR[dtype], "dx")
+    else:
+        rdh = torch.stack([(g2[:, lag:] * u[:, :L - lag]).sum((0, 1, 3)) for lag in reversed(range(hl))], dim=1)
+        assert_close(dh[:, 0].cpu().double() * up, rdh * up, TOL_DH[torch.float32], "dh")
+
+
+@pytest.mark.parametrize("types", ["f32", "bf16w"])
+def test_large_results_of_moderate_values(gcg_lib, types):
+    """y2 and du of 2^85 and a filter gradient of 2^90 are beyond what the scaled products hold and within fp32."""
+    bs, L, g, dg, hl = 1, 600, 3, 6, 40
+    dtype, filt = TYPES[types]
+    gen = torch.Generator().manual_seed(9)
+    x, B, C, dy = (torch.randn(bs, L, g, dg, generator=gen).to(dtype) for _ in range(4))
+    h = torch.randn(g, 1, hl, generator=gen) * 2.0 ** 45
+    x, dy = x * 2.0 ** 40, dy * 2.0 ** 40
+    _, y2, _ = _lib.fwd(*(t.to(DEV) for t in (x, B, C, h)), return_y2=True)
+    dx, _, _, dh = _lib.bwd(*(t.to(DEV) for t in (dy, x, B, C, h)))
+    u, g2, taps = (x.float() * B.float()).double(), (dy.float() * C.float()).double(), h[:, 0].double().flip(-1)
+    assert_close(y2, _taps_form(u, taps, 1), BAR[dtype], "y2")
+    assert_close(dx, B.double() * _taps_form(g2, taps, -1), BAR[dtype], "dx")
+    rdh = torch.stack([(g2[:, lag:] * u[:, :L - lag]).sum((0, 1, 3)) for lag in reversed(range(hl))], dim=1)
+    assert_close(dh[:, 0], rdh, TOL_DH[torch.float32], "dh")
