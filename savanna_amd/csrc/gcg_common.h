@@ -208,7 +208,8 @@ template <bool KEEP> __device__ __forceinline__ void win_store_as(win_t w, uint3
 __device__ __forceinline__ int64_t xcd_contiguous_id(int64_t id, int64_t n)
 {
 #if GCG_XCD_SWIZZLE
-    if ((n & 7) == 0) return (id & 7) * (n >> 3) + (id >> 3);
+    const int64_t x = id & 7, q = n >> 3, r = n & 7;      // the first n % 8 XCDs have one workgroup more
+    return x * q + (x < r ? x : r) + (id >> 3);
 #endif
     return id;
 }
@@ -216,7 +217,8 @@ __device__ __forceinline__ int64_t xcd_contiguous_id(int64_t id, int64_t n)
 __device__ __forceinline__ uint32_t xcd_contiguous_u32(uint32_t id, uint32_t n)
 {
 #if GCG_XCD_SWIZZLE
-    if ((n & 7u) == 0) return (id & 7u) * (n >> 3) + (id >> 3);
+    const uint32_t x = id & 7u, q = n >> 3, r = n & 7u;
+    return x * q + (x < r ? x : r) + (id >> 3);
 #endif
     return id;
 }

@@ -59,14 +59,8 @@ __device__ unsigned long long g_trace[(size_t)TRACE_WGS * TRACE_SLOTS];
 #ifndef GCG_MFMA_BWD_ST
 #define GCG_MFMA_BWD_ST WIN_NT_ST
 #endif
-#ifndef GCG_MFMA_BWD_ST_DC
-#define GCG_MFMA_BWD_ST_DC GCG_MFMA_BWD_ST
-#endif
 #ifndef GCG_MFMA_FWD_LD
 #define GCG_MFMA_FWD_LD WIN_NT
-#endif
-#ifndef GCG_MFMA_FWD_LEAD_LD
-#define GCG_MFMA_FWD_LEAD_LD WIN_NT
 #endif
 // Idle cycles in front of each output store of the backward's long runs (tuning builds may override).  Measured
 // at the 7B layer shape (2 x 8192 x 4096, bf16): 0 cycles 172.3 - 173.8 us, 16: 171.0, 24: 169.5, 32: 167.3 - 170.4,
@@ -79,6 +73,19 @@ __device__ unsigned long long g_trace[(size_t)TRACE_WGS * TRACE_SLOTS];
 #ifndef GCG_MFMA_BWD_LD
 #define GCG_MFMA_BWD_LD WIN_NT
 #endif
+// Cache policies by element type and by how rows lie on the 128-byte lines.
+// fp32: a lane's 8 channels are two 16-byte accesses 32 bytes apart, so every line is asked for twice; with the
+// nontemporal hint on the loads the second request went to memory again (1 x 12000 x 4096: forward 163 -> 146 us, backward
+// 348 -> 320 us with plain loads; 2 x 4096 x 2048, 64 taps: 61 -> 57 and 124 -> 113 us).
+// RAG (backward, 16 bits): rows that do not start and end on lines.  A workgroup's 128-byte pieces of a row then share their
+// first and last line with its neighbours', and with the hint each half is read, and written to memory, by itself: 1 x 12000 x
+// 4048 257 us, against 149 with plain accesses, where the halves meet in the XCD's L2 (4096 channels: 131 either way; nontemporal
+// loads and plain stores 179, sc1 stores 160 - 190).
+template <typename T, bool RAG> struct Policy {
+    static constexpr bool WIDE = sizeof(T) == 4;
+    static constexpr int FWD_LD = WIDE ? 0 : GCG_MFMA_FWD_LD, FWD_ST = WIDE ? WIN_NT_ST : GCG_MFMA_FWD_ST;
+    static constexpr int BWD_LD = WIDE || RAG ? 0 : GCG_MFMA_BWD_LD, BWD_ST = RAG ? 0 : GCG_MFMA_BWD_ST;
+};
 
 // ---------------------------------------------------------------------------- forward
 // EXTRA: also write the convolution before the post-gate (y2o) and the pre-gate product (bxo).
@@ -157,16 +164,16 @@ __global__ __launch_bounds__(64 * NW) void mfma_fwd_kernel(const T *__restrict__
 #pragma unroll
         for (int i = 1; i < NK; ++i) {
             const uint32_t o = lane_in + IM * step_off(s_lo - i);
-            lx[i - 1] = ldw_row_policy<T, GCG_MFMA_FWD_LEAD_LD>(wx, o);
-            lB[i - 1] = ldw_row_policy<T, GCG_MFMA_FWD_LEAD_LD>(wB, o);
+            lx[i - 1] = ldw_row_policy<T, Policy<T, false>::FWD_LD>(wx, o);
+            lB[i - 1] = ldw_row_policy<T, Policy<T, false>::FWD_LD>(wB, o);
         }
     }
     Row<T> xr, Br, Cr;
     auto fetch = [&](int64_t s, Row<T> &xo, Row<T> &Bo, Row<T> &Co) {
         const uint32_t o = lane_in + IM * step_off(s);
-        xo = ldw_row_policy<T, GCG_MFMA_FWD_LD>(wx, o);
-        Bo = ldw_row_policy<T, GCG_MFMA_FWD_LD>(wB, o);
-        Co = ldw_row_policy<T, GCG_MFMA_FWD_LD>(wC, o);
+        xo = ldw_row_policy<T, Policy<T, false>::FWD_LD>(wx, o);
+        Bo = ldw_row_policy<T, Policy<T, false>::FWD_LD>(wB, o);
+        Co = ldw_row_policy<T, Policy<T, false>::FWD_LD>(wC, o);
     };
     fetch(s_lo, xr, Br, Cr);
     TR(1);
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(64 * NW) void mfma_fwd_kernel(const T *__restrict__
                     unpack8<T>(Cr, Cf);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) yf[e] = Cf[e] * y2f[e];
-                    stw_row_policy<T, (ES == 2 ? GCG_MFMA_FWD_ST : WIN_NT_ST)>(wy, o, pack8<T>(yf));
+                    stw_row_policy<T, Policy<T, false>::FWD_ST>(wy, o, pack8<T>(yf));
                     if constexpr (EXTRA) stw_row<T>(wy2, o, pack8<T>(y2f));
                 }
                 xr = xn; Br = Bn; Cr = Cn;
@@ -272,8 +279,8 @@ __global__ __launch_bounds__(64 * NW) void mfma_fwd_kernel(const T *__restrict__
 // end the diagonals of the P tiles are summed in a fixed order into per-wave partials in
 // the workspace, and a second kernel adds the partials in a fixed order.
 // PL: x, B, C and dx, dB, dC are thirds of the rows of (bs, L, 3 d) tensors (Dims::planar).
-// GAP: idle cycles in front of the output stores (GCG_MFMA_BWD_ST_GAP), for long runs.
-template <typename T, int NK, int NW, bool PL = false, bool GAP = false>
+// GAP: idle cycles in front of the output stores (GCG_MFMA_BWD_ST_GAP), for long runs.  RAG: Policy.
+template <typename T, int NK, int NW, bool PL = false, bool GAP = false, bool RAG = false>
 __global__ __launch_bounds__(64 * NW) void mfma_bwd_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                        const T *__restrict__ B, const T *__restrict__ C,
                                                        const T *__restrict__ h, T *__restrict__ dx,
@@ -366,10 +373,10 @@ __global__ __launch_bounds__(64 * NW) void mfma_bwd_kernel(const T *__restrict__
     // rows of iteration sg: x, B of step sg and dy, C of step sg+NK-1 (zero outside the windows)
     auto fetch = [&](int64_t sg, Row<T> &xo, Row<T> &Bo, Row<T> &dyo, Row<T> &Co) {
         const uint32_t o = lane_in + IM * step_off(sg), o2 = lane_off + step_off(sg + NK - 1);
-        xo = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wx, o);
-        Bo = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wB, o);
-        dyo = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wdy, o2);
-        Co = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wC, PL ? lane_in + IM * step_off(sg + NK - 1) : o2);
+        xo = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wx, o);
+        Bo = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wB, o);
+        dyo = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wdy, o2);
+        Co = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wC, PL ? lane_in + IM * step_off(sg + NK - 1) : o2);
     };
 
     // Lead-in: u of the NK-1 steps before the segment and g2 of its first NK-1 steps, i.e. the
@@ -489,7 +496,7 @@ __global__ __launch_bounds__(64 * NW) void mfma_bwd_kernel(const T *__restrict__
 #pragma unroll
                         for (int e = 0; e < 8; ++e) of[e] = dyf[e] * y2f[e];
                         if constexpr (GAP) idle_cycles<GCG_MFMA_BWD_ST_GAP>();
-                        stw_row_policy<T, GCG_MFMA_BWD_ST_DC>(wdC, o, pack8<T>(of));
+                        stw_row_policy<T, Policy<T, RAG>::BWD_ST>(wdC, o, pack8<T>(of));
                     }
                     {
                         const f32x4 p0 = *(const f32x4 *)d_rd;
@@ -499,11 +506,11 @@ __global__ __launch_bounds__(64 * NW) void mfma_bwd_kernel(const T *__restrict__
 #pragma unroll
                         for (int e = 0; e < 8; ++e) of[e] = duf[e] * Bf[e];
                         if constexpr (GAP) idle_cycles<GCG_MFMA_BWD_ST_GAP>();
-                        stw_row_policy<T, GCG_MFMA_BWD_ST>(wdx, o, pack8<T>(of));
+                        stw_row_policy<T, Policy<T, RAG>::BWD_ST>(wdx, o, pack8<T>(of));
 #pragma unroll
                         for (int e = 0; e < 8; ++e) of[e] = duf[e] * xf[e];
                         if constexpr (GAP) idle_cycles<GCG_MFMA_BWD_ST_GAP>();
-                        stw_row_policy<T, GCG_MFMA_BWD_ST>(wdB, o, pack8<T>(of));
+                        stw_row_policy<T, Policy<T, RAG>::BWD_ST>(wdB, o, pack8<T>(of));
                     }
                 }
                 xr = xn; Br = Bn; dyr = dyn; Cr = Cn;
@@ -538,7 +545,7 @@ template <typename T> constexpr bool duo_type() { return std::is_same<T, bf16w_t
 // a ring of NK+1 steps of g2, which both kinds of waves read) and accumulate the filter-gradient tiles of step sigma
 // from the ring.
 // Five-slice filters only (the rings' periods fix the unrolling: 2 NK for the product waves, NK+1 for the row waves).
-template <typename T, bool PL = false>
+template <typename T, bool PL = false, bool RAG = false>
 __global__ __launch_bounds__(512) void mfma_bwd_duo_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                        const T *__restrict__ B, const T *__restrict__ C,
                                                        const T *__restrict__ h, T *__restrict__ dx,
@@ -606,10 +613,10 @@ __global__ __launch_bounds__(512) void mfma_bwd_duo_kernel(const T *__restrict__
         // rows of iteration sg: x, B of step sg and dy, C of step sg+NK-1 (zero outside the windows)
         auto fetch = [&](int64_t sg, Row<T> &xo, Row<T> &Bo, Row<T> &dyo, Row<T> &Co) {
             const uint32_t o = lane_in + IM * step_off(sg), o2 = lane_off + step_off(sg + NK - 1);
-            xo = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wx, o);
-            Bo = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wB, o);
-            dyo = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wdy, o2);
-            Co = ldw_row_policy<T, GCG_MFMA_BWD_LD>(wC, PL ? lane_in + IM * step_off(sg + NK - 1) : o2);
+            xo = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wx, o);
+            Bo = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wB, o);
+            dyo = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wdy, o2);
+            Co = ldw_row_policy<T, Policy<T, RAG>::BWD_LD>(wC, PL ? lane_in + IM * step_off(sg + NK - 1) : o2);
         };
         // u = x * B into a u tile; g2 = dy * C into a slot of the ring
         auto gate_rows = [&](const Row<T> &xo, const Row<T> &Bo, const Row<T> &dyo, const Row<T> &Co, unsigned char *u_t,
@@ -638,7 +645,7 @@ __global__ __launch_bounds__(512) void mfma_bwd_duo_kernel(const T *__restrict__
                 unpack8<T>(dyo, dyf);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) of[e] = dyf[e] * y2f[e];
-                stw_row_policy<T, GCG_MFMA_BWD_ST_DC>(wdC, o, pack8<T>(of));
+                stw_row_policy<T, Policy<T, RAG>::BWD_ST>(wdC, o, pack8<T>(of));
             }
             {
                 const f32x4 p0 = *(const f32x4 *)(d_t + yd_rd);
@@ -649,10 +656,10 @@ __global__ __launch_bounds__(512) void mfma_bwd_duo_kernel(const T *__restrict__
                 unpack8<T>(Bo, Bf);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) of[e] = duf[e] * Bf[e];
-                stw_row_policy<T, GCG_MFMA_BWD_ST>(wdx, o, pack8<T>(of));
+                stw_row_policy<T, Policy<T, RAG>::BWD_ST>(wdx, o, pack8<T>(of));
 #pragma unroll
                 for (int e = 0; e < 8; ++e) of[e] = duf[e] * xf[e];
-                stw_row_policy<T, GCG_MFMA_BWD_ST>(wdB, o, pack8<T>(of));
+                stw_row_policy<T, Policy<T, RAG>::BWD_ST>(wdB, o, pack8<T>(of));
             }
         };
 
@@ -746,7 +753,9 @@ int fwd_launch(const void *x, const void *B, const void *C, const void *h, void 
     // with fewer, dealing the blocks round-robin measured 3-5 % faster in the forward (d = 2048, 4096) and the same
     // from d = 8192 on.  (The backward is 3 % faster XCD-contiguous at every width.)
     static const int order = env_int("GCG_MFMA_FWD_ORDER", -1);   // tuning override: 0 round-robin, 1 XCD-contiguous
-    p.xcd = order >= 0 ? (order != 0) : (p.ncb >= 32);
+    // Rows that do not end on a 128-byte line: neighbouring blocks share a line of every row, which one XCD's L2 reads and
+    // writes once (1 x 12000 x 4048: 83 -> 75 us, x 976: 30 -> 26).
+    p.xcd = order >= 0 ? (order != 0) : (p.ncb >= 32 || (dm.d * sizeof(T)) % 128 != 0);
     if constexpr (NK == 5) {
         // planar operands: instantiated for the five-slice walk only (fwd_t sends every filter length there)
         if (dm.planar)
@@ -838,17 +847,24 @@ int bwd_launch(const void *dy, const void *x, const void *B, const void *C, cons
         return launch_main(kernel, dim3((unsigned)p.nwg), dim3(threads), st, (const T *)dy, (const T *)x, (const T *)B,
                            (const T *)C, (const T *)h, (T *)dx, (T *)dB, (T *)dC, (T *)dh, (float *)ws, dm, p);
     };
+    // Rows or outputs off the 128-byte lines take plain accesses (Policy).  In fp32 arithmetic pieces that still start on half a
+    // line keep the hint: 1 x 12000 x 5536 245 us against 251, 4064 channels 168 against 163.
+    constexpr bool R = sizeof(T) == 2;
+    const bool rag = R && ((dm.d * sizeof(T)) | (uintptr_t)dx | (uintptr_t)dB | (uintptr_t)dC) % (MT<T>::SPLIT ? 64 : 128) != 0;
     if constexpr (NK == 5 && duo_type<T>()) {
         // product waves and row waves in one workgroup: the types whose backward is bound by instruction issue
-        e = dm.planar ? launch(mfma_bwd_duo_kernel<T, true>, 512) : launch(mfma_bwd_duo_kernel<T, false>, 512);
+        if (rag) e = dm.planar ? launch(mfma_bwd_duo_kernel<T, true, true>, 512) : launch(mfma_bwd_duo_kernel<T, false, true>, 512);
+        else e = dm.planar ? launch(mfma_bwd_duo_kernel<T, true>, 512) : launch(mfma_bwd_duo_kernel<T, false>, 512);
     } else if constexpr (NK == 5) {
         // planar operands: instantiated for the five-slice walk only (bwd_t sends every filter length there);
         // plain 16-bit tensors in runs of 32 steps and more: with the idle cycles in front of the stores
-        if (dm.planar) e = launch(mfma_bwd_kernel<T, NK, NW, true>, 64 * NW);
+        if (rag && dm.planar) e = launch(mfma_bwd_kernel<T, NK, NW, true, false, R>, 64 * NW);
+        else if (rag) e = launch(mfma_bwd_kernel<T, NK, NW, false, false, R>, 64 * NW);
+        else if (dm.planar) e = launch(mfma_bwd_kernel<T, NK, NW, true>, 64 * NW);
         else if (!MT<T>::SPLIT && p.steps_per_seg >= 32) e = launch(mfma_bwd_kernel<T, NK, NW, false, !MT<T>::SPLIT>, 64 * NW);
         else e = launch(mfma_bwd_kernel<T, NK, NW>, 64 * NW);
     } else {
-        e = launch(mfma_bwd_kernel<T, NK, NW>, 64 * NW);
+        e = rag ? launch(mfma_bwd_kernel<T, NK, NW, false, false, R>, 64 * NW) : launch(mfma_bwd_kernel<T, NK, NW>, 64 * NW);
     }
     if (e || p.fuse_dh) return e;
     const int64_t n = (int64_t)dm.g * (dm.fw ? dm.lc : dm.hl);
