@@ -182,6 +182,21 @@ template <int AUX> __device__ __forceinline__ u32x4 win_load_policy(win_t w, uin
 {
     return __builtin_amdgcn_raw_buffer_load_b128(w, (int)off, 0, AUX);
 }
+// any vector of 4 to 16 bytes with the cache-policy bits given
+template <int AUX, typename R> __device__ __forceinline__ R win_load_aux(win_t w, uint32_t off)
+{
+    R r;
+    if constexpr (sizeof(R) == 4) { const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(w, (int)off, 0, AUX); __builtin_memcpy(&r, &v, 4); }
+    else if constexpr (sizeof(R) == 8) r = __builtin_amdgcn_raw_buffer_load_b64(w, (int)off, 0, AUX);
+    else r = __builtin_amdgcn_raw_buffer_load_b128(w, (int)off, 0, AUX);
+    return r;
+}
+template <int AUX, typename R> __device__ __forceinline__ void win_store_aux(win_t w, uint32_t off, const R &v)
+{
+    if constexpr (sizeof(R) == 4) { uint32_t u; __builtin_memcpy(&u, &v, 4); __builtin_amdgcn_raw_buffer_store_b32(u, w, (int)off, 0, AUX); }
+    else if constexpr (sizeof(R) == 8) __builtin_amdgcn_raw_buffer_store_b64(v, w, (int)off, 0, AUX);
+    else __builtin_amdgcn_raw_buffer_store_b128(v, w, (int)off, 0, AUX);
+}
 // The same without the nontemporal hint, for an output the next kernel of a chain reads back at once
 // (the featurized tensor, the gradient of the features): stored through the cache it is still
 // partly there when that kernel starts.  A kernel timed alone loses a few percent this way, which

@@ -837,20 +837,18 @@ MixPlan plan(const Dims &dm, int ch, bool backward)
     MixPlan p;
     p.ch = ch;
     p.nvec = (int)(dm.d / ch);
-    // The longest runs that still leave two workgroups per CU: the halo of up to 10 rows each side
-    // and the filter-gradient partials cost 9 % of the traffic at 128 rows, 4 % at 512.  The
-    // backward, which holds two workgroups per CU at a time, gains nothing beyond 512 rows; the
-    // forward does (measured at the 40B shape: 409 us at 512 rows, 383 at 1024).  Multiples of 16
-    // (the backward's longest ring) down to 16.
-    p.ts = backward ? 512 : 1024;
-    while (p.ts > 16 && dm.bs * ((dm.L + p.ts - 1) / p.ts) * p.nvec < 128 * 1024) p.ts >>= 1;
+    // Long runs keep the halo of up to 10 rows each side and the filter-gradient partials small (9 % of the traffic at 128
+    // rows, 4 % at 512).  The backward gains nothing beyond 512 rows; the forward does (40B shape: 409 us at 512 rows, 383 at
+    // 1024).  Multiples of 16 (the backward's longest ring).
+    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, 16, backward ? 512 : 1024, 9, 1.1, INT64_MAX);
+    p.ts = r.ts;
     static const char *env = tuning_env("GCG_MIXER_ROWS");      // tuning override: rows per lane, a multiple of 16
     if (env && atoi(env) >= 16 && atoi(env) % 16 == 0) p.ts = atoi(env);
-    while (p.ts > 16 && (int64_t)(p.ts + 32) * 3 * dm.d * 4 > WIN_MAX_BYTES) p.ts >>= 1;
+    while (p.ts > 16 && (int64_t)(p.ts + 32) * 3 * dm.d * 4 > WIN_MAX_BYTES) p.ts = p.ts / 32 * 16;
     p.nseg = (int)((dm.L + p.ts - 1) / p.ts);
     p.nrows = dm.bs * p.nseg;
-    p.threads = p.nvec >= 256 ? 256 : ((p.nvec + 63) / 64) * 64;
-    p.ncvb = (p.nvec + p.threads - 1) / p.threads;
+    p.threads = 64 * r.waves;
+    p.ncvb = r.ncvb;
     p.nwg = dm.bs * p.nseg * p.ncvb;
     return p;
 }

@@ -37,6 +37,16 @@ template <bool KEEP> __device__ __forceinline__ void store_piece_as(win_t w, uin
 {
     win_store_as<KEEP>(w, off, u32x3{p[0][0], p[1][0], p[2][0]});
 }
+// (with the cache-policy bits given)
+template <int AUX> __device__ __forceinline__ void load_piece_aux(win_t w, uint32_t off, u32x1 (&p)[3])
+{
+    const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(w, (int)off, 0, AUX);
+    p[0][0] = v[0]; p[1][0] = v[1]; p[2][0] = v[2];
+}
+template <int AUX> __device__ __forceinline__ void store_piece_aux(win_t w, uint32_t off, const u32x1 (&p)[3])
+{
+    __builtin_amdgcn_raw_buffer_store_b96(u32x3{p[0][0], p[1][0], p[2][0]}, w, (int)off, 0, AUX);
+}
 template <typename R> __device__ __forceinline__ void load_piece(win_t w, uint32_t off, R (&p)[3])
 {
     constexpr int NB = sizeof(R);
@@ -100,6 +110,42 @@ template <typename T, int VV> __device__ __forceinline__ typename Vec<T, VV>::ra
     return r;
 }
 
+
+// How a walk kernel cuts (bs, L) rows of nvec lane vectors into workgroups of `waves` waves (64 lanes each, ncvb of them
+// side by side) and runs of ts rows.  The waves that the fullest SIMD gets, together or one after the other, times the rows a
+// wave walks -- its run and `extra` rows of halo and set-up -- is what a launch takes, so the plan is the smallest such
+// product over the 256 CUs of four SIMDs, times `alone` for one wave per SIMD, which waits for its rows alone.
+// Runs are multiples of `unit` and at most `longest` rows; workgroups of four waves unless fewer leave less idle.  No more than
+// most_lanes lanes have work, unless even the longest runs need more (lanes leave partial sums behind).
+// (Against runs of a power of two that fill two workgroups per CU at least: mixer 3 x 17810 x 2512 bf16 backward 545 -> 435 us,
+// forward 296 -> 262, 2 x 5000 x 1600 fp32 backward 122 -> 105; operator backward 4 x 2000 x 1232 bf16 70 -> 49,
+// 3 x 20000 x 800 fp32 291 -> 255, 4 x 7000 x 2400 f16 240 -> 211; widths that are powers of two keep their plans.)
+struct RunPlan { int waves, ncvb, ts; };
+inline RunPlan plan_runs(int64_t bs, int64_t L, int64_t nvec, int unit, int longest, int extra, double alone,
+                         int64_t most_lanes)
+{
+    RunPlan best{0, 0, 0};
+    double least = 0;
+    const int64_t nw = (nvec + 63) / 64;
+    for (int k = nw < 4 ? (int)nw : 4; k >= 1; --k) {
+        const int64_t ncvb = (nw + k - 1) / k, per = bs * ncvb;                 // workgroups of one run's rows
+        const int64_t m0 = (per * ((L + longest - 1) / longest) * k + 1023) / 1024;     // waves per SIMD with the longest runs
+        for (int64_t m = m0; m < m0 + 6; ++m) {
+            const int64_t nseg = 256 * (4 * m / k) / per;
+            if (nseg < 1) continue;
+            const int64_t ts = ((L + nseg - 1) / nseg + unit - 1) / unit * unit;
+            const int64_t runs = (L + ts - 1) / ts;
+            if (ts > longest || bs * runs * nvec > most_lanes) continue;
+            const int64_t per_cu = (per * runs + 255) / 256, per_simd = (per_cu * k + 3) / 4;
+            const double cost = (double)per_simd * (double)(ts + extra) * (per_simd == 1 ? alone : 1.0);
+            if (best.waves == 0 || cost < least * (k == best.waves ? 1.0 : 0.97)) { best = RunPlan{k, (int)ncvb, (int)ts}; least = cost; }
+            if (ts == unit) break;
+        }
+        if (nw % k == 0) break;                                                  // no lane idle: fewer waves gain nothing
+    }
+    if (best.waves == 0) best = RunPlan{nw < 4 ? (int)nw : 4, (int)((nw + 3) / 4), longest};
+    return best;
+}
 
 // Filter-gradient reduction shared by the register-window kernels.  The walk kernels leave
 // partials ws[tap][row][col]: one row per (batch, run), one column per lane (or per channel);

@@ -66,25 +66,27 @@ __device__ __forceinline__ void row_floats(const typename Vec<T, V>::raw (&p)[3]
     }
 }
 
-struct WinPlan { int v, nvec, nseg, ts, ncvb, threads; int64_t nthreads, nwg; };
+struct WinPlan { int v, nvec, nseg, ts, ncvb, threads, xcd; int64_t nthreads, nwg; };
 
 
 // ---------------------------------------------------------------------------- forward
 // PK: x, B, C are interleaved in one tensor that starts at C (element stride 3).
 // EXTRA: also write the convolution before the post-gate (y2) and the pre-gate product (bx).
+// RAG: rows off the 128-byte lines (fwd_form).
 // Tensors are addressed through windows over the rows of this run, so no load or store sits
 // behind a branch: rows before the sequence start read as zero, rows past the run are dropped.
-template <typename T, int HL, int V, bool PK, bool EXTRA>
+template <typename T, int HL, int V, bool PK, bool EXTRA, bool RAG = false>
 __global__ __launch_bounds__(256) void window_fwd_kernel(const T *__restrict__ x, const T *__restrict__ B,
                                                          const T *__restrict__ C, const T *__restrict__ h,
                                                          T *__restrict__ y, T *__restrict__ y2,
                                                          T *__restrict__ bx, Dims dm, WinPlan pl)
 {
     typedef typename Vec<T, V>::raw raw_t;
+    constexpr int LD = RAG ? 0 : WIN_NT, ST = RAG ? 0 : WIN_NT_ST;    // cache policy
     constexpr int ES = sizeof(T), IS = PK ? 3 : 1;     // element bytes, element stride of the inputs
     // (batch, run, block of channel vectors) come from the workgroup index, so row offsets
     // are wave-uniform and only the channel offset is per lane
-    int64_t wg = blockIdx.x;
+    int64_t wg = pl.xcd ? xcd_contiguous_id(blockIdx.x, gridDim.x) : blockIdx.x;
     const int cvb = (int)(wg % pl.ncvb); wg /= pl.ncvb;
     const int seg = (int)(wg % pl.nseg);
     const int64_t b = wg / pl.nseg;
@@ -118,11 +120,11 @@ __global__ __launch_bounds__(256) void window_fwd_kernel(const T *__restrict__ x
     auto load_in = [&](int64_t t, raw_t (&p)[3], bool with_c) {
         const uint32_t o = lane_i + (uint32_t)(t - t0) * irow;
         if constexpr (PK) {
-            load_piece(wx, o, p);
+            load_piece_aux<LD>(wx, o, p);
         } else {
-            p[0] = win_load<raw_t>(wx, o);
-            p[1] = win_load<raw_t>(wB, o);
-            p[2] = with_c ? win_load<raw_t>(wC, o) : zero_raw<T, V>();
+            p[0] = win_load_aux<LD, raw_t>(wx, o);
+            p[1] = win_load_aux<LD, raw_t>(wB, o);
+            p[2] = with_c ? win_load_aux<LD, raw_t>(wC, o) : zero_raw<T, V>();
         }
     };
 
@@ -179,12 +181,12 @@ __global__ __launch_bounds__(256) void window_fwd_kernel(const T *__restrict__ x
                     for (int v = 0; v < V; ++v) acc[v] = fmaf(hr[j], ring[(k - j) & (RING - 1)][v], acc[v]);
                 const uint32_t o = lane_o + (uint32_t)(t - t0) * orow;
                 if constexpr (EXTRA) {
-                    win_store(wy2, o, packv<T, V>(acc));
-                    win_store(wbx, o, packv<T, V>(ring[k]));
+                    win_store_aux<ST>(wy2, o, packv<T, V>(acc));
+                    win_store_aux<ST>(wbx, o, packv<T, V>(ring[k]));
                 }
 #pragma unroll
                 for (int v = 0; v < V; ++v) out[v] = Cf[v] * acc[v];
-                win_store(wy, o, packv<T, V>(out));
+                win_store_aux<ST>(wy, o, packv<T, V>(out));
             }
         }
     }
@@ -388,53 +390,73 @@ __global__ __launch_bounds__(256) void window_bwd_kernel(const T *__restrict__ d
         if (j < hl) slot[(size_t)(hl - 1 - j) * pl.nthreads] = dha[j];
 }
 
-WinPlan plan(const Dims &dm, int v)
+WinPlan plan(const Dims &dm, int v, int longest, int64_t most_lanes)
 {
     WinPlan p;
     p.v = v;
     p.nvec = (int)(dm.d / v);
-    p.ts = 1024;
-    // the longest runs (up to 1024 rows) that still leave two workgroups per CU: measured best at the
-    // 7B and 40B shapes for either operand layout (fewer halo rows and filter-gradient partials;
-    // one step further and the machine is no longer covered)
-    while (p.ts > 8 && dm.bs * ((dm.L + p.ts - 1) / p.ts) * p.nvec < 128 * 1024) p.ts >>= 1;
+    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, 1.3, most_lanes);
+    p.ts = r.ts;
     static const char *env = tuning_env("GCG_WINDOW_ROWS");   // tuning override: rows per lane, a multiple of 8
     if (env && atoi(env) >= 8 && atoi(env) % 8 == 0) p.ts = atoi(env);
     // the rows of a run, its halo and an interleaved fp32 row width must fit one tensor window
-    while (p.ts > 8 && (int64_t)(p.ts + 2 * RING) * 3 * dm.d * 4 * (dm.tmajor ? dm.bs : 1) > WIN_MAX_BYTES) p.ts >>= 1;   // (planar rows are 3 d wide too)
+    while (p.ts > 8 && (int64_t)(p.ts + 2 * RING) * 3 * dm.d * 4 * (dm.tmajor ? dm.bs : 1) > WIN_MAX_BYTES) p.ts = p.ts / 2 / RING * RING;   // (planar rows are 3 d wide too)
+    p.xcd = 0;
     p.nseg = (int)((dm.L + p.ts - 1) / p.ts);
     p.nthreads = dm.bs * p.nseg * p.nvec;       // workspace slots (one per lane with work)
-    p.threads = p.nvec >= 256 ? 256 : ((p.nvec + 63) / 64) * 64;   // narrow tensors: fewer idle lanes
-    p.ncvb = (p.nvec + p.threads - 1) / p.threads;
+    p.threads = 64 * r.waves;
+    p.ncvb = r.ncvb;
     p.nwg = dm.bs * p.nseg * p.ncvb;
     return p;
 }
+// the longest runs of the backward: up to 1024 rows, measured best at the 7B and 40B shapes for either operand layout (fewer
+// halo rows and filter-gradient partials).  Lanes: eight filter-gradient partials of each fill the static scratch.
+constexpr int BWD_ROWS = 1024;
+constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(float));
 
 constexpr int BWD_V = 4;   // the backward keeps four rings per lane: 4 channels is what fits
 // interleaved operands: the lane width that makes a row piece 12 contiguous bytes
 template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
+
+// How the forward walks, by how its rows lie.  Rows of a multiple of 8 KB: long runs, streaming accesses, plain order of
+// workgroups (1 x 32768 x 8192 bf16 377 us; short runs in XCD order 411).  Other whole lines: runs of at most 128 rows in
+// XCD-contiguous order (1 x 399457 x 1344 1032 -> 840 us, 1 x 38836 x 3456 227 -> 214).  Rows off the lines: plain accesses,
+// so that the parts of a shared line meet in the L2, and at most 64 rows (1 x 264208 x 2032 1415 -> 865 us, 1 x 46091 x 2912
+// 262 -> 217; with streaming accesses 925 and 225).
+struct FwdForm { int longest; bool rag, xcd; };
+FwdForm fwd_form(const Dims &dm, size_t es)
+{
+    const uint64_t row = (uint64_t)dm.d * es;
+    const bool rag = row % 128 != 0, wide = row % 8192 == 0;
+    return FwdForm{wide ? 1024 : rag ? 64 : 128, rag, !wide && !dm.tmajor};
+}
 
 template <typename T, int HL, int V>
 int fwd_v(const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
           const Dims &dm, hipStream_t st)
 {
     int e = 0;
+    const FwdForm form = fwd_form(dm, sizeof(T));
+    const bool rag = form.rag;
     if (dm.es == 3) {
         constexpr int VI = il_v<T>();
-        const WinPlan p = plan(dm, VI);
+        WinPlan p = plan(dm, VI, form.longest, INT64_MAX);
+        p.xcd = form.xcd;
         if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-        e = launch_main((window_fwd_kernel<T, HL, VI, true, false>), dim3((unsigned)p.nwg), dim3(p.threads), st,
+        const auto kern = rag ? window_fwd_kernel<T, HL, VI, true, false, true> : window_fwd_kernel<T, HL, VI, true, false>;
+        e = launch_main(kern, dim3((unsigned)p.nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
         return e;
     }
-    const WinPlan p = plan(dm, V);
+    WinPlan p = plan(dm, V, form.longest, INT64_MAX);
+    p.xcd = form.xcd;
     const int64_t nwg = p.nwg;
     if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if (y2 || bx)
         e = launch_main((window_fwd_kernel<T, HL, V, false, true>), dim3((unsigned)nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
     else
-        e = launch_main((window_fwd_kernel<T, HL, V, false, false>), dim3((unsigned)nwg), dim3(p.threads), st,
+        e = launch_main(rag ? window_fwd_kernel<T, HL, V, false, false, true> : window_fwd_kernel<T, HL, V, false, false>, dim3((unsigned)nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
     return e;
 }
@@ -444,7 +466,7 @@ int bwd_t(const void *dy, const void *x, const void *B, const void *C, const voi
           void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const WinPlan p = plan(dm, dm.es == 3 ? il_v<T>() : BWD_V);
+    const WinPlan p = plan(dm, dm.es == 3 ? il_v<T>() : BWD_V, BWD_ROWS, BWD_LANES);
     const int64_t nwg = p.nwg;
     if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if (dm.es == 3 && dm.keep_out)
@@ -521,7 +543,7 @@ size_t window_bwd_workspace(const Dims &dm)
     int64_t n = 0;
     for (int v : {1, 2, BWD_V}) {
         if (dm.d % v) continue;
-        const WinPlan p = plan(dm, v);
+        const WinPlan p = plan(dm, v, BWD_ROWS, BWD_LANES);
         if (p.nthreads > n) n = p.nthreads;
     }
     return (size_t)n * dm.hl * sizeof(float);

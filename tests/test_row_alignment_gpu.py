@@ -50,3 +50,33 @@ def test_planar_features(dtype, arith, hl, g):
     assert torch.equal(_lib.fwd_planar(fw, h)[..., :g, :], _lib.fwd_planar(fn, h[:g].contiguous()))
     rw, rn = _lib.bwd_planar(dyw, fw, h), _lib.bwd_planar(dyn, fn, h[:g].contiguous())
     assert torch.equal(rw[0][..., :g, :], rn[0])
+
+
+@pytest.mark.parametrize("dtype,arith", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("bs,L,g,wide", [(1, 700, 5, 8), (2, 3001, 29, 32), (3, 90, 54, 64), (1, 40000, 11, 16)])
+@pytest.mark.parametrize("planar", [False, True])
+def test_register_window_kernels(dtype, arith, bs, L, g, wide, planar):
+    """Run lengths and workgroups of one to four waves, chosen by the width: operator on interleaved features, short mixer."""
+    dg, hl = 16, 7
+    gen = torch.Generator(device=DEV).manual_seed(L + g)
+    lay = {"lead": (3,)} if planar else {"tail": (3,)}
+    cut = (lambda t: t[..., :g, :]) if planar else (lambda t: t[:, :, :g])
+    rw, rn = _pair(bs, L, g, wide, dg, dtype, gen, **lay)
+    dyw, dyn = _pair(bs, L, g, wide, dg, dtype, gen)
+    h = (torch.randn(wide, 1, hl, generator=gen, device=DEV) / hl ** 0.5).to(arith)
+    hn = h[:g].contiguous()
+    wf = torch.randn(3, wide, dg, 3, generator=gen, device=DEV).to(dtype) / 2
+    wfw, wfn = ((t if planar else t.permute(1, 2, 0, 3)).reshape(-1, 1, 3).contiguous() for t in (wf, wf[:, :g]))
+    if not planar:
+        assert torch.equal(_lib.fwd_interleaved(rw, h)[:, :, :g], _lib.fwd_interleaved(rn, hn))
+        assert torch.equal(cut(_lib.bwd_interleaved(dyw, rw, h)[0]), _lib.bwd_interleaved(dyn, rn, hn)[0])
+    assert torch.equal(_lib.mixer_se_fwd(rw, wfw, h, planar)[:, :, :g], _lib.mixer_se_fwd(rn, wfn, hn, planar))
+    a, b = _lib.mixer_se_bwd(dyw, rw, wfw, h, planar), _lib.mixer_se_bwd(dyn, rn, wfn, hn, planar)
+    assert torch.equal(cut(a[0]), b[0])
+    # filter gradients: the same fp32 products in sums that are cut differently (errors of sums grow like the root of
+    # their terms, as the sums themselves do), one rounding to the filter's type
+    ulp = {torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11, torch.float32: 1e-5}
+    dwa = a[1].reshape(3, wide, dg, 3) if planar else a[1].reshape(wide, dg, 3, 3).permute(2, 0, 1, 3)
+    dwb = b[1].reshape(3, g, dg, 3) if planar else b[1].reshape(g, dg, 3, 3).permute(2, 0, 1, 3)
+    assert (dwa[:, :g].float() - dwb.float()).abs().max() <= ulp[dtype] * dwa.float().abs().max()
+    assert (a[2][:g].float() - b[2].float()).abs().max() <= ulp[arith] * a[2].float().abs().max()

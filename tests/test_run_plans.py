@@ -1,4 +1,5 @@
 """How the matrix-core backwards cut their work into runs and launches, seen through the scratch their partial sums need."""
+import random
 import time
 
 import pytest
@@ -35,6 +36,23 @@ def test_static_scratch_holds_what_it_held(bs, nsteps, hl):
 def test_small_launches_stay_far_below_it(cols, hl):
     for nsteps in (1, 7, 16, 31, 75, 200):
         assert 0 < scratch(cols, 32 * nsteps, 4, hl) <= 2304 * 2048 + 4096
+
+
+def test_register_window_backward_stays_in_static_scratch():
+    """Runs cut to fill the SIMDs leave no more partial sums than 8 MiB hold, or than runs of a power of two up to 1024 rows
+    that give 2^17 lanes work."""
+    rng = random.Random(7)
+    for _ in range(3000):
+        bs, L, g = int(2 ** rng.uniform(0, 6)), int(2 ** rng.uniform(0, 18)), int(2 ** rng.uniform(0, 10))
+        dg, hl = rng.choice([4, 8, 12, 16, 32, 64]), rng.randint(1, 8)
+        most = 0
+        for v in (1, 2, 4):
+            ts = 1024
+            while ts > 8 and bs * -(-L // ts) * (g * dg // v) < 1 << 17:
+                ts >>= 1
+            most = max(most, bs * -(-L // ts) * (g * dg // v))
+        got = _lib.load().gcg_bwd_workspace_bytes(bs, L, g, dg, hl, _lib.GCG_BF16, _lib.ALGO_NAMES["window"])
+        assert 0 < got <= max(STATIC, most * hl * 4 + 256), (bs, L, g, dg, hl)
 
 
 @pytest.mark.parametrize("code", CODES)
