@@ -39,6 +39,9 @@ OP_NAMES = (
     "fwd_planar", "bwd_planar",
 )
 
+# differentiable as they are: C++ autograd nodes around operators above, which a trace sees in their place
+NODE_NAMES = ("gate_conv_gate", "gate_conv_gate_decay", "short_hyena", "mixer_mr", "mixer_mr_decay")
+
 
 # ---- autograd --------------------------------------------------------------------------------------------
 # Every forward operator has its backward formula registered, so that a call of torch.ops.gcg.* on tensors that

@@ -11,6 +11,7 @@
 // as TwoPassChunkedGateConvGate calls them (cgcg/interface.py:27-127).
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 #include <torch/types.h>
 
@@ -857,10 +858,153 @@ std::tuple<Tensor, Tensor, Tensor> mixer_mr_bwd_meta(const Tensor &dy, const Ten
     return {at::empty_like(raw), at::empty_like(wf), at::empty_like(h)};
 }
 
+// ---- differentiable calls without Python in the graph ------------------------------------------------
+// The autograd functions of the layers (savanna_amd/kernels, savanna_amd/operators) as C++ nodes: same operators, same
+// tensors saved, but the backward runs on autograd's device thread without the interpreter, whose lock that thread and the
+// caller otherwise hand to and fro.  Forward and backward call the operators above through the dispatcher, so modes see them.
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+template <typename F> c10::TypedOperatorHandle<F> op(const char *name)
+{
+    return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
+}
+
+struct GatedConvGate : torch::autograd::Function<GatedConvGate> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &B, const Tensor &C, const Tensor &h)
+    {
+        static const auto f = op<Tensor(const Tensor &, const Tensor &, const Tensor &, const Tensor &, int64_t)>("gcg::fwd");
+        at::AutoDispatchBelowADInplaceOrView below;
+        ctx->save_for_backward({x, B, C, h});
+        return f.call(x, B, C, h, GCG_ALGO_AUTO);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list dy)
+    {
+        static const auto f = op<std::tuple<Tensor, Tensor, Tensor, Tensor>(const Tensor &, const Tensor &, const Tensor &,
+                                                                           const Tensor &, const Tensor &, int64_t)>("gcg::bwd");
+        const variable_list s = ctx->get_saved_variables();
+        auto [dx, dB, dC, dh] = f.call(dy[0].contiguous(), s[0], s[1], s[2], s[3], GCG_ALGO_AUTO);
+        return {dx, dB, dC, dh};
+    }
+};
+
+struct DecayedGateConvGate : torch::autograd::Function<DecayedGateConvGate> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &B, const Tensor &C, const Tensor &w,
+                          const Tensor &decay, int64_t hl, at::ScalarType filt)
+    {
+        static const auto f = op<Tensor(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const Tensor &, int64_t,
+                                        at::ScalarType)>("gcg::fwd_decay");
+        at::AutoDispatchBelowADInplaceOrView below;
+        ctx->save_for_backward({x, B, C, w, decay});
+        ctx->saved_data["hl"] = hl;
+        ctx->saved_data["filt"] = (int64_t)filt;
+        return f.call(x, B, C, w, decay, hl, filt);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list dy)
+    {
+        static const auto f = op<std::tuple<Tensor, Tensor, Tensor, Tensor>(const Tensor &, const Tensor &, const Tensor &,
+                                                                           const Tensor &, const Tensor &, const Tensor &, int64_t,
+                                                                           at::ScalarType)>("gcg::bwd_decay");
+        const variable_list s = ctx->get_saved_variables();
+        auto [dx, dB, dC, dw] = f.call(dy[0].contiguous(), s[0], s[1], s[2], s[3], s[4], ctx->saved_data["hl"].toInt(),
+                                       (at::ScalarType)ctx->saved_data["filt"].toInt());
+        return {dx, dB, dC, dw, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// run_short_hyena's operands: y = q * conv(k * v, w)
+struct TimeMajorShortHyena : torch::autograd::Function<TimeMajorShortHyena> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &w)
+    {
+        static const auto f = op<Tensor(const Tensor &, const Tensor &, const Tensor &, const Tensor &)>("gcg::fwd_time_major");
+        at::AutoDispatchBelowADInplaceOrView below;
+        ctx->save_for_backward({q, k, v, w});
+        return f.call(v, k, q, w);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list dy)
+    {
+        static const auto f = op<std::tuple<Tensor, Tensor, Tensor, Tensor>(const Tensor &, const Tensor &, const Tensor &,
+                                                                           const Tensor &, const Tensor &)>("gcg::bwd_time_major");
+        const variable_list s = ctx->get_saved_variables();
+        auto [dv, dk, dq, dw] = f.call(dy[0].contiguous(), s[2], s[1], s[0], s[3]);
+        return {dq, dk, dv, dw};
+    }
+};
+
+struct FeaturizedGateConvGate : torch::autograd::Function<FeaturizedGateConvGate> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &raw, const Tensor &wf, const Tensor &h, bool planar)
+    {
+        static const auto f = op<Tensor(const Tensor &, const Tensor &, const Tensor &, bool)>("gcg::mixer_mr_fwd");
+        at::AutoDispatchBelowADInplaceOrView below;
+        ctx->save_for_backward({raw, wf, h});
+        ctx->saved_data["planar"] = planar;
+        return f.call(raw, wf, h, planar);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list dz)
+    {
+        static const auto f = op<std::tuple<Tensor, Tensor, Tensor>(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
+                                                                   bool)>("gcg::mixer_mr_bwd");
+        const variable_list s = ctx->get_saved_variables();
+        auto [draw, dwf, dh] = f.call(dz[0].contiguous(), s[0], s[1], s[2], ctx->saved_data["planar"].toBool());
+        return {draw, dwf, dh, Tensor()};
+    }
+};
+
+struct FeaturizedDecayedGateConvGate : torch::autograd::Function<FeaturizedDecayedGateConvGate> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &raw, const Tensor &wf, const Tensor &w, const Tensor &decay,
+                          int64_t hl, at::ScalarType filt, bool planar)
+    {
+        static const auto f = op<Tensor(const Tensor &, const Tensor &, const Tensor &, const Tensor &, int64_t, at::ScalarType,
+                                        bool)>("gcg::mixer_mr_fwd_decay");
+        at::AutoDispatchBelowADInplaceOrView below;
+        ctx->save_for_backward({raw, wf, w, decay});
+        ctx->saved_data["hl"] = hl;
+        ctx->saved_data["filt"] = (int64_t)filt;
+        ctx->saved_data["planar"] = planar;
+        return f.call(raw, wf, w, decay, hl, filt, planar);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list dz)
+    {
+        static const auto f = op<std::tuple<Tensor, Tensor, Tensor>(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
+                                                                   const Tensor &, int64_t, at::ScalarType, bool)>("gcg::mixer_mr_bwd_decay");
+        const variable_list s = ctx->get_saved_variables();
+        auto [draw, dwf, dw] = f.call(dz[0].contiguous(), s[0], s[1], s[2], s[3], ctx->saved_data["hl"].toInt(),
+                                      (at::ScalarType)ctx->saved_data["filt"].toInt(), ctx->saved_data["planar"].toBool());
+        return {draw, dwf, dw, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor gate_conv_gate(const Tensor &x, const Tensor &B, const Tensor &C, const Tensor &h)
+{
+    return GatedConvGate::apply(x, B, C, h);
+}
+Tensor gate_conv_gate_decay(const Tensor &x, const Tensor &B, const Tensor &C, const Tensor &w, const Tensor &decay, int64_t hl,
+                            at::ScalarType filt)
+{
+    return DecayedGateConvGate::apply(x, B, C, w, decay, hl, filt);
+}
+Tensor short_hyena(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &w) { return TimeMajorShortHyena::apply(q, k, v, w); }
+Tensor mixer_mr(const Tensor &raw, const Tensor &wf, const Tensor &h, bool planar)
+{
+    return FeaturizedGateConvGate::apply(raw, wf, h, planar);
+}
+Tensor mixer_mr_decay(const Tensor &raw, const Tensor &wf, const Tensor &w, const Tensor &decay, int64_t hl, at::ScalarType filt,
+                      bool planar)
+{
+    return FeaturizedDecayedGateConvGate::apply(raw, wf, w, decay, hl, filt, planar);
+}
+
 } // namespace
 
 TORCH_LIBRARY(gcg, m)
 {
+    m.def("gate_conv_gate(Tensor x, Tensor B, Tensor C, Tensor h) -> Tensor", &gate_conv_gate);
+    m.def("gate_conv_gate_decay(Tensor x, Tensor B, Tensor C, Tensor w, Tensor decay, int hl, ScalarType filt) -> Tensor",
+          &gate_conv_gate_decay);
+    m.def("short_hyena(Tensor q, Tensor k, Tensor v, Tensor w) -> Tensor", &short_hyena);
+    m.def("mixer_mr(Tensor raw, Tensor wf, Tensor h, bool planar=False) -> Tensor", &mixer_mr);
+    m.def("mixer_mr_decay(Tensor raw, Tensor wf, Tensor w, Tensor decay, int hl, ScalarType filt, bool planar=False) -> Tensor",
+          &mixer_mr_decay);
     m.def("fwd(Tensor x, Tensor B, Tensor C, Tensor h, int algo=0) -> Tensor");
     m.def("fwd_full(Tensor x, Tensor B, Tensor C, Tensor h, bool return_bx, bool return_y2, int algo=0)"
           " -> (Tensor, Tensor, Tensor)");

@@ -62,7 +62,8 @@ def run_short_hyena(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w: torch.
         groups, width = g * dg, 1
     if repeat_interleave and q.is_cuda and _lib.time_major_supported(dg, hl, q, k, v):
         w3 = w.reshape(g, 1, hl)
-        y = _TimeMajorShortHyena.apply(q, k, v, w3 if w3.is_contiguous() else w3.contiguous())
+        w3 = w3 if w3.is_contiguous() else w3.contiguous()
+        y = _lib.fwd_time_major(v, k, q, w3) if _lib.native_nodes(q) else _TimeMajorShortHyena.apply(q, k, v, w3)
         return y.permute(0, 2, 1, 3)
     to_blgd = lambda t: t.permute(1, 0, 2, 3).reshape(bs, seqlen, groups, width)
     y = two_pass_chunked_gate_conv_gate(to_blgd(v), to_blgd(k), to_blgd(q), w.reshape(groups, 1, hl),

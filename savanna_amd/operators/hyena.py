@@ -26,8 +26,8 @@ import torch
 import torch.nn as nn
 
 from .. import _lib
-from ..kernels.cgcg.interface import (DecayedGateConvGate, InterleavedDecayedGateConvGate,
-                                       planar_source, two_pass_chunked_gate_conv_gate,
+from ..kernels.cgcg.interface import (DecayedGateConvGate, InterleavedDecayedGateConvGate,  # noqa: F401
+                                       decayed_gate_conv_gate, planar_source, two_pass_chunked_gate_conv_gate,
                                        two_pass_chunked_gate_conv_gate_interleaved,
                                        two_pass_chunked_gate_conv_gate_planar)
 from ..kernels.cgcg.src.kernel_utils import BwdKernelConfigRefactor, FwdKernelConfigRefactor
@@ -150,7 +150,7 @@ class _CgcgOperatorBase(nn.Module):
         fused = self._filter_in_kernel(x1.shape[1], x1.shape[2], x1.shape[3], dtype, x1, x2, v)
         if fused is not None:
             hl, filt = fused
-            z = DecayedGateConvGate.apply(v, x2, x1, self.filter.h, self.filter.decay, hl, filt)
+            z = decayed_gate_conv_gate(v, x2, x1, self.filter.h, self.filter.decay, hl, filt)
             return z.reshape(z.shape[0], z.shape[1], -1)
         h = self._filter(x1.shape[1])
         x, B, C = v, x2, x1
@@ -373,6 +373,13 @@ class _FeaturizedDecayedGateConvGate(torch.autograd.Function):
         return draw, dwf, dw, None, None, None, None
 
 
+def _featurized(entry, function, tensors, *rest):
+    """The entry point itself, or its Python autograd function (``_lib.native_nodes``)."""
+    if _lib.native_nodes(tensors[0]):
+        return entry(*(t if t.is_contiguous() else t.contiguous() for t in tensors), *rest)
+    return function.apply(*tensors, *rest)
+
+
 class HyenaMixer(nn.Module):
     """The convolutional part of ParallelSequenceMixer.forward for the hyena operators
     (savanna/model/block.py:865-890): featurizer conv on the projected features, interleaved split,
@@ -454,13 +461,14 @@ class HyenaMixer(nn.Module):
         # Hyena-MR: one kernel each way, with the decayed filter formed inside it where the operator allows that
         fused = op._filter_in_kernel(seqlen, g, dg, features.dtype, features)
         if fused is not None and self._medium(features, fused[0]):
-            z = _FeaturizedDecayedGateConvGate.apply(features.reshape(shape), conv.short_conv_weight.to(features.dtype),
-                                                     op.filter.h, op.filter.decay, fused[0], fused[1], planar)
+            z = _featurized(_lib.mixer_mr_fwd_decay, _FeaturizedDecayedGateConvGate,
+                            (features.reshape(shape), conv.short_conv_weight.to(features.dtype), op.filter.h, op.filter.decay),
+                            fused[0], fused[1], planar)
             return z.reshape(bs, seqlen, g * dg)
         h = op._filter(seqlen)
         if self._medium(features, h.shape[-1]):
-            z = _FeaturizedGateConvGate.apply(features.reshape(shape), conv.short_conv_weight.to(features.dtype),
-                                              h.to(op.cgcg_dtype), planar)
+            z = _featurized(_lib.mixer_mr_fwd, _FeaturizedGateConvGate,
+                            (features.reshape(shape), conv.short_conv_weight.to(features.dtype), h.to(op.cgcg_dtype)), planar)
             return z.reshape(bs, seqlen, g * dg)
         # Hyena-SE: one kernel each way
         if self._fusable(features, h.shape[-1]):
