@@ -31,7 +31,7 @@ __device__ __forceinline__ void load_taps(const T *w, int64_t c, int dg, int hl,
     }
 }
 
-template <typename T, int HL, int V, bool PCF, bool KEEP>
+template <typename T, int HL, int V, bool PCF, bool KEEP, bool RAG = false>
 __global__ __launch_bounds__(256) void dwconv_fwd_kernel(const T *__restrict__ x, const T *__restrict__ w,
                                                          T *__restrict__ y, Dims dm, DwPlan pl)
 {
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void dwconv_fwd_kernel(const T *__restrict__ x
     {   // halo: rows t_start-(HL-1) .. t_start-1 (zero before the sequence) go to slots (t & 7)
         raw_t halo[HL - 1 > 0 ? HL - 1 : 1];
 #pragma unroll
-        for (int i = 1; i < HL; ++i) halo[i - 1] = win_load<raw_t>(wx, lane + (uint32_t)(t_start - i - t0) * row);
+        for (int i = 1; i < HL; ++i) halo[i - 1] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wx, lane + (uint32_t)(t_start - i - t0) * row);
 #pragma unroll
         for (int i = 1; i < HL; ++i) unpackv<T, V>(halo[i - 1], ring[RING - i]);
     }
@@ -71,14 +71,14 @@ __global__ __launch_bounds__(256) void dwconv_fwd_kernel(const T *__restrict__ x
     // rows are fetched BATCH at a time, one batch ahead
     raw_t in[2][BATCH];
 #pragma unroll
-    for (int kk = 0; kk < BATCH; ++kk) in[0][kk] = win_load<raw_t>(wx, lane + (uint32_t)(t_start + kk - t0) * row);
+    for (int kk = 0; kk < BATCH; ++kk) in[0][kk] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wx, lane + (uint32_t)(t_start + kk - t0) * row);
     for (int64_t tb = t_start; tb < t_end; tb += RING) {
 #pragma unroll
         for (int half = 0; half < RING / BATCH; ++half) {
             const int cur = half % 2, nxt = (half + 1) % 2;
 #pragma unroll
             for (int kk = 0; kk < BATCH; ++kk)
-                in[nxt][kk] = win_load<raw_t>(wx, lane + (uint32_t)(tb + (half + 1) * BATCH + kk - t0) * row);
+                in[nxt][kk] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wx, lane + (uint32_t)(tb + (half + 1) * BATCH + kk - t0) * row);
 #pragma unroll
             for (int kk = 0; kk < BATCH; ++kk) {
                 const int k = half * BATCH + kk;
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void dwconv_fwd_kernel(const T *__restrict__ x
 #pragma unroll
                     for (int v = 0; v < V; ++v)
                         acc[v] = fmaf(hr[j][PCF ? v : 0], ring[(k - j) & (RING - 1)][v], acc[v]);
-                win_store_as<KEEP>(wy, lane + (uint32_t)(tb + k - t0) * row, packv<T, V>(acc));
+                win_store_aux<KEEP || RAG ? 0 : WIN_NT_ST>(wy, lane + (uint32_t)(tb + k - t0) * row, packv<T, V>(acc));
             }
         }
     }
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void dwconv_fwd_kernel(const T *__restrict__ x
 // Backward: dx[t] = sum_j w[hl-1-j] dy[t+j] looks forward, so the walk runs HL-1 rows past the
 // run reading only dy; dw[hl-1-j] = sum_t dy[t] x[t-j] is accumulated per lane over the rows of
 // the run and reduced by a second kernel in a fixed order.
-template <typename T, int HL, int V, bool PCF>
+template <typename T, int HL, int V, bool PCF, bool RAG = false>
 __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                          const T *__restrict__ w, T *__restrict__ dx,
                                                          float *__restrict__ ws, Dims dm, DwPlan pl)
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ d
     {
         raw_t halo[HL - 1 > 0 ? HL - 1 : 1];
 #pragma unroll
-        for (int i = 1; i < HL; ++i) halo[i - 1] = win_load<raw_t>(wx, lane + (uint32_t)(t_start - i - t0) * row);
+        for (int i = 1; i < HL; ++i) halo[i - 1] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wx, lane + (uint32_t)(t_start - i - t0) * row);
 #pragma unroll
         for (int i = 1; i < HL; ++i) unpackv<T, V>(halo[i - 1], ur[RING - i]);
     }
@@ -156,8 +156,8 @@ __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ d
 #pragma unroll
             for (int kk = 0; kk < BATCH; ++kk) {
                 const uint32_t o = lane + (uint32_t)(tb + half * BATCH + kk - t0) * row;
-                xr[kk] = win_load<raw_t>(wx, o);      // zero past the run
-                dyr[kk] = win_load<raw_t>(wdy, o);
+                xr[kk] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wx, o);      // zero past the run
+                dyr[kk] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wdy, o);
             }
 #pragma unroll
             for (int kk = 0; kk < BATCH; ++kk) {
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ d
 #pragma unroll
                     for (int v = 0; v < V; ++v)
                         du[v] = fmaf(hr[j][PCF ? v : 0], gr[(k - (HL - 1) + j) & (RING - 1)][v], du[v]);
-                win_store(wdx, lane + (uint32_t)(t - (HL - 1) - t_start) * row, packv<T, V>(du));
+                win_store_aux<RAG ? 0 : WIN_NT_ST>(wdx, lane + (uint32_t)(t - (HL - 1) - t_start) * row, packv<T, V>(du));
             }
         }
     }
@@ -214,31 +214,43 @@ int lane_width(int dtype, const Dims &dm)
     return 4;
 }
 
-DwPlan plan(const Dims &dm, int V)
+// Forward: the longest runs of a power of two up to 128 rows that give two workgroups per CU (the other plan: 119 against
+// 127 us at 1 x 12000 x 12288 bf16).  Backward: plan_runs (187 -> 178 us there, 12144 channels 219 -> 210).
+DwPlan plan(const Dims &dm, int V, bool backward)
 {
     DwPlan p;
     p.v = V;
     p.nvec = (int)(dm.d / V);
-    p.ts = 128;
-    while (p.ts > 8 && dm.bs * ((dm.L + p.ts - 1) / p.ts) * p.nvec < 128 * 1024) p.ts >>= 1;
+    RunPlan r{p.nvec >= 256 ? 4 : (p.nvec + 63) / 64, 0, 128};
+    if (backward) r = plan_runs(dm.bs, dm.L, p.nvec, RING, 128, RING, 1.3, INT64_MAX, true);
+    else while (r.ts > 8 && dm.bs * ((dm.L + r.ts - 1) / r.ts) * p.nvec < 128 * 1024) r.ts >>= 1;
+    p.ts = r.ts;
     static const char *env = tuning_env("GCG_DWCONV_ROWS");     // tuning override: rows per lane, a multiple of 8
     if (env && atoi(env) >= 8 && atoi(env) % 8 == 0) p.ts = atoi(env);
-    while (p.ts > 8 && (int64_t)(p.ts + 2 * RING) * dm.d * 4 > WIN_MAX_BYTES) p.ts >>= 1;
+    while (p.ts > 8 && (int64_t)(p.ts + 2 * RING) * dm.d * 4 > WIN_MAX_BYTES) p.ts = p.ts / 2 / RING * RING;
     p.nseg = (int)((dm.L + p.ts - 1) / p.ts);
     p.nrows = dm.bs * p.nseg;
-    p.threads = p.nvec >= 256 ? 256 : ((p.nvec + 63) / 64) * 64;
+    p.threads = 64 * r.waves;
     p.ncvb = (p.nvec + p.threads - 1) / p.threads;
     p.nwg = dm.bs * p.nseg * p.ncvb;
     return p;
 }
 
+// Rows that start and end on odd 32-byte sectors are accessed without the streaming hint: the parts of a shared 64 bytes then
+// meet in the L2 (3 x 17810 x 7536 bf16: forward 400 -> 390 us, 426 -> 390 with GCG_KEEP_OUTPUT, backward 608 -> 583; rows of
+// whole lines 154 -> 165 and 236 -> 254).
+template <typename T> bool ragged(const Dims &dm) { return (uint64_t)dm.d * sizeof(T) % 64 != 0; }
+
 template <typename T, int HL, int V, bool PCF>
 int fwd_launch(const void *x, const void *w, void *y, const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const DwPlan p = plan(dm, V);
+    const DwPlan p = plan(dm, V, false);
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-    if (dm.keep_out)
+    if (ragged<T>(dm))
+        e = launch_plain((dwconv_fwd_kernel<T, HL, V, PCF, true, true>), dim3((unsigned)p.nwg), dim3(p.threads), st,
+                           (const T *)x, (const T *)w, (T *)y, dm, p);
+    else if (dm.keep_out)
         e = launch_plain((dwconv_fwd_kernel<T, HL, V, PCF, true>), dim3((unsigned)p.nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)w, (T *)y, dm, p);
     else
@@ -252,9 +264,9 @@ int bwd_launch(const void *dy, const void *x, const void *w, void *dx, void *dw,
                hipStream_t st)
 {
     int e = 0;
-    const DwPlan p = plan(dm, V);
+    const DwPlan p = plan(dm, V, true);
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-    e = launch_plain((dwconv_bwd_kernel<T, HL, V, PCF>), dim3((unsigned)p.nwg), dim3(p.threads), st,
+    e = launch_plain(ragged<T>(dm) ? dwconv_bwd_kernel<T, HL, V, PCF, true> : dwconv_bwd_kernel<T, HL, V, PCF>, dim3((unsigned)p.nwg), dim3(p.threads), st,
                        (const T *)dy, (const T *)x, (const T *)w, (T *)dx, (float *)ws, dm, p);
     if (e) return e;
     // partials are ws[tap][(batch, run)][slot], slot = channel (per-channel filters) or lane
@@ -327,7 +339,7 @@ size_t dwconv_bwd_workspace(const Dims &dm)
     size_t n = 0;
     for (int v : {4, 8}) {
         if (dm.d % v) continue;
-        const DwPlan p = plan(dm, v);
+        const DwPlan p = plan(dm, v, true);
         const int64_t nslot = dm.dg % v == 0 ? p.nvec : dm.d;
         const size_t need = (size_t)dm.hl * p.nrows * nslot * sizeof(float);
         if (need > n) n = need;

@@ -81,21 +81,22 @@ template <bool PL, int CH> __device__ __forceinline__ int64_t feat_channel(int64
 {
     return PL ? (int64_t)(e / CH) * d + c + e % CH : 3 * c + e;
 }
-template <bool PL> __device__ __forceinline__ u32x3 piece_load(win_t w, uint32_t off, uint32_t orow)
+// (LD, ST: cache-policy bits)
+template <bool PL, int LD = WIN_NT> __device__ __forceinline__ u32x3 piece_load(win_t w, uint32_t off, uint32_t orow)
 {
     if constexpr (PL)
-        return u32x3{win_load<uint32_t>(w, off), win_load<uint32_t>(w, off + orow), win_load<uint32_t>(w, off + 2 * orow)};
+        return u32x3{win_load_aux<LD, uint32_t>(w, off), win_load_aux<LD, uint32_t>(w, off + orow), win_load_aux<LD, uint32_t>(w, off + 2 * orow)};
     else
-        return win_load<u32x3>(w, off);
+        return __builtin_amdgcn_raw_buffer_load_b96(w, (int)off, 0, LD);
 }
-template <bool PL> __device__ __forceinline__ void piece_store(win_t w, uint32_t off, uint32_t orow, const u32x3 &v)
+template <bool PL, int ST = WIN_NT_ST> __device__ __forceinline__ void piece_store(win_t w, uint32_t off, uint32_t orow, const u32x3 &v)
 {
     if constexpr (PL) {
-        win_store(w, off, (uint32_t)v[0]);
-        win_store(w, off + orow, (uint32_t)v[1]);
-        win_store(w, off + 2 * orow, (uint32_t)v[2]);
+        win_store_aux<ST>(w, off, (uint32_t)v[0]);
+        win_store_aux<ST>(w, off + orow, (uint32_t)v[1]);
+        win_store_aux<ST>(w, off + 2 * orow, (uint32_t)v[2]);
     } else {
-        win_store(w, off, v);
+        __builtin_amdgcn_raw_buffer_store_b96(v, w, (int)off, 0, ST);
     }
 }
 
@@ -534,11 +535,12 @@ __device__ __forceinline__ void featurize16(const uint32_t (&Wa)[6], const uint3
     featurize16<T>(Wa, Wb, pe_t, pe_t2, f, fp);
 }
 
-template <typename T, int HL, bool PL = false, typename FT = T>
+template <typename T, int HL, bool PL = false, typename FT = T, bool RAG = false>
 __global__ __launch_bounds__(256) void mixer_se_fwd16_kernel(const T *__restrict__ raw, const T *__restrict__ wf,
                                                              const FT *__restrict__ h, T *__restrict__ y, Dims dm,
                                                              int kf, MixPlan pl)
 {
+    constexpr int LD = RAG ? 0 : WIN_NT, ST = RAG ? 0 : WIN_NT_ST;      // cache policy (ragged)
     constexpr int ES = 2, CH = 2, NH = HL - 1 + 3;
     int64_t wg = blockIdx.x;
     const int cvb = (int)(wg % pl.ncvb); wg /= pl.ncvb;
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(256) void mixer_se_fwd16_kernel(const T *__restrict
     const win_t wr = make_window(raw + 3 * (b * L + t0) * d, (t_end - t0) * irow);
     const win_t wy = make_window(y + (b * L + t_start) * d, (t_end - t_start) * orow);
     const uint32_t lane_o = (uint32_t)(c * ES), lane_i = PL ? lane_o : 3 * lane_o;
-    auto load_raw = [&](int64_t t) { return piece_load<PL>(wr, lane_i + (uint32_t)(t - t0) * irow, orow); };
+    auto load_raw = [&](int64_t t) { return piece_load<PL, LD>(wr, lane_i + (uint32_t)(t - t0) * irow, orow); };
 
     // pe[row & 3] = pair_rows(raw[row], raw[row - 1]); ur[row & 7] = u of the row
     uint32_t pe[4][6];
@@ -618,7 +620,7 @@ __global__ __launch_bounds__(256) void mixer_se_fwd16_kernel(const T *__restrict
                     for (int j = HL - 1; j >= 0; --j) acc = fmaf(hr[j], ur[(k - j) & 7][ch], acc);
                     out[ch] = f[ei<PL, CH>(ch, 0)] * acc;
                 }
-                win_store(wy, lane_o + (uint32_t)(tb + k - t_start) * orow, Pair<T>::pack2(out[0], out[1]));
+                win_store_aux<ST>(wy, lane_o + (uint32_t)(tb + k - t_start) * orow, Pair<T>::pack2(out[0], out[1]));
             }
         }
     }
@@ -626,12 +628,13 @@ __global__ __launch_bounds__(256) void mixer_se_fwd16_kernel(const T *__restrict
 
 // The backward walk above with the featurizer's three sums done two taps (or two rows) at a time.
 // d raw lags d f by three rows whatever the filter length (the fourth tap is zero for shorter filters).
-template <typename T, int HL, int KF, bool PL = false, typename FT = T>
+template <typename T, int HL, int KF, bool PL = false, typename FT = T, bool RAG = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MIXER_WPE)))
 void mixer_se_bwd16_kernel(const T *__restrict__ dy, const T *__restrict__ raw, const T *__restrict__ wf,
                            const FT *__restrict__ h, T *__restrict__ draw, float *__restrict__ ws_h,
                            float *__restrict__ ws_w, Dims dm, int kf, MixPlan pl)
 {
+    constexpr int LD = RAG ? 0 : WIN_NT, ST = RAG ? 0 : WIN_NT_ST;      // cache policy (ragged)
     typedef Piece<T> P;
     constexpr int ES = 2, CH = 2, E = 6, D1 = HL - 1, D2 = 3, NH = D1 + D2;
     int64_t wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
@@ -686,7 +689,7 @@ void mixer_se_bwd16_kernel(const T *__restrict__ dy, const T *__restrict__ raw, 
     {
         u32x3 hp[NH];
 #pragma unroll
-        for (int i = 1; i <= NH; ++i) hp[i - 1] = piece_load<PL>(wr, lane_i + (uint32_t)(t_start - i - t0) * irow, orow);
+        for (int i = 1; i <= NH; ++i) hp[i - 1] = piece_load<PL, LD>(wr, lane_i + (uint32_t)(t_start - i - t0) * irow, orow);
 #pragma unroll
         for (int i = NH; i >= 1; --i) {
             rp[(-i) & 15] = hp[i - 1];
@@ -715,8 +718,8 @@ void mixer_se_bwd16_kernel(const T *__restrict__ dy, const T *__restrict__ raw, 
     auto fetch = [&](int slot) {
 #pragma unroll
         for (int kk = 0; kk < BATCH16; ++kk) {
-            in[slot][kk] = piece_load<PL>(wr, vin, orow);     // zero past t_far
-            dyr[slot][kk] = win_load<uint32_t>(wdy, vdy);
+            in[slot][kk] = piece_load<PL, LD>(wr, vin, orow);     // zero past t_far
+            dyr[slot][kk] = win_load_aux<LD, uint32_t>(wdy, vdy);
             vin += irow;
             vdy += orow;
         }
@@ -797,7 +800,7 @@ void mixer_se_bwd16_kernel(const T *__restrict__ dy, const T *__restrict__ raw, 
 #pragma unroll
             for (int e = 0; e < E; ++e)
                 dr[e] = Pair<T>::dot2(pd[(k1 - 2) & 3][e], Wa[e], Pair<T>::dot2(pd[k1 & 3][e], Wb[e], 0.f));
-            piece_store<PL>(wdr, vout, orow, pack6<T>(dr));
+            piece_store<PL, ST>(wdr, vout, orow, pack6<T>(dr));
             vout += irow;
         }
     };
@@ -840,7 +843,7 @@ MixPlan plan(const Dims &dm, int ch, bool backward)
     // Long runs keep the halo of up to 10 rows each side and the filter-gradient partials small (9 % of the traffic at 128
     // rows, 4 % at 512).  The backward gains nothing beyond 512 rows; the forward does (40B shape: 409 us at 512 rows, 383 at
     // 1024).  Multiples of 16 (the backward's longest ring).
-    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, 16, backward ? 512 : 1024, 9, 1.1, INT64_MAX);
+    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, 16, backward ? 512 : 1024, 9, 1.1, INT64_MAX, false);
     p.ts = r.ts;
     static const char *env = tuning_env("GCG_MIXER_ROWS");      // tuning override: rows per lane, a multiple of 16
     if (env && atoi(env) >= 16 && atoi(env) % 16 == 0) p.ts = atoi(env);
@@ -855,6 +858,11 @@ MixPlan plan(const Dims &dm, int ch, bool backward)
 
 int lane_channels(int dtype) { return dtype == GCG_F32 ? 1 : 2; }
 
+// 16-bit rows that start and end on odd 32-byte sectors are accessed without the streaming hint: the parts of a shared 64 bytes
+// then meet in the L2 instead of being written one by one (3 x 17810 x 2512: forward 265 -> 239 us and 297 -> 247 planar,
+// backward 438 -> 423 and 531 -> 451; rows of whole or half lines are as fast or faster with it).
+bool ragged(const Dims &dm) { return (uint64_t)dm.d * 2 % 64 != 0; }
+
 // FT: element type of h and dh (float with 16-bit T: fp32 filter and arithmetic on 16-bit tensors)
 template <typename T, int HL, int KF, typename FT>
 int fwd_launch(const void *raw, const void *wf, const void *h, void *y, const Dims &dm, int kf, hipStream_t st)
@@ -864,10 +872,10 @@ int fwd_launch(const void *raw, const void *wf, const void *h, void *y, const Di
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if constexpr (sizeof(T) == 2) {
         if (dm.planar)
-            e = launch_plain((mixer_se_fwd16_kernel<T, HL, true, FT>), dim3((unsigned)p.nwg), dim3(p.threads), st,
+            e = launch_plain(ragged(dm) ? mixer_se_fwd16_kernel<T, HL, true, FT, true> : mixer_se_fwd16_kernel<T, HL, true, FT>, dim3((unsigned)p.nwg), dim3(p.threads), st,
                              (const T *)raw, (const T *)wf, (const FT *)h, (T *)y, dm, kf, p);
         else
-            e = launch_plain((mixer_se_fwd16_kernel<T, HL, false, FT>), dim3((unsigned)p.nwg), dim3(p.threads), st,
+            e = launch_plain(ragged(dm) ? mixer_se_fwd16_kernel<T, HL, false, FT, true> : mixer_se_fwd16_kernel<T, HL, false, FT>, dim3((unsigned)p.nwg), dim3(p.threads), st,
                              (const T *)raw, (const T *)wf, (const FT *)h, (T *)y, dm, kf, p);
     } else {
         if (dm.planar)
@@ -891,10 +899,10 @@ int bwd_launch(const void *dy, const void *raw, const void *wf, const void *h, v
     float *ws_w = ws_h + (size_t)dm.hl * p.nrows * p.nvec;
     if constexpr (sizeof(T) == 2) {
         if (dm.planar)
-            e = launch_plain((mixer_se_bwd16_kernel<T, HL, KF, true, FT>), dim3((unsigned)p.nwg), dim3(p.threads), st,
+            e = launch_plain(ragged(dm) ? mixer_se_bwd16_kernel<T, HL, KF, true, FT, true> : mixer_se_bwd16_kernel<T, HL, KF, true, FT>, dim3((unsigned)p.nwg), dim3(p.threads), st,
                              (const T *)dy, (const T *)raw, (const T *)wf, (const FT *)h, (T *)draw, ws_h, ws_w, dm, kf, p);
         else
-            e = launch_plain((mixer_se_bwd16_kernel<T, HL, KF, false, FT>), dim3((unsigned)p.nwg), dim3(p.threads), st,
+            e = launch_plain(ragged(dm) ? mixer_se_bwd16_kernel<T, HL, KF, false, FT, true> : mixer_se_bwd16_kernel<T, HL, KF, false, FT>, dim3((unsigned)p.nwg), dim3(p.threads), st,
                              (const T *)dy, (const T *)raw, (const T *)wf, (const FT *)h, (T *)draw, ws_h, ws_w, dm, kf, p);
     } else {
         if (dm.planar)

@@ -114,7 +114,8 @@ template <typename T, int VV> __device__ __forceinline__ typename Vec<T, VV>::ra
 // How a walk kernel cuts (bs, L) rows of nvec lane vectors into workgroups of `waves` waves (64 lanes each, ncvb of them
 // side by side) and runs of ts rows.  The waves that the fullest SIMD gets, together or one after the other, times the rows a
 // wave walks -- its run and `extra` rows of halo and set-up -- is what a launch takes, so the plan is the smallest such
-// product over the 256 CUs of four SIMDs, times `alone` for one wave per SIMD, which waits for its rows alone.
+// product over the 256 CUs of four SIMDs (streams: the kernel waits for memory, and three waves on four SIMDs count as that;
+// 8192 x 16 x 768 time-major, backward, 1.5 waves of 256 rows 293 us, 3 of 128 302), times `alone` for one wave per SIMD, which waits for its rows alone.
 // Runs are multiples of `unit` and at most `longest` rows; workgroups of four waves unless fewer leave less idle.  No more than
 // most_lanes lanes have work, unless even the longest runs need more (lanes leave partial sums behind).
 // (Against runs of a power of two that fill two workgroups per CU at least: mixer 3 x 17810 x 2512 bf16 backward 545 -> 435 us,
@@ -122,7 +123,7 @@ template <typename T, int VV> __device__ __forceinline__ typename Vec<T, VV>::ra
 // 3 x 20000 x 800 fp32 291 -> 255, 4 x 7000 x 2400 f16 240 -> 211; widths that are powers of two keep their plans.)
 struct RunPlan { int waves, ncvb, ts; };
 inline RunPlan plan_runs(int64_t bs, int64_t L, int64_t nvec, int unit, int longest, int extra, double alone,
-                         int64_t most_lanes)
+                         int64_t most_lanes, bool streams)
 {
     RunPlan best{0, 0, 0};
     double least = 0;
@@ -136,8 +137,9 @@ inline RunPlan plan_runs(int64_t bs, int64_t L, int64_t nvec, int unit, int long
             const int64_t ts = ((L + nseg - 1) / nseg + unit - 1) / unit * unit;
             const int64_t runs = (L + ts - 1) / ts;
             if (ts > longest || bs * runs * nvec > most_lanes) continue;
-            const int64_t per_cu = (per * runs + 255) / 256, per_simd = (per_cu * k + 3) / 4;
-            const double cost = (double)per_simd * (double)(ts + extra) * (per_simd == 1 ? alone : 1.0);
+            const int64_t per_cu = (per * runs + 255) / 256;
+            const double per_simd = k == 3 && streams ? 0.75 * (double)per_cu : (double)((per_cu * k + 3) / 4);
+            const double cost = per_simd * (double)(ts + extra) * (per_simd <= 1 ? alone : 1.0);
             if (best.waves == 0 || cost < least * (k == best.waves ? 1.0 : 0.97)) { best = RunPlan{k, (int)ncvb, (int)ts}; least = cost; }
             if (ts == unit) break;
         }

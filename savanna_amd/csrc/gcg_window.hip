@@ -395,7 +395,7 @@ WinPlan plan(const Dims &dm, int v, int longest, int64_t most_lanes)
     WinPlan p;
     p.v = v;
     p.nvec = (int)(dm.d / v);
-    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, 1.3, most_lanes);
+    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, 1.3, most_lanes, true);
     p.ts = r.ts;
     static const char *env = tuning_env("GCG_WINDOW_ROWS");   // tuning override: rows per lane, a multiple of 8
     if (env && atoi(env) >= 8 && atoi(env) % 8 == 0) p.ts = atoi(env);
@@ -422,13 +422,13 @@ template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
 // workgroups (1 x 32768 x 8192 bf16 377 us; short runs in XCD order 411).  Other whole lines: runs of at most 128 rows in
 // XCD-contiguous order (1 x 399457 x 1344 1032 -> 840 us, 1 x 38836 x 3456 227 -> 214).  Rows off the lines: plain accesses,
 // so that the parts of a shared line meet in the L2, and at most 64 rows (1 x 264208 x 2032 1415 -> 865 us, 1 x 46091 x 2912
-// 262 -> 217; with streaming accesses 925 and 225).
+// 262 -> 217; with streaming accesses 925 and 225).  Time-major 8192 x 16 x 768: 164 -> 156 us with that order.
 struct FwdForm { int longest; bool rag, xcd; };
 FwdForm fwd_form(const Dims &dm, size_t es)
 {
     const uint64_t row = (uint64_t)dm.d * es;
     const bool rag = row % 128 != 0, wide = row % 8192 == 0;
-    return FwdForm{wide ? 1024 : rag ? 64 : 128, rag, !wide && !dm.tmajor};
+    return FwdForm{wide ? 1024 : rag ? 64 : 128, rag, !wide};
 }
 
 template <typename T, int HL, int V>
