@@ -4,6 +4,8 @@
 #pragma once
 #include "gcg_mfma_tile.h"
 
+#include <type_traits>
+
 namespace gcg {
 namespace {
 
@@ -115,18 +117,74 @@ template <typename T, int NR> __device__ __forceinline__ Row<T> units_row(const 
 // it back.  A lane then owns NR consecutive rows of a step instead of rows RP apart, and also fetches the
 // KF-1 rows before them: rows its neighbours own and request at the same time, so they cost cache hits, not
 // memory traffic.
-// tap[m][v]: what feature channel f0 + v multiplies the row KF-1-m rows in the past with (zero where kf < KF)
-template <typename T, int KF, int NV>
-__device__ __forceinline__ void load_feat_taps(const T *wfeat, int64_t f0, int kf, float (&tap)[KF][NV])
+// A lane's taps: tap[m][v] is what its feature value v multiplies the row KF-1-m rows in the past with (zero where
+// kf < KF).  They are 36 bytes of wfeat, or 12 of each of its planes (PL): requested as three accesses before the rows and
+// converted once those are requested too -- as 18 elements loaded and converted one by one, with the rows requested after
+// the last conversion, they put a memory latency in front of every launch (mixer forward of 1 x 24 x 2544: 14.4 us of kernel).
+// (f16 tensors load and convert element by element: there the compiler folds conversions into the featurizer's
+// multiply-adds, which rounds differently, and what it folds has to be alike in the kernels of either layout.)
+template <typename T, int KF, int NV> struct FeatTaps {
+    static constexpr bool BY_WORD = !std::is_same_v<T, f16_t> && !std::is_same_v<T, f16w_t>;
+    uint32_t w[9];
+    float t[KF][NV];
+};
+// c: the lane's first channel
+template <typename T, int KF, int NV, bool PL = false>
+__device__ __forceinline__ FeatTaps<T, KF, NV> request_feat_taps(const T *wfeat, int64_t c, bool valid, int64_t d, int kf)
 {
+    constexpr int ES = sizeof(T);
+    static_assert(NV * KF * ES == 36 && (!PL || ES == 2), "a lane's taps are nine words");
+    FeatTaps<T, KF, NV> r;
+    auto element = [&](int v, int m) {
+        const int kk = m - (KF - kf);                                    // index into the kf taps of the filter
+        const int64_t f = !valid ? 0 : PL ? (int64_t)(v / 2) * d + c + v % 2 : 3 * c + v;
+        return wfeat + f * kf + (kk >= 0 ? kk : 0);
+    };
+    if constexpr (!FeatTaps<T, KF, NV>::BY_WORD) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v)
+        for (int v = 0; v < NV; ++v)
 #pragma unroll
-        for (int m = 0; m < KF; ++m) {
-            const int kk = m - (KF - kf);                // index into the kf taps of the filter
-            const float t = Elem<T>::load(wfeat + (f0 + v) * kf + (kk >= 0 ? kk : 0));
-            tap[m][v] = kk >= 0 ? t : 0.f;
+            for (int m = 0; m < KF; ++m) {
+                const float t = Elem<T>::load(element(v, m));
+                r.t[m][v] = m - (KF - kf) >= 0 ? t : 0.f;
+            }
+    } else if (kf == KF && ((uintptr_t)wfeat & 3) == 0) {
+        const win_t win = make_window(wfeat, 3 * d * KF * ES);
+        const uint32_t off = (uint32_t)((PL ? c : 3 * c) * KF * ES) + (valid ? 0u : WIN_OFF);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const u32x3 t = __builtin_amdgcn_raw_buffer_load_b96(win, (int)(off + (PL ? (uint32_t)(p * d * KF * ES) : 12u * p)), 0, 0);
+            r.w[3 * p] = t[0]; r.w[3 * p + 1] = t[1]; r.w[3 * p + 2] = t[2];
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) r.w[i] = 0u;
+#pragma unroll
+        for (int i = 0; i < NV * KF; ++i) {
+            uint32_t bits = 0u;
+            __builtin_memcpy(&bits, element(i / KF, i % KF), ES);
+            r.w[i * ES / 4] |= (i % KF - (KF - kf) >= 0 ? bits : 0u) << (8 * (i * ES % 4));
+        }
+    }
+    return r;
+}
+template <typename T, int KF, int NV>
+__device__ __forceinline__ void feat_taps(const FeatTaps<T, KF, NV> &r, float (&tap)[KF][NV])
+{
+    if constexpr (FeatTaps<T, KF, NV>::BY_WORD) {
+        if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);     // after the requests above (fp32: nothing to convert)
+#pragma unroll
+        for (int i = 0; i < NV * KF; ++i) {
+            T t;
+            __builtin_memcpy(&t, (const char *)r.w + i * sizeof(T), sizeof(T));
+            tap[i % KF][i / KF] = Elem<T>::load(&t);
+        }
+    } else {
+#pragma unroll
+        for (int m = 0; m < KF; ++m)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) tap[m][v] = r.t[m][v];
+    }
 }
 // (C, B, x) of a lane's NR rows from the KF-1 + NR fetched pieces of the projection output, oldest row first;
 // sums in the featurizer kernel's order (oldest sample first, fp32) and rounded to T like its output

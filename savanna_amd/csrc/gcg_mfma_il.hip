@@ -105,7 +105,8 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_fwd_kernel(const T *__restric
         for (int k = 0; k < NR; ++k) store_operand_unit<T>(u_wr + KS * k * UROW, UROW, &uf[CH * k]);
     };
     float tap[FEAT ? KF : 1][NV];
-    if constexpr (FEAT) load_feat_taps<T, KF, NV>(wfeat, cvalid ? 3 * (c0 + CH * a) : 0, kf, tap);
+    FeatTaps<T, FEAT ? KF : 1, NV> tap_words;
+    if constexpr (FEAT) tap_words = request_feat_taps<T, KF, NV>(wfeat, c0 + CH * a, cvalid, d, kf);
     // (C, B, x) of the lane's rows from the fetched pieces
     auto rows_of = [&](const u32x3 (&p)[NH + NR], float (&xf)[8], float (&Bf)[8], float (&Cf)[8]) {
         if constexpr (FEAT) featurized_rows<T, NR, KF>(p, tap, xf, Bf, Cf);
@@ -128,6 +129,7 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_fwd_kernel(const T *__restric
     }
     u32x3 in[NH + NR];
     fetch(3 * step_off(s_lo), in);
+    if constexpr (FEAT) feat_taps<T, KF, NV>(tap_words, tap);
 
     store_taps(htab[w], l, hv);
     __syncthreads();
@@ -138,7 +140,9 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_fwd_kernel(const T *__restric
         W1[i] = M::toeplitz(htab[w], 32 * i + 16, j, q);
     }
 
-    if constexpr (NK > 1) {
+    // (before the sequence there is nothing to rebuild; three-plane operands leave no registers for a choice)
+    constexpr bool THREE_PLANES = std::is_same_v<T, float> || std::is_same_v<T, f16w_t>;
+    if (NK > 1 && (THREE_PLANES || s_lo > 0)) {
 #pragma unroll
         for (int i = 1; i < NK; ++i) {
             float xf[8], Bf[8], Cf[8], uf[8];
@@ -163,14 +167,21 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_fwd_kernel(const T *__restric
 #pragma unroll
         for (int ph = 0; ph < NK; ++ph) {
             if (s < n_steps) {
-                u32x3 nx[NH + NR];   // rows of the next step; past the segment they fall outside the window
-                fetch(so3 + step_b3, nx);
+                // rows of the next step (past the segment they fall outside the window); with the featurizer in fp32 once this
+                // step's have been taken up, because two steps' rows do not fit the registers
+                constexpr bool LATE = FEAT && sizeof(T) == 4;
+                u32x3 nx[NH + NR];
+                if constexpr (!LATE) fetch(so3 + step_b3, nx);
 
                 float xf[8], Bf[8], Cf[8], uf[8];
                 rows_of(in, xf, Bf, Cf);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) uf[e] = xf[e] * Bf[e];
                 store_u(uf);
+                if constexpr (LATE) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch(so3 + step_b3, nx);
+                }
                 __syncthreads();
                 A[ph] = M::load_operand(u_rm, UROW, w, j, q, false);
                 {
@@ -326,7 +337,8 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_bwd_kernel(const T *__restric
         for (int k = 0; k < NH + NR; ++k) p[k] = ldw12(wf, feat_off3 + (so3 + (uint32_t)(k - NH) * pass_off3));
     };
     float tap[FEAT ? KF : 1][NV];
-    if constexpr (FEAT) load_feat_taps<T, KF, NV>(wfeat, cvalid ? 3 * (c0 + CH * a) : 0, kf, tap);
+    FeatTaps<T, FEAT ? KF : 1, NV> tap_words;
+    if constexpr (FEAT) tap_words = request_feat_taps<T, KF, NV>(wfeat, c0 + CH * a, cvalid, d, kf);
     // x, B, C of the lane's rows from the fetched pieces
     auto rows_of = [&](const u32x3 (&p)[NH + NR], float (&xo)[8], float (&Bo)[8], float (&Co)[8]) {
         if constexpr (FEAT) featurized_rows<T, NR, KF>(p, tap, xo, Bo, Co);
@@ -368,6 +380,7 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_bwd_kernel(const T *__restric
     }
     fetch_feat(3 * step_off(s_lo + NK - 1), in);
     fetch_dy(step_off(s_lo + NK - 1), dyr);
+    if constexpr (FEAT) feat_taps<T, KF, NV>(tap_words, tap);
 
     store_taps(htab + w * HTAB, l, hv);
     __syncthreads();
@@ -628,7 +641,8 @@ __global__ __launch_bounds__(512) void mfma_il_bwd_duo_kernel(const T *__restric
             r.dy = units_row<T, NR>(u);
         };
         float tap[FEAT ? KF : 1][NV];
-        if constexpr (FEAT) load_feat_taps<T, KF, NV>(wfeat, cvalid ? 3 * (c0 + CH * a) : 0, kf, tap);
+        FeatTaps<T, FEAT ? KF : 1, NV> tap_words;
+        if constexpr (FEAT) tap_words = request_feat_taps<T, KF, NV>(wfeat, c0 + CH * a, cvalid, d, kf);
         auto rows_of = [&](const u32x3 (&p)[NH + NR], float (&xo)[8], float (&Bo)[8], float (&Co)[8]) {
             if constexpr (FEAT) featurized_rows<T, NR, KF>(p, tap, xo, Bo, Co);
             else il_split<T, NR>(p, xo, Bo, Co);
@@ -696,6 +710,7 @@ __global__ __launch_bounds__(512) void mfma_il_bwd_duo_kernel(const T *__restric
             for (int jj = NK - 2; jj >= 0; --jj) fetch(step_off(s_lo + jj), 3 * step_off(s_lo + jj), lead[jj]);
             fetch(step_off(s_lo + NK - 1), 3 * step_off(s_lo + NK - 1), lead[NK - 1]);
             fetch(step_off(s_lo + NK), 3 * step_off(s_lo + NK), st[1]);
+            if constexpr (FEAT) feat_taps<T, KF, NV>(tap_words, tap);
             __syncthreads();                                          // (A)
             __syncthreads();                                          // (A2): the filter tables' place is free
             float f0[8], f1[8], f2[8];

@@ -115,26 +115,6 @@ template <bool PL> __device__ __forceinline__ void piece_store(win_t w, uint32_t
         stw12(w, off, v);
     }
 }
-// taps of a lane's six feature channels, oldest sample first, zero-padded in front to KF taps
-template <typename T, int KF, bool PL>
-__device__ __forceinline__ void lane_feat_taps(const T *wfeat, int64_t c, bool valid, int64_t d, int kf, float (&tap)[KF][6])
-{
-    if constexpr (PL) {
-#pragma unroll
-        for (int v = 0; v < 6; ++v) {
-            const T *wp = wfeat + (valid ? feature_channel<true>(c, v, d) : 0) * kf;
-#pragma unroll
-            for (int m = 0; m < KF; ++m) {
-                const int kk = m - (KF - kf);                // index into the kf taps of the filter
-                const float t = Elem<T>::load(wp + (kk >= 0 ? kk : 0));
-                tap[m][v] = kk >= 0 ? t : 0.f;
-            }
-        }
-    } else {
-        load_feat_taps<T, KF, 6>(wfeat, valid ? 3 * c : 0, kf, tap);
-    }
-}
-
 struct Blk { uint4 w[3]; };       // four 12-byte pieces
 struct Halo { uint2 w[3]; };      // two 12-byte pieces
 
@@ -319,11 +299,10 @@ __global__ __launch_bounds__(MixGeo<T>::NT) void mixer_mr_bwd_kernel(const T *__
     unsigned char *raw_rg = smem + G::OFF_RAW, *df_rg = smem + G::OFF_DF;
     hraw_t *htab = (hraw_t *)(smem + G::OFF_H);
 
-    const int64_t wg_id = xcd_contiguous_id(blockIdx.x, gridDim.x);
-    int64_t wg = wg_id;
-    const int cb = (int)(wg % pl.ncb); wg /= pl.ncb;
-    const int seg = (int)(wg % pl.nseg);
-    const int64_t b = wg / pl.nseg;
+    const uint32_t wg_id = xcd_contiguous_u32(blockIdx.x, gridDim.x);
+    int cb, seg, bi;
+    wg_place(wg_id, pl, cb, seg, bi);
+    const int64_t b = bi;
 
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
     const bool is_m = w < MW;
@@ -350,7 +329,7 @@ __global__ __launch_bounds__(MixGeo<T>::NT) void mixer_mr_bwd_kernel(const T *__
                                  : 3u * ((uint32_t)(NR * rr - NH) * rb + col_b) + bad;     // row NR*rr-NH of a step
     auto step_base = [&](int64_t step, int64_t origin) { return (uint32_t)((step * STEP - origin) * row_bytes); };
     float tap[KF][NV];
-    lane_feat_taps<T, KF, PL>(wfeat, c0 + 2 * a, cvalid, d, kf, tap);
+    const auto tap_words = request_feat_taps<T, KF, NV, PL>(wfeat, c0 + 2 * a, cvalid, d, kf);
     const int own_off = (rr * LPR + a) * G::BLK;                                   // own rows in a slot
     const int halo_off = rr ? ((rr - 1) * LPR + a) * G::BLK + 24 : G::PRE + a * 24;    // the NH rows before them
 
@@ -359,8 +338,9 @@ __global__ __launch_bounds__(MixGeo<T>::NT) void mixer_mr_bwd_kernel(const T *__
         const int xw = w - MW, j = l & 15, q = l >> 4;
         const bool wave_valid = c0 + 16 * xw < d;
         hraw_t hv[HTAB / 64];
-        load_taps<T>(dm, h, wave_valid ? (c0 + 16 * xw) / dm.dg : 0, l, hv);
+        load_taps<T>(dm, h, wave_valid ? fdiv((uint32_t)(cb * XW + xw), pl.q_dg16) : 0, l, hv);
         store_taps(htab + xw * HTAB, l, hv);
+        feat_taps<T, KF, NV>(tap_words, tap);
         __syncthreads();
         typename M::wop_t W0[NK], W1[NK];
 #pragma unroll
@@ -566,6 +546,7 @@ __global__ __launch_bounds__(MixGeo<T>::NT) void mixer_mr_bwd_kernel(const T *__
         fetch(in1, raw_b, dy_b);
         raw_b += step_b;
         dy_b += step_b;
+        feat_taps<T, KF, NV>(tap_words, tap);
 #pragma unroll
         for (int i = 0; i < NK; ++i) arrive(lead[i], i * G::SLOT);
     }
@@ -834,7 +815,7 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
     const int64_t T0 = s_lo * STEP, T1 = s_hi * STEP < L ? s_hi * STEP : L;
     const uint32_t lane_raw = 3u * ((uint32_t)(NR * rr - NH) * rb + (uint32_t)((c0 + 2 * a) * 2)) + bad;  // row NR*rr-NH of a step
     float tap[KF][NV];
-    load_feat_taps<T, KF, NV>(wfeat, cvalid ? 3 * (c0 + 2 * a) : 0, kf, tap);
+    const auto tap_words = request_feat_taps<T, KF, NV>(wfeat, c0 + 2 * a, cvalid, d, kf);
     const int own_off = vt * G::BLK;
     const int j = l & 15, q = l >> 4;
 
@@ -852,6 +833,7 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
         const int y_wr = j * YROW + (16 * w + 4 * q) * 4;
         const int d_wr = (15 - j) * YROW + (16 * w + 4 * q) * 4;      // columns come out reversed
         store_taps(htab + w * HTAB, l, hv);
+        feat_taps<T, KF, NV>(tap_words, tap);
         __syncthreads();                                              // (A)
         M::wop_t W0[NK], W1[NK];
 #pragma unroll
@@ -1078,6 +1060,7 @@ __global__ __launch_bounds__(WideGeo::NT) void mixer_mr_bwd_wide_kernel(
             fetch_c(raw_0 + (uint32_t)(NK - 1) * step_b3, dy_0 + (uint32_t)(NK - 1) * step_b, lead[NK - 1]);
             fetch_raw(raw_0, first);
             fetch_c(raw_0 + (uint32_t)NK * step_b3, dy_0 + (uint32_t)NK * step_b, st[1]);
+            feat_taps<T, KF, NV>(tap_words, tap);
             __syncthreads();                                          // (A)
             __syncthreads();                                          // (A2): the filter tables' place is free
 #pragma unroll
@@ -1262,23 +1245,23 @@ __global__ __launch_bounds__(MixFwdGeo<T>::NT) void mixer_mr_fwd_kernel(const T 
     unsigned char *u_rm = smem + G::OFF_U, *y_st = smem + G::OFF_Y;
     hraw_t *htab = (hraw_t *)(smem + G::OFF_H);
 
-    const int64_t wg_id = xcd_contiguous_id(blockIdx.x, gridDim.x);
-    int64_t wg = wg_id;
-    const int cb = (int)(wg % pl.ncb); wg /= pl.ncb;
-    const int seg = (int)(wg % pl.nseg);
-    const int64_t b = wg / pl.nseg;
+    const uint32_t wg_id = xcd_contiguous_u32(blockIdx.x, gridDim.x);
+    int cb, seg, bi;
+    wg_place(wg_id, pl, cb, seg, bi);
+    const int64_t b = bi;
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
     const int64_t d = dm.d, L = dm.L;
     const int64_t c0 = (int64_t)cb * CB;
     const int64_t s_lo = (int64_t)seg * pl.steps_per_seg;
     const int64_t s_hi = (s_lo + pl.steps_per_seg < pl.nsteps) ? s_lo + pl.steps_per_seg : pl.nsteps;
-    const int64_t k_first = s_lo - (NK - 1);                    // u of the NK-1 steps before the run is made again
+    // u of the NK-1 steps before the run is made again (those of the sequence: nothing before it)
+    const int64_t k_first = s_lo > NK - 1 ? s_lo - (NK - 1) : 0;
 
     if (w >= MW) {
         // ------------------------------------------------------------------ matrix waves
         const int xw = w - MW, j = l & 15, q = l >> 4;
         hraw_t hv[HTAB / 64];
-        load_taps<T>(dm, h, (c0 + 16 * xw < d) ? (c0 + 16 * xw) / dm.dg : 0, l, hv);
+        load_taps<T>(dm, h, (c0 + 16 * xw < d) ? fdiv((uint32_t)(cb * G::XW + xw), pl.q_dg16) : 0, l, hv);
         store_taps(htab + xw * HTAB, l, hv);
         __syncthreads();
         typename M::wop_t W0[NK], W1[NK];   // output rows 0..15 / 16..31 of the step against input step k-i
@@ -1335,7 +1318,7 @@ __global__ __launch_bounds__(MixFwdGeo<T>::NT) void mixer_mr_fwd_kernel(const T 
     const uint32_t lane_y = (uint32_t)(NR * rr) * rb + col_b + bad;                     // row NR*rr
     auto step_base = [&](int64_t step, int64_t origin) { return (uint32_t)((step * STEP - origin) * row_bytes); };
     float tap[KF][NV];
-    lane_feat_taps<T, KF, PL>(wfeat, c0 + 2 * a, cvalid, d, kf, tap);
+    const auto tap_words = request_feat_taps<T, KF, NV, PL>(wfeat, c0 + 2 * a, cvalid, d, kf);
     unsigned char *u_own = u_rm + NR * rr * UROW + 4 * a;
     const unsigned char *y_rd = y_st + NR * rr * YROW + 8 * a;
 
@@ -1369,6 +1352,7 @@ __global__ __launch_bounds__(MixFwdGeo<T>::NT) void mixer_mr_fwd_kernel(const T 
     raw_b += step_b;
     fetch(in1, raw_b);
     raw_b += step_b;
+    feat_taps<T, KF, NV>(tap_words, tap);
     __syncthreads();
     __syncthreads();
     arrive(in0);                                     // step k_first
