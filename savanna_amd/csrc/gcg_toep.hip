@@ -166,18 +166,22 @@ __device__ __forceinline__ void ring_store(uint16_t *ring, int cl, int pos, cons
 {
     typedef Reach<NK> G;
     constexpr int NPA = GT<T>::NPA;
-    uint16_t v[NPA][8];
+    uint32_t v[NPA][4];                          // (two samples a conversion: split_planes of each)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        uint16_t o[NPA];
-        split_planes<NPA>(f[e] * LIFT<T>, o);
+    for (int e = 0; e < 4; ++e) {
+        float r0 = f[2 * e] * LIFT<T>, r1 = f[2 * e + 1] * LIFT<T>;
 #pragma unroll
-        for (int m = 0; m < NPA; ++m) v[m][e] = o[m];
+        for (int m = 0; m < NPA; ++m) {
+            v[m][e] = pack_bf16x2(r0, r1);
+            if (m + 1 < NPA) {
+                r0 -= __uint_as_float(v[m][e] << 16);
+                r1 -= __uint_as_float(v[m][e] & 0xffff0000u);
+            }
+        }
     }
 #pragma unroll
     for (int m = 0; m < NPA; ++m) {
-        uint4 t;
-        __builtin_memcpy(&t, v[m], 16);
+        const uint4 t = make_uint4(v[m][0], v[m][1], v[m][2], v[m][3]);
         uint16_t *row = ring + (m * CB + cl) * G::RP;
         *(uint4 *)(row + pos) = t;
         if (pos == 0) *(uint4 *)(row + G::R) = t;
@@ -326,24 +330,25 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
         ring_store<T, NK, CB>(ring, cl, 8 * g, u);
     }
     uint32_t rx[8], rB[8], rC[8];
-    uint32_t row = (uint32_t)(T0 - tw) + 8 * tg;                          // first row of the thread, from tw
+    // offsets of the thread's first row, running (as products each access costs a multiplication at a quarter of the rate)
+    uint32_t oi = ((uint32_t)(T0 - tw) + 8 * tg) * ri + ci, oo = ((uint32_t)(T0 - tw) + 8 * tg) * ro + co;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const uint32_t off = (row + e) * ri + ci;
+        const uint32_t off = oi + e * ri;
         rx[e] = ld_raw<T>(wx, off); rB[e] = ld_raw<T>(wB, off); rC[e] = ld_raw<T>(wC, off);
     }
-    for (int64_t t0 = T0; t0 < T1; t0 += TT, row += TT) {
+    for (int64_t t0 = T0; t0 < T1; t0 += TT, oi += TT * ri, oo += TT * ro) {
         float u[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) u[e] = raw_float<T>(rx[e]) * raw_float<T>(rB[e]);
         ring_store<T, NK, CB>(ring, cl, wrap<G::R>(oldest + G::OFF + 8 * tg), u);
         if (bx)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) st_elem<T>(wbx, (row + e) * ro + co, u[e]);
+            for (int e = 0; e < 8; ++e) st_elem<T>(wbx, oo + e * ro, u[e]);
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < 8; ++e) {                                     // next tile; past the run the window ends
-            const uint32_t off = (row + TT + e) * ri + ci;
+            const uint32_t off = oi + (TT + e) * ri;
             rx[e] = ld_raw<T>(wx, off); rB[e] = ld_raw<T>(wB, off);
         }
         f32x4 acc[2];
@@ -357,12 +362,12 @@ __global__ __launch_bounds__(32 * CB) void toep_fwd_kernel(const T *__restrict__
         if (!all_finite(v)) *flag = 1;
         if (y2)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) st_elem<T>(wy2, (row + e) * ro + co, v[e]);
+            for (int e = 0; e < 8; ++e) st_elem<T>(wy2, oo + e * ro, v[e]);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const float cv = raw_float<T>(rC[e]);
-            rC[e] = ld_raw<T>(wC, (row + TT + e) * ri + ci);
-            st_elem<T>(wy, (row + e) * ro + co, cv * v[e]);
+            rC[e] = ld_raw<T>(wC, oi + (TT + e) * ri);
+            st_elem<T>(wy, oo + e * ro, cv * v[e]);
         }
         oldest = wrap<G::R>(oldest + TT);
     }
@@ -451,18 +456,17 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         ring_store<T, NK, CB>(rg, cl, 8 * g, v);
     }
     uint32_t rx[8], rB[8], rl[8], rC[8], rd[8];                           // rl, rC: dy and C of the look-ahead; rd: dy of the tile
-    uint32_t row = (uint32_t)(T0 - tw) + 8 * tg;
+    uint32_t oi = ((uint32_t)(T0 - tw) + 8 * tg) * ri + ci, oo = ((uint32_t)(T0 - tw) + 8 * tg) * ro + co;   // (running: see the forward)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const uint32_t r = row + e, rr = r + G::OFF;
-        rx[e] = ld_raw<T>(wx, r * ri + ci); rB[e] = ld_raw<T>(wB, r * ri + ci);
-        rl[e] = ld_raw<T>(wdy, rr * ro + co); rC[e] = ld_raw<T>(wC, rr * ri + ci);
+        rx[e] = ld_raw<T>(wx, oi + e * ri); rB[e] = ld_raw<T>(wB, oi + e * ri);
+        rl[e] = ld_raw<T>(wdy, oo + (G::OFF + e) * ro); rC[e] = ld_raw<T>(wC, oi + (G::OFF + e) * ri);
     }
     f32x4 dh[2];
     dh[0] = dh[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
     const int n = lane & 15, q = lane >> 4;
     const int ga = min(n, (dm.hl - 1) >> 4) * 16;                         // row a of the filter-gradient tile, in samples
-    for (int64_t t0 = T0; t0 < T1; t0 += TT, row += TT) {
+    for (int64_t t0 = T0; t0 < T1; t0 += TT, oi += TT * ri, oo += TT * ro) {
         float u[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) u[e] = raw_float<T>(rx[e]) * raw_float<T>(rB[e]);
@@ -473,9 +477,8 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            rd[e] = ld_raw<T>(wdy, (row + e) * ro + co);
-            const uint32_t rr = row + TT + G::OFF + e;
-            rl[e] = ld_raw<T>(wdy, rr * ro + co); rC[e] = ld_raw<T>(wC, rr * ri + ci);
+            rd[e] = ld_raw<T>(wdy, oo + e * ro);
+            rl[e] = ld_raw<T>(wdy, oo + (TT + G::OFF + e) * ro); rC[e] = ld_raw<T>(wC, oi + (TT + G::OFF + e) * ri);
         }
         f32x4 acc[2];
         float v[8];
@@ -487,7 +490,7 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         *(f32x4 *)v = *(const f32x4 *)yr;
         *(f32x4 *)(v + 4) = *(const f32x4 *)(yr + 4);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) st_elem<T>(wdC, (row + e) * ri + ci, raw_float<T>(rd[e]) * v[e]);
+        for (int e = 0; e < 8; ++e) st_elem<T>(wdC, oi + e * ri, raw_float<T>(rd[e]) * v[e]);
         if (!all_finite(v)) *flag = 1;
         // filter gradient: 32 rows' products by themselves, added to the tile's sum and that to the run's; half of the
         // products with a negated operand (see the head of this file)
@@ -522,7 +525,7 @@ __global__ __launch_bounds__(32 * CB) void toep_bwd_kernel(const T *__restrict__
         *(f32x4 *)(v + 4) = *(const f32x4 *)(yr + 4);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const uint32_t o = (row + e) * ri + ci;
+            const uint32_t o = oi + e * ri;
             const float xv = raw_float<T>(rx[e]), bv = raw_float<T>(rB[e]);
             rx[e] = ld_raw<T>(wx, o + TT * ri); rB[e] = ld_raw<T>(wB, o + TT * ri);
             st_elem<T>(wdx, o, v[e] * bv);
