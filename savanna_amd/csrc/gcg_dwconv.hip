@@ -214,15 +214,17 @@ int lane_width(int dtype, const Dims &dm)
     return 4;
 }
 
-// Forward: the longest runs of a power of two up to 128 rows that give two workgroups per CU (the other plan: 119 against
-// 127 us at 1 x 12000 x 12288 bf16).  Backward: plan_runs (187 -> 178 us there, 12144 channels 219 -> 210).
-DwPlan plan(const Dims &dm, int V, bool backward)
+// Forward: the longest runs of a power of two that give two workgroups per CU (the other plan: 119 against 127 us at
+// 1 x 12000 x 12288 bf16), up to 128 rows where a row is a multiple of 8 KB (2 x 8192 x 12288 bf16 154 us, with 64 rows 165),
+// else 64, so that the rows in flight lie closer together (1 x 12000 x 12144 bf16 141 -> 134 us, 3 x 17810 x 7536 378 -> 366,
+// 1 x 6000 x 12192 fp32 127 -> 121).  Backward: plan_runs (187 -> 178 us there, 12144 channels 219 -> 210).
+DwPlan plan(const Dims &dm, int V, int longest, bool backward)
 {
     DwPlan p;
     p.v = V;
     p.nvec = (int)(dm.d / V);
-    RunPlan r{p.nvec >= 256 ? 4 : (p.nvec + 63) / 64, 0, 128};
-    if (backward) r = plan_runs(dm.bs, dm.L, p.nvec, RING, 128, RING, 1.3, INT64_MAX, true);
+    RunPlan r{p.nvec >= 256 ? 4 : (p.nvec + 63) / 64, 0, longest};
+    if (backward) r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, 1.3, INT64_MAX, true);
     else while (r.ts > 8 && dm.bs * ((dm.L + r.ts - 1) / r.ts) * p.nvec < 128 * 1024) r.ts >>= 1;
     p.ts = r.ts;
     static const char *env = tuning_env("GCG_DWCONV_ROWS");     // tuning override: rows per lane, a multiple of 8
@@ -245,7 +247,7 @@ template <typename T, int HL, int V, bool PCF>
 int fwd_launch(const void *x, const void *w, void *y, const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const DwPlan p = plan(dm, V, false);
+    const DwPlan p = plan(dm, V, (uint64_t)dm.d * sizeof(T) % 8192 == 0 ? 128 : 64, false);
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if (ragged<T>(dm))
         e = launch_plain((dwconv_fwd_kernel<T, HL, V, PCF, true, true>), dim3((unsigned)p.nwg), dim3(p.threads), st,
@@ -264,7 +266,7 @@ int bwd_launch(const void *dy, const void *x, const void *w, void *dx, void *dw,
                hipStream_t st)
 {
     int e = 0;
-    const DwPlan p = plan(dm, V, true);
+    const DwPlan p = plan(dm, V, 128, true);
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     e = launch_plain(ragged<T>(dm) ? dwconv_bwd_kernel<T, HL, V, PCF, true> : dwconv_bwd_kernel<T, HL, V, PCF>, dim3((unsigned)p.nwg), dim3(p.threads), st,
                        (const T *)dy, (const T *)x, (const T *)w, (T *)dx, (float *)ws, dm, p);
@@ -339,7 +341,7 @@ size_t dwconv_bwd_workspace(const Dims &dm)
     size_t n = 0;
     for (int v : {4, 8}) {
         if (dm.d % v) continue;
-        const DwPlan p = plan(dm, v, true);
+        const DwPlan p = plan(dm, v, 128, true);
         const int64_t nslot = dm.dg % v == 0 ? p.nvec : dm.d;
         const size_t need = (size_t)dm.hl * p.nrows * nslot * sizeof(float);
         if (need > n) n = need;

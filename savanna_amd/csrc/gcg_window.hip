@@ -420,15 +420,19 @@ template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
 
 // How the forward walks, by how its rows lie.  Rows of a multiple of 8 KB: long runs, streaming accesses, plain order of
 // workgroups (1 x 32768 x 8192 bf16 377 us; short runs in XCD order 411).  Other whole lines: runs of at most 128 rows in
-// XCD-contiguous order (1 x 399457 x 1344 1032 -> 840 us, 1 x 38836 x 3456 227 -> 214).  Rows off the lines: plain accesses,
-// so that the parts of a shared line meet in the L2, and at most 64 rows (1 x 264208 x 2032 1415 -> 865 us, 1 x 46091 x 2912
-// 262 -> 217; with streaming accesses 925 and 225).  Time-major 8192 x 16 x 768: 164 -> 156 us with that order.
+// XCD-contiguous order (1 x 399457 x 1344 1032 -> 840 us, 1 x 38836 x 3456 227 -> 214; 16 rows 902 and 204).  Rows off the
+// lines: plain accesses, so that the parts of a shared line meet in the L2, and 16 rows in plain order, so that the
+// neighbours of a line run at once (1 x 264208 x 2032 1415 -> 850 us, 1 x 64527 x 2080 224 -> 215, 1 x 46091 x 2912 262 ->
+// 210; 64 rows in XCD order 865, 250 and 227, streaming accesses 925 with those).  Interleaved 16-bit operands take that
+// form for whole lines too, their pieces being 12 bytes a lane (1 x 38836 x 3456 213 -> 197, 1 x 100000 x 1344 210 -> 199;
+// fp32 2 x 20000 x 2240 stays: 265, with 16 rows 268).  Time-major 8192 x 16 x 768: 164 -> 156 us in XCD order.
 struct FwdForm { int longest; bool rag, xcd; };
 FwdForm fwd_form(const Dims &dm, size_t es)
 {
     const uint64_t row = (uint64_t)dm.d * es;
-    const bool rag = row % 128 != 0, wide = row % 8192 == 0;
-    return FwdForm{wide ? 1024 : rag ? 64 : 128, rag, !wide};
+    if (row % 8192 == 0) return FwdForm{1024, false, false};
+    if (row % 128 != 0 || (dm.es == 3 && es == 2)) return FwdForm{16, true, false};
+    return FwdForm{128, false, true};
 }
 
 template <typename T, int HL, int V>
