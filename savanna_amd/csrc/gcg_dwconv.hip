@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void dwconv_fwd_kernel(const T *__restrict__ x
 // Backward: dx[t] = sum_j w[hl-1-j] dy[t+j] looks forward, so the walk runs HL-1 rows past the
 // run reading only dy; dw[hl-1-j] = sum_t dy[t] x[t-j] is accumulated per lane over the rows of
 // the run and reduced by a second kernel in a fixed order.
-template <typename T, int HL, int V, bool PCF, bool RAG = false>
+template <typename T, int HL, int V, bool PCF>
 __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                          const T *__restrict__ w, T *__restrict__ dx,
                                                          float *__restrict__ ws, Dims dm, DwPlan pl)
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ d
     {
         raw_t halo[HL - 1 > 0 ? HL - 1 : 1];
 #pragma unroll
-        for (int i = 1; i < HL; ++i) halo[i - 1] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wx, lane + (uint32_t)(t_start - i - t0) * row);
+        for (int i = 1; i < HL; ++i) halo[i - 1] = win_load<raw_t>(wx, lane + (uint32_t)(t_start - i - t0) * row);
 #pragma unroll
         for (int i = 1; i < HL; ++i) unpackv<T, V>(halo[i - 1], ur[RING - i]);
     }
@@ -156,8 +156,8 @@ __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ d
 #pragma unroll
             for (int kk = 0; kk < BATCH; ++kk) {
                 const uint32_t o = lane + (uint32_t)(tb + half * BATCH + kk - t0) * row;
-                xr[kk] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wx, o);      // zero past the run
-                dyr[kk] = win_load_aux<RAG ? 0 : WIN_NT, raw_t>(wdy, o);
+                xr[kk] = win_load<raw_t>(wx, o);      // zero past the run
+                dyr[kk] = win_load<raw_t>(wdy, o);
             }
 #pragma unroll
             for (int kk = 0; kk < BATCH; ++kk) {
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void dwconv_bwd_kernel(const T *__restrict__ d
 #pragma unroll
                     for (int v = 0; v < V; ++v)
                         du[v] = fmaf(hr[j][PCF ? v : 0], gr[(k - (HL - 1) + j) & (RING - 1)][v], du[v]);
-                win_store_aux<RAG ? 0 : WIN_NT_ST>(wdx, lane + (uint32_t)(t - (HL - 1) - t_start) * row, packv<T, V>(du));
+                win_store(wdx, lane + (uint32_t)(t - (HL - 1) - t_start) * row, packv<T, V>(du));
             }
         }
     }
@@ -238,9 +238,11 @@ DwPlan plan(const Dims &dm, int V, int longest, bool backward)
     return p;
 }
 
-// Rows that start and end on odd 32-byte sectors are accessed without the streaming hint: the parts of a shared 64 bytes then
-// meet in the L2 (3 x 17810 x 7536 bf16: forward 400 -> 390 us, 426 -> 390 with GCG_KEEP_OUTPUT, backward 608 -> 583; rows of
-// whole lines 154 -> 165 and 236 -> 254).
+// Rows that start and end on odd 32-byte sectors: the forward's accesses go without the streaming hint, and the parts of a
+// shared 64 bytes meet in the L2 (followed by the operator, 3 x 17810 x 7536 bf16 645 -> 620 us, planar 8 x 3021 x 16656
+// 630 -> 590; 1 x 12000 x 12144 199 -> 204; rows of whole lines 154 -> 165 alone).  The backward keeps it: alone it gained
+// 600 -> 582 us without, behind the operator's backward, whose gradient is partly in the cache then, it lost 960 -> 971, and
+// in fp32 arithmetic at 1 x 12000 x 12144 344 -> 365.
 template <typename T> bool ragged(const Dims &dm) { return (uint64_t)dm.d * sizeof(T) % 64 != 0; }
 
 template <typename T, int HL, int V, bool PCF>
@@ -268,7 +270,7 @@ int bwd_launch(const void *dy, const void *x, const void *w, void *dx, void *dw,
     int e = 0;
     const DwPlan p = plan(dm, V, 128, true);
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-    e = launch_plain(ragged<T>(dm) ? dwconv_bwd_kernel<T, HL, V, PCF, true> : dwconv_bwd_kernel<T, HL, V, PCF>, dim3((unsigned)p.nwg), dim3(p.threads), st,
+    e = launch_plain((dwconv_bwd_kernel<T, HL, V, PCF>), dim3((unsigned)p.nwg), dim3(p.threads), st,
                        (const T *)dy, (const T *)x, (const T *)w, (T *)dx, (float *)ws, dm, p);
     if (e) return e;
     // partials are ws[tap][(batch, run)][slot], slot = channel (per-channel filters) or lane

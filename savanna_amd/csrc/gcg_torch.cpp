@@ -4,7 +4,8 @@
 // implementation checks its arguments, allocates the outputs with torch's allocator, and
 // enqueues the C-ABI entry point on torch's current stream under a device guard; error codes
 // become exceptions.  The backward formulas of the forward operators are registered on the Python side
-// (savanna_amd/_ops.py: torch.library.register_autograd), each in terms of the backward operator defined here.
+// (savanna_amd/_ops.py: torch.library.register_autograd), each in terms of the backward operator defined here; the calls
+// of a training step that need no tracing take C++ autograd nodes instead (gate_conv_gate and the others below).
 //
 // This is the counterpart of the Triton launch wrappers two_pass_fwd_grouped /
 // two_pass_bwd_refactor (savanna/kernels/triton_src/cgcg/src/fwd.py:13-233, src/bwd.py:347-474)
