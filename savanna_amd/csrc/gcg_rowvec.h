@@ -115,7 +115,8 @@ template <typename T, int VV> __device__ __forceinline__ typename Vec<T, VV>::ra
 // side by side) and runs of ts rows.  The waves that the fullest SIMD gets, together or one after the other, times the rows a
 // wave walks -- its run and `extra` rows of halo and set-up -- is what a launch takes, so the plan is the smallest such
 // product over the 256 CUs of four SIMDs (streams: the kernel waits for memory, and three waves on four SIMDs count as that;
-// 8192 x 16 x 768 time-major, backward, 1.5 waves of 256 rows 293 us, 3 of 128 302), times `alone` for one wave per SIMD, which waits for its rows alone.
+// 8192 x 16 x 768 time-major, backward, 1.5 waves of 256 rows 293 us, 3 of 128 302); fewer than `alone` waves per SIMD count as
+// that many, since nothing hides their waits (a factor on one wave alone: 3 x 3000 x 640 f16 forward 20 us, so 15 - 16).
 // Runs are multiples of `unit` and at most `longest` rows; workgroups of four waves unless fewer leave less idle.  No more than
 // most_lanes lanes have work, unless even the longest runs need more (lanes leave partial sums behind).
 // (Against runs of a power of two that fill two workgroups per CU at least: mixer 3 x 17810 x 2512 bf16 backward 545 -> 435 us,
@@ -139,7 +140,7 @@ inline RunPlan plan_runs(int64_t bs, int64_t L, int64_t nvec, int unit, int long
             if (ts > longest || bs * runs * nvec > most_lanes) continue;
             const int64_t per_cu = (per * runs + 255) / 256;
             const double per_simd = k == 3 && streams ? 0.75 * (double)per_cu : (double)((per_cu * k + 3) / 4);
-            const double cost = per_simd * (double)(ts + extra) * (per_simd <= 1 ? alone : 1.0);
+            const double cost = (per_simd < alone ? alone : per_simd) * (double)(ts + extra);
             if (best.waves == 0 || cost < least * (k == best.waves ? 1.0 : 0.97)) { best = RunPlan{k, (int)ncvb, (int)ts}; least = cost; }
             if (ts == unit) break;
         }

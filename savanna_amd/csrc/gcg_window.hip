@@ -10,6 +10,7 @@
 #include "gcg_rowvec.h"
 
 #include <cstdlib>
+#include <type_traits>
 
 namespace gcg {
 namespace {
@@ -72,7 +73,7 @@ struct WinPlan { int v, nvec, nseg, ts, ncvb, threads, xcd; int64_t nthreads, nw
 // ---------------------------------------------------------------------------- forward
 // PK: x, B, C are interleaved in one tensor that starts at C (element stride 3).
 // EXTRA: also write the convolution before the post-gate (y2) and the pre-gate product (bx).
-// RAG: rows off the 128-byte lines (fwd_form).
+// RAG: accesses without the streaming hint (fwd_form).
 // Tensors are addressed through windows over the rows of this run, so no load or store sits
 // behind a branch: rows before the sequence start read as zero, rows past the run are dropped.
 template <typename T, int HL, int V, bool PK, bool EXTRA, bool RAG = false>
@@ -390,12 +391,12 @@ __global__ __launch_bounds__(256) void window_bwd_kernel(const T *__restrict__ d
         if (j < hl) slot[(size_t)(hl - 1 - j) * pl.nthreads] = dha[j];
 }
 
-WinPlan plan(const Dims &dm, int v, int longest, int64_t most_lanes)
+WinPlan plan(const Dims &dm, int v, int longest, double alone, int64_t most_lanes)
 {
     WinPlan p;
     p.v = v;
     p.nvec = (int)(dm.d / v);
-    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, 1.3, most_lanes, true);
+    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, alone, most_lanes, true);
     p.ts = r.ts;
     static const char *env = tuning_env("GCG_WINDOW_ROWS");   // tuning override: rows per lane, a multiple of 8
     if (env && atoi(env) >= 8 && atoi(env) % 8 == 0) p.ts = atoi(env);
@@ -414,25 +415,44 @@ WinPlan plan(const Dims &dm, int v, int longest, int64_t most_lanes)
 constexpr int BWD_ROWS = 1024;
 constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(float));
 
+// What a plan counts for a wave that has its SIMD to itself (plan_runs), by what that costs in each kernel.  The backward of
+// separate fp32 operands, and of f16 ones beyond four taps, holds over 256 registers: its waves run one at a time whatever
+// the plan, and a second round only adds its halo (3 x 3000 x 640 f16 43 -> 33 us, 2 x 4000 x 2880 85 -> 77, 2 x 1896 x 2880
+// fp32 79 -> 70; the others lose 5 - 15 % with that figure: 1 x 14000 x 272, 3 taps, f16 36 -> 42, 1 x 9000 x 1152 bf16
+// 47 -> 56).  The 4 % are for long runs, where that halo is little and two rounds are ahead (2 x 8192 x 4096 fp32 361 and 366 us).
+constexpr double ALONE = 1.3, BWD_ONE_WAVE = 1.04;
+template <typename T, int HL> constexpr double bwd_alone()
+{
+    return std::is_same_v<T, float> || (HL > 4 && (std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t>)) ? BWD_ONE_WAVE : ALONE;
+}
+
 constexpr int BWD_V = 4;   // the backward keeps four rings per lane: 4 channels is what fits
 // interleaved operands: the lane width that makes a row piece 12 contiguous bytes
 template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
 
-// How the forward walks, by how its rows lie.  Rows of a multiple of 8 KB: long runs, streaming accesses, plain order of
-// workgroups (1 x 32768 x 8192 bf16 377 us; short runs in XCD order 411).  Other whole lines: runs of at most 128 rows in
-// XCD-contiguous order (1 x 399457 x 1344 1032 -> 840 us, 1 x 38836 x 3456 227 -> 214; 16 rows 902 and 204).  Rows off the
-// lines: plain accesses, so that the parts of a shared line meet in the L2, and 16 rows in plain order, so that the
-// neighbours of a line run at once (1 x 264208 x 2032 1415 -> 850 us, 1 x 64527 x 2080 224 -> 215, 1 x 46091 x 2912 262 ->
-// 210; 64 rows in XCD order 865, 250 and 227, streaming accesses 925 with those).  Interleaved 16-bit operands take that
-// form for whole lines too, their pieces being 12 bytes a lane (1 x 38836 x 3456 213 -> 197, 1 x 100000 x 1344 210 -> 199;
-// fp32 2 x 20000 x 2240 stays: 265, with 16 rows 268).  Time-major 8192 x 16 x 768: 164 -> 156 us in XCD order.
-struct FwdForm { int longest; bool rag, xcd; };
-FwdForm fwd_form(const Dims &dm, size_t es)
+// How the forward walks.  Runs of at most 128 rows in XCD-contiguous order, except:
+// - rows of a multiple of 8 KB (but separate fp32 operands): long runs in plain order (1 x 32768 x 8192 bf16 377 us, short runs
+//   in XCD order 411; 2 x 8192 x 4096 fp32 separate 211, in XCD order 189, interleaved 183 and 187);
+// - operands and result beyond the last-level cache, with rows off the 128-byte lines (but separate fp32 operands) or
+//   interleaved in 16 bits: 16 rows in plain order without the streaming hint, so that the neighbours of a line run at once and
+//   its parts meet in the L2 (1 x 264208 x 2032 bf16 1415 -> 850 us, 2 x 20000 x 2400 152 against 167 in the common form,
+//   interleaved 149 and 168, 1 x 38836 x 3456 interleaved 197 and 213; in the cache the common form is ahead: 2 x 9000 x 1456
+//   47 and 49, 3 x 5000 x 1440 40 and 43, interleaved 2 x 4000 x 2880 37 and 41; fp32 1 x 30000 x 2032 198 and 212).
+// The common form against long runs in plain order: 1 x 399457 x 1344 840 and 1032 us, 2 x 20000 x 2240 fp32 270 and 281.
+// Separate fp32 operands wait for their 16-byte rows longest: in the cache 2.5 waves per SIMD hide it (2 x 3000 x 960 30 -> 27
+// us, 4 x 1500 x 1600 38 -> 36), beyond it 2 do (2 x 8192 x 4096 200 -> 212 at 2.5); separate f16 ones 1.75
+// (1 x 5000 x 2048 23 -> 21, 3 x 3000 x 640 16.3 -> 15.2; bf16 loses 2 % at it).
+struct FwdForm { int longest; bool rag, xcd; double alone; };
+template <typename T> FwdForm fwd_form(const Dims &dm)
 {
+    constexpr size_t es = sizeof(T);
+    constexpr bool f16 = std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t>;
     const uint64_t row = (uint64_t)dm.d * es;
-    if (row % 8192 == 0) return FwdForm{1024, false, false};
-    if (row % 128 != 0 || (dm.es == 3 && es == 2)) return FwdForm{16, true, false};
-    return FwdForm{128, false, true};
+    const bool big = 4 * (double)dm.bs * (double)dm.L * (double)row > 256.0 * 1024 * 1024, f32 = es == 4 && dm.es == 1;
+    const double alone = f32 ? big ? 2.0 : 2.5 : f16 && dm.es == 1 ? 1.75 : ALONE;
+    if (row % 8192 == 0 && !f32) return FwdForm{1024, false, false, alone};
+    if (big && !f32 && (row % 128 != 0 || (dm.es == 3 && es == 2))) return FwdForm{16, true, false, alone};
+    return FwdForm{128, false, true, alone};
 }
 
 template <typename T, int HL, int V>
@@ -440,11 +460,11 @@ int fwd_v(const void *x, const void *B, const void *C, const void *h, void *y, v
           const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const FwdForm form = fwd_form(dm, sizeof(T));
+    const FwdForm form = fwd_form<T>(dm);
     const bool rag = form.rag;
     if (dm.es == 3) {
         constexpr int VI = il_v<T>();
-        WinPlan p = plan(dm, VI, form.longest, INT64_MAX);
+        WinPlan p = plan(dm, VI, form.longest, form.alone, INT64_MAX);
         p.xcd = form.xcd;
         if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
         const auto kern = rag ? window_fwd_kernel<T, HL, VI, true, false, true> : window_fwd_kernel<T, HL, VI, true, false>;
@@ -452,7 +472,7 @@ int fwd_v(const void *x, const void *B, const void *C, const void *h, void *y, v
                            (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
         return e;
     }
-    WinPlan p = plan(dm, V, form.longest, INT64_MAX);
+    WinPlan p = plan(dm, V, form.longest, form.alone, INT64_MAX);
     p.xcd = form.xcd;
     const int64_t nwg = p.nwg;
     if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
@@ -470,7 +490,7 @@ int bwd_t(const void *dy, const void *x, const void *B, const void *C, const voi
           void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const WinPlan p = plan(dm, dm.es == 3 ? il_v<T>() : BWD_V, BWD_ROWS, BWD_LANES);
+    const WinPlan p = plan(dm, dm.es == 3 ? il_v<T>() : BWD_V, BWD_ROWS, dm.es == 3 ? ALONE : bwd_alone<T, HL>(), BWD_LANES);
     const int64_t nwg = p.nwg;
     if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if (dm.es == 3 && dm.keep_out)
@@ -541,14 +561,17 @@ int window_fwd_launch(int dtype, const void *x, const void *B, const void *C, co
 }
 
 // one figure for the separate-tensor backward (4 channels per lane) and the interleaved one
-// (2 or 1) of every element type: the largest of the three plans
+// (2 or 1) of every element type: the largest of their plans
 size_t window_bwd_workspace(const Dims &dm)
 {
     int64_t n = 0;
     for (int v : {1, 2, BWD_V}) {
         if (dm.d % v) continue;
-        const WinPlan p = plan(dm, v, BWD_ROWS, BWD_LANES);
-        if (p.nthreads > n) n = p.nthreads;
+        for (double alone : {ALONE, BWD_ONE_WAVE}) {
+            if (alone != ALONE && v != BWD_V) continue;         // (separate tensors alone have the second figure)
+            const WinPlan p = plan(dm, v, BWD_ROWS, alone, BWD_LANES);
+            if (p.nthreads > n) n = p.nthreads;
+        }
     }
     return (size_t)n * dm.hl * sizeof(float);
 }

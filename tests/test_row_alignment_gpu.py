@@ -80,3 +80,28 @@ def test_register_window_kernels(dtype, arith, bs, L, g, wide, planar):
     dwb = b[1].reshape(3, g, dg, 3) if planar else b[1].reshape(g, dg, 3, 3).permute(2, 0, 1, 3)
     assert (dwa[:, :g].float() - dwb.float()).abs().max() <= ulp[dtype] * dwa.float().abs().max()
     assert (a[2][:g].float() - b[2].float()).abs().max() <= ulp[arith] * a[2].float().abs().max()
+
+
+@pytest.mark.parametrize("dtype,g,interleaved", [(torch.bfloat16, 29, False), (torch.float16, 61, True), (torch.bfloat16, 28, True),
+                                                 (torch.float32, 30, True), (torch.float32, 31, False)])
+def test_window_forward_beyond_the_cache(dtype, g, interleaved):
+    """Tensors that together exceed the last-level cache are walked in another form; a row depends on the six before it, so
+    pieces of the result are those of the same rows by themselves."""
+    dg, hl = 16, 7
+    row = g * dg * dtype.itemsize
+    L = (1 << 26) // row + 1003
+    gen = torch.Generator(device=DEV).manual_seed(g)
+    h = (torch.randn(g, 1, hl, generator=gen, device=DEV) / hl ** 0.5).to(dtype)
+    if interleaved:
+        ops = [torch.empty(1, L, g, dg, 3, device=DEV, dtype=dtype).normal_(generator=gen)]
+        f = lambda a: _lib.fwd_interleaved(a[0], h)
+    else:
+        ops = [torch.empty(1, L, g, dg, device=DEV, dtype=dtype).normal_(generator=gen) for _ in range(3)]
+        f = lambda a: _lib.fwd(*a, h)[2]
+    assert 4 * L * row > 1 << 28
+    y = f(ops)
+    n = 4000
+    assert torch.equal(y[:, :n], f([t[:, :n].contiguous() for t in ops]))
+    for t0 in (n, L // 2 + 5, L - n):
+        part = f([t[:, t0 - hl + 1:t0 + n].contiguous() for t in ops])
+        assert torch.equal(y[:, t0:t0 + n], part[:, hl - 1:])
