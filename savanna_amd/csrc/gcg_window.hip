@@ -417,7 +417,7 @@ constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(floa
 
 // What a plan counts for a wave that has its SIMD to itself (plan_runs), by what that costs in each kernel.  The backward of
 // separate fp32 operands, and of f16 ones beyond four taps, holds over 256 registers: its waves run one at a time whatever
-// the plan, and a second round only adds its halo (3 x 3000 x 640 f16 43 -> 33 us, 2 x 4000 x 2880 85 -> 77, 2 x 1896 x 2880
+// the plan, and a second round only adds its halo (2 x 4000 x 2880 f16 85 -> 78 us, 1 x 30000 x 480 72 -> 62, 2 x 1896 x 2880
 // fp32 79 -> 70; the others lose 5 - 15 % with that figure: 1 x 14000 x 272, 3 taps, f16 36 -> 42, 1 x 9000 x 1152 bf16
 // 47 -> 56).  The 4 % are for long runs, where that halo is little and two rounds are ahead (2 x 8192 x 4096 fp32 361 and 366 us).
 constexpr double ALONE = 1.3, BWD_ONE_WAVE = 1.04;
