@@ -140,9 +140,14 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_fwd_kernel(const T *__restric
         W1[i] = M::toeplitz(htab[w], 32 * i + 16, j, q);
     }
 
-    // (before the sequence there is nothing to rebuild; three-plane operands leave no registers for a choice)
-    constexpr bool THREE_PLANES = std::is_same_v<T, float> || std::is_same_v<T, f16w_t>;
-    if (NK > 1 && (THREE_PLANES || s_lo > 0)) {
+    // (Before the sequence there is nothing to rebuild.  The branch costs registers, since the lead-in's rows stay requested
+    // in front of it, and is taken where it pays: bf16 tensors in fp32 arithmetic.  Up to 97 taps, 2 x 8192 x 4096 16 taps
+    // 105 -> 93 us, 80 taps 108 -> 95, 1 x 20000 x 976 16 taps 42 -> 38; 128 taps 106 either way.  With the featurizer 8-wave
+    // workgroups, 1 x 701 x 4096 15.9 -> 15.7; 4-wave ones hold one wave per SIMD instead of two with it, 8 x 40000 x 64 47 -> 63,
+    // 1 x 221 x 64 12.7 -> 11.1.  16-bit arithmetic: three waves per SIMD instead of four, 8 x 20000 x 48, 128 taps, 20.5 -> 23.5,
+    // 2 x 8192 x 4096, 16 taps, 90 -> 93.  Three-plane operands leave no registers for it.)
+    constexpr bool SKIP = std::is_same_v<T, bf16w_t> && (FEAT ? NW == 8 : NK <= 4);
+    if (NK > 1 && (!SKIP || s_lo > 0)) {
 #pragma unroll
         for (int i = 1; i < NK; ++i) {
             float xf[8], Bf[8], Cf[8], uf[8];
@@ -370,6 +375,8 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_bwd_kernel(const T *__restric
     constexpr int NLEAD = NK > 1 ? NK - 1 : 1;
     u32x3 past[NLEAD][NH + NR], lead[NLEAD][NH + NR];
     Row<T> wdy[NLEAD];
+    constexpr bool EARLY_TAPS = FEAT && sizeof(T) == 2;
+    if constexpr (EARLY_TAPS) feat_taps<T, KF, NV>(tap_words, tap);
     if constexpr (NK > 1) {
 #pragma unroll
         for (int i = 1; i < NK; ++i) {
@@ -380,7 +387,7 @@ __global__ __launch_bounds__(64 * NW) void mfma_il_bwd_kernel(const T *__restric
     }
     fetch_feat(3 * step_off(s_lo + NK - 1), in);
     fetch_dy(step_off(s_lo + NK - 1), dyr);
-    if constexpr (FEAT) feat_taps<T, KF, NV>(tap_words, tap);
+    if constexpr (FEAT && !EARLY_TAPS) feat_taps<T, KF, NV>(tap_words, tap);
 
     store_taps(htab + w * HTAB, l, hv);
     __syncthreads();
@@ -706,11 +713,13 @@ __global__ __launch_bounds__(512) void mfma_il_bwd_duo_kernel(const T *__restric
             Rows lead[NK];
 #pragma unroll
             for (int i = 1; i < NK; ++i) fetch_feat(3 * step_off(s_lo - i), past[i - 1]);
+            // (converted before the other requests, whose rows leave no registers for the words beside the taps: behind them
+            // nine registers spilled, 1 x 1183 x 128 36.9 us against 35.6, 3 x 1224 x 320 46.6 and 45.3)
+            if constexpr (FEAT) feat_taps<T, KF, NV>(tap_words, tap);
 #pragma unroll
             for (int jj = NK - 2; jj >= 0; --jj) fetch(step_off(s_lo + jj), 3 * step_off(s_lo + jj), lead[jj]);
             fetch(step_off(s_lo + NK - 1), 3 * step_off(s_lo + NK - 1), lead[NK - 1]);
             fetch(step_off(s_lo + NK), 3 * step_off(s_lo + NK), st[1]);
-            if constexpr (FEAT) feat_taps<T, KF, NV>(tap_words, tap);
             __syncthreads();                                          // (A)
             __syncthreads();                                          // (A2): the filter tables' place is free
             float f0[8], f1[8], f2[8];
