@@ -292,6 +292,10 @@ namespace gcg {
 struct KernelTimer { hipEvent_t start, stop; };
 KernelTimer take_kernel_timer();
 
+// What a launch can hold: 2^31 - 1 workgroups and 2^32 - 1 work-items.  Narrow tensors in short runs reach the second first (one
+// group of four channels is one lane of a wave: 2^30 rows in runs of 16).
+inline bool launch_holds(int64_t nwg, int64_t threads) { return nwg <= 0x7fffffffLL && nwg * threads <= 0xffffffffLL; }
+
 // Every launch returns the runtime's own code for that launch (hipLaunchKernel / hipExtLaunchKernel)
 // rather than the thread's sticky last error, so an error left behind by other code on the thread is
 // neither reported as this library's nor cleared from under its owner.
@@ -299,6 +303,8 @@ template <typename... KArgs, size_t... I>
 inline int launch_packed(const void *fn, dim3 grid, dim3 block, hipStream_t st, const KernelTimer &t,
                          std::tuple<KArgs...> &vals, std::index_sequence<I...>, size_t lds = 0)
 {
+    // the runtime takes a grid of 2^32 work-items or more and runs what is left of it modulo 2^32
+    if (!launch_holds((int64_t)grid.x * grid.y * grid.z, (int64_t)block.x * block.y * block.z)) return (int)hipErrorInvalidConfiguration;
     void *ptrs[] = {(void *)&std::get<I>(vals)...};
     if (t.start || t.stop)
         return (int)hipExtLaunchKernel(fn, grid, block, ptrs, lds, st, t.start, t.stop, 0);

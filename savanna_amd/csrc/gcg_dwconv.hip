@@ -249,7 +249,8 @@ template <typename T, int HL, int V, bool PCF>
 int fwd_launch(const void *x, const void *w, void *y, const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const DwPlan p = plan(dm, V, (uint64_t)dm.d * sizeof(T) % 8192 == 0 ? 128 : 64, false);
+    DwPlan p = plan(dm, V, (uint64_t)dm.d * sizeof(T) % 8192 == 0 ? 128 : 64, false);
+    if (!launch_holds(p.nwg, p.threads)) p = plan(dm, V, 128, false);
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if (ragged<T>(dm))
         e = launch_plain((dwconv_fwd_kernel<T, HL, V, PCF, true, true>), dim3((unsigned)p.nwg), dim3(p.threads), st,

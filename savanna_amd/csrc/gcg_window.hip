@@ -455,32 +455,42 @@ template <typename T> FwdForm fwd_form(const Dims &dm)
     return FwdForm{128, false, true, alone};
 }
 
+// the plan of a forward in its form, or in long runs where that would be more than a launch holds
+template <typename T> WinPlan fwd_plan(const Dims &dm, int v, FwdForm &form)
+{
+    form = fwd_form<T>(dm);
+    WinPlan p = plan(dm, v, form.longest, form.alone, INT64_MAX);
+    if (!launch_holds(p.nwg, p.threads)) {
+        form = FwdForm{1024, false, false, form.alone};
+        p = plan(dm, v, form.longest, form.alone, INT64_MAX);
+    }
+    p.xcd = form.xcd;
+    return p;
+}
+
 template <typename T, int HL, int V>
 int fwd_v(const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
           const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const FwdForm form = fwd_form<T>(dm);
-    const bool rag = form.rag;
+    FwdForm form;
     if (dm.es == 3) {
         constexpr int VI = il_v<T>();
-        WinPlan p = plan(dm, VI, form.longest, form.alone, INT64_MAX);
-        p.xcd = form.xcd;
+        const WinPlan p = fwd_plan<T>(dm, VI, form);
         if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-        const auto kern = rag ? window_fwd_kernel<T, HL, VI, true, false, true> : window_fwd_kernel<T, HL, VI, true, false>;
+        const auto kern = form.rag ? window_fwd_kernel<T, HL, VI, true, false, true> : window_fwd_kernel<T, HL, VI, true, false>;
         e = launch_main(kern, dim3((unsigned)p.nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
         return e;
     }
-    WinPlan p = plan(dm, V, form.longest, form.alone, INT64_MAX);
-    p.xcd = form.xcd;
+    const WinPlan p = fwd_plan<T>(dm, V, form);
     const int64_t nwg = p.nwg;
     if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if (y2 || bx)
         e = launch_main((window_fwd_kernel<T, HL, V, false, true>), dim3((unsigned)nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
     else
-        e = launch_main(rag ? window_fwd_kernel<T, HL, V, false, false, true> : window_fwd_kernel<T, HL, V, false, false>, dim3((unsigned)nwg), dim3(p.threads), st,
+        e = launch_main(form.rag ? window_fwd_kernel<T, HL, V, false, false, true> : window_fwd_kernel<T, HL, V, false, false>, dim3((unsigned)nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
     return e;
 }
