@@ -437,7 +437,8 @@ template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
 //   interleaved in 16 bits: 16 rows in plain order without the streaming hint, so that the neighbours of a line run at once and
 //   its parts meet in the L2 (1 x 264208 x 2032 bf16 1415 -> 850 us, 2 x 20000 x 2400 152 against 167 in the common form,
 //   interleaved 149 and 168, 1 x 38836 x 3456 interleaved 197 and 213; in the cache the common form is ahead: 2 x 9000 x 1456
-//   47 and 49, 3 x 5000 x 1440 40 and 43, interleaved 2 x 4000 x 2880 37 and 41; fp32 1 x 30000 x 2032 198 and 212).
+//   47 and 49, 3 x 5000 x 1440 40 and 43, interleaved 2 x 4000 x 2880 37 and 41; fp32 1 x 30000 x 2032 198 and 212).  With y2
+//   and Bx written as well 1 x 30000 x 2032 169 us, in the common form 195, in these runs with the hint 214; y2 alone 137, 154, 173.
 // The common form against long runs in plain order: 1 x 399457 x 1344 840 and 1032 us, 2 x 20000 x 2240 fp32 270 and 281.
 // Separate fp32 operands wait for their 16-byte rows longest: in the cache 2.5 waves per SIMD hide it (2 x 3000 x 960 30 -> 27
 // us, 4 x 1500 x 1600 38 -> 36), beyond it 2 do (2 x 8192 x 4096 200 -> 212 at 2.5); separate f16 ones 1.75
@@ -468,31 +469,20 @@ template <typename T> WinPlan fwd_plan(const Dims &dm, int v, FwdForm &form)
     return p;
 }
 
-template <typename T, int HL, int V>
+// the plan and the kernel of one form together: what walks without the streaming hint walks in its runs, and nothing else does
+template <typename T, int HL, int V, bool PK, bool EXTRA>
 int fwd_v(const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
           const Dims &dm, hipStream_t st)
 {
-    int e = 0;
     FwdForm form;
-    if (dm.es == 3) {
-        constexpr int VI = il_v<T>();
-        const WinPlan p = fwd_plan<T>(dm, VI, form);
-        if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-        const auto kern = form.rag ? window_fwd_kernel<T, HL, VI, true, false, true> : window_fwd_kernel<T, HL, VI, true, false>;
-        e = launch_main(kern, dim3((unsigned)p.nwg), dim3(p.threads), st,
-                           (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
-        return e;
-    }
     const WinPlan p = fwd_plan<T>(dm, V, form);
-    const int64_t nwg = p.nwg;
-    if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-    if (y2 || bx)
-        e = launch_main((window_fwd_kernel<T, HL, V, false, true>), dim3((unsigned)nwg), dim3(p.threads), st,
-                           (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
-    else
-        e = launch_main(form.rag ? window_fwd_kernel<T, HL, V, false, false, true> : window_fwd_kernel<T, HL, V, false, false>, dim3((unsigned)nwg), dim3(p.threads), st,
-                           (const T *)x, (const T *)B, (const T *)C, (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
-    return e;
+    if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
+    auto kernel = window_fwd_kernel<T, HL, V, PK, EXTRA>;
+    if constexpr (PK || sizeof(T) == 2) {                   // (fwd_form: never for separate fp32 operands)
+        if (form.rag) kernel = window_fwd_kernel<T, HL, V, PK, EXTRA, true>;
+    }
+    return launch_main(kernel, dim3((unsigned)p.nwg), dim3(p.threads), st, (const T *)x, (const T *)B, (const T *)C,
+                       (const T *)h, (T *)y, (T *)y2, (T *)bx, dm, p);
 }
 
 template <typename T, int HL>
@@ -527,7 +517,9 @@ template <typename T, int HL>
 int fwd_t(const void *x, const void *B, const void *C, const void *h, void *y, void *y2, void *bx,
           const Dims &dm, hipStream_t st)
 {
-    return fwd_v<T, HL, 4>(x, B, C, h, y, y2, bx, dm, st);
+    if (dm.es == 3) return fwd_v<T, HL, il_v<T>(), true, false>(x, B, C, h, y, y2, bx, dm, st);
+    if (y2 || bx) return fwd_v<T, HL, 4, false, true>(x, B, C, h, y, y2, bx, dm, st);
+    return fwd_v<T, HL, 4, false, false>(x, B, C, h, y, y2, bx, dm, st);
 }
 
 template <typename T>

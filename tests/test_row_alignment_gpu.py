@@ -82,26 +82,37 @@ def test_register_window_kernels(dtype, arith, bs, L, g, wide, planar):
     assert (a[2][:g].float() - b[2].float()).abs().max() <= ulp[arith] * a[2].float().abs().max()
 
 
-@pytest.mark.parametrize("dtype,g,interleaved", [(torch.bfloat16, 29, False), (torch.float16, 61, True), (torch.bfloat16, 28, True),
-                                                 (torch.float32, 30, True), (torch.float32, 31, False)])
-def test_window_forward_beyond_the_cache(dtype, g, interleaved):
-    """Tensors that together exceed the last-level cache are walked in another form; a row depends on the six before it, so
-    pieces of the result are those of the same rows by themselves."""
-    dg, hl = 16, 7
+# layout, tensors' and filter's type, groups, taps, sequences
+BEYOND = [("separate", "bfloat16", "bfloat16", 29, 7, 1), ("separate", "bfloat16", "float32", 29, 3, 2),
+          ("separate", "float16", "float16", 27, 8, 1), ("separate", "float32", "float32", 31, 7, 1),
+          ("extra", "bfloat16", "bfloat16", 29, 7, 2), ("extra", "float16", "float32", 27, 4, 1), ("extra", "float32", "float32", 31, 7, 1),
+          ("interleaved", "float16", "float16", 61, 7, 1), ("interleaved", "bfloat16", "bfloat16", 28, 8, 2),
+          ("interleaved", "float32", "float32", 30, 7, 1), ("interleaved", "float32", "float32", 31, 3, 2),
+          ("time_major", "bfloat16", "bfloat16", 29, 7, 2), ("time_major", "float16", "float32", 29, 3, 3),
+          ("planar", "float16", "float16", 27, 7, 1), ("planar", "bfloat16", "float32", 29, 8, 2)]
+
+
+@pytest.mark.parametrize("layout,dtype,arith,g,hl,bs", BEYOND)
+def test_window_forward_beyond_the_cache(layout, dtype, arith, g, hl, bs):
+    """Tensors that together exceed the last-level cache are walked in another form; a row depends on the hl - 1 before it, so
+    pieces of the result are those of the same rows by themselves.  (Pieces start at a multiple of eight rows: the walks are
+    unrolled by eight, and an f16 y2 is converted from the sum or folded into its last step by the row's place among them.)"""
+    dg, dtype = 16, getattr(torch, dtype)
     row = g * dg * dtype.itemsize
-    L = (1 << 26) // row + 1003
-    gen = torch.Generator(device=DEV).manual_seed(g)
-    h = (torch.randn(g, 1, hl, generator=gen, device=DEV) / hl ** 0.5).to(dtype)
-    if interleaved:
-        ops = [torch.empty(1, L, g, dg, 3, device=DEV, dtype=dtype).normal_(generator=gen)]
-        f = lambda a: _lib.fwd_interleaved(a[0], h)
-    else:
-        ops = [torch.empty(1, L, g, dg, device=DEV, dtype=dtype).normal_(generator=gen) for _ in range(3)]
-        f = lambda a: _lib.fwd(*a, h)[2]
-    assert 4 * L * row > 1 << 28
-    y = f(ops)
+    L = (1 << 26) // (row * bs) + 1003
+    gen = torch.Generator(device=DEV).manual_seed(g + hl)
+    h = (torch.randn(g, 1, hl, generator=gen, device=DEV) / hl ** 0.5).to(getattr(torch, arith))
+    shape = {"interleaved": (bs, L, g, dg, 3), "planar": (bs, L, 3, g, dg), "time_major": (L, bs, g, dg)}.get(layout, (bs, L, g, dg))
+    time = 0 if layout == "time_major" else 1
+    ops = [torch.empty(shape, device=DEV, dtype=dtype).normal_(generator=gen) for _ in range(1 if len(shape) == 5 else 3)]
+    f = {"interleaved": lambda a: [_lib.fwd_interleaved(a[0], h)], "planar": lambda a: [_lib.fwd_planar(a[0], h)],
+         "time_major": lambda a: [_lib.fwd_time_major(*a, h)], "separate": lambda a: [_lib.fwd(*a, h)[2]],
+         "extra": lambda a: list(_lib.fwd(*a, h, return_bx=True, return_y2=True))}[layout]
+    assert 4 * bs * L * row > 1 << 28
+    ys = f(ops)
     n = 4000
-    assert torch.equal(y[:, :n], f([t[:, :n].contiguous() for t in ops]))
-    for t0 in (n, L // 2 + 5, L - n):
-        part = f([t[:, t0 - hl + 1:t0 + n].contiguous() for t in ops])
-        assert torch.equal(y[:, t0:t0 + n], part[:, hl - 1:])
+    for t0, t1 in ((0, n), (n, 2 * n), (L // 2 + 5, L // 2 + 5 + n), (L - n, L)):
+        first = max(t0 - hl + 1, 0) // 8 * 8
+        parts = f([t.narrow(time, first, t1 - first).clone() for t in ops])
+        for y, part in zip(ys, parts):
+            assert torch.equal(y[:, t0:t1], part[:, t0 - first:])
