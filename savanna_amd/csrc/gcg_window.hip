@@ -432,27 +432,31 @@ template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
 
 // How the forward walks.  Runs of at most 128 rows in XCD-contiguous order, except:
 // - rows of a multiple of 8 KB (but separate fp32 operands): long runs in plain order (1 x 32768 x 8192 bf16 377 us, short runs
-//   in XCD order 411; 2 x 8192 x 4096 fp32 separate 211, in XCD order 189, interleaved 183 and 187);
+//   in XCD order 411; 2 x 8192 x 4096 fp32 interleaved 183, in XCD order 187);
 // - operands and result beyond the last-level cache, with rows off the 128-byte lines (but separate fp32 operands) or
 //   interleaved in 16 bits: 16 rows in plain order without the streaming hint, so that the neighbours of a line run at once and
 //   its parts meet in the L2 (1 x 264208 x 2032 bf16 1415 -> 850 us, 2 x 20000 x 2400 152 against 167 in the common form,
-//   interleaved 149 and 168, 1 x 38836 x 3456 interleaved 197 and 213; in the cache the common form is ahead: 2 x 9000 x 1456
-//   47 and 49, 3 x 5000 x 1440 40 and 43, interleaved 2 x 4000 x 2880 37 and 41; fp32 1 x 30000 x 2032 198 and 212).  With y2
-//   and Bx written as well 1 x 30000 x 2032 169 us, in the common form 195, in these runs with the hint 214; y2 alone 137, 154, 173.
+//   interleaved 149 and 168, 1 x 38836 x 3456 interleaved 197 and 213, fp32 interleaved 1 x 30000 x 2032 190 and 207,
+//   2 x 20000 x 1200 157 and 167; in the cache the common form is ahead: 2 x 9000 x 1456 47 and 49, 3 x 5000 x 1440 40 and 43,
+//   interleaved 2 x 4000 x 2880 37 and 41).  With y2 and Bx written as well 1 x 30000 x 2032 169 us, in the common form 195, in
+//   these runs with the hint 214; y2 alone 137, 154, 173.
 // The common form against long runs in plain order: 1 x 399457 x 1344 840 and 1032 us, 2 x 20000 x 2240 fp32 270 and 281.
-// Separate fp32 operands wait for their 16-byte rows longest: in the cache 2.5 waves per SIMD hide it (2 x 3000 x 960 30 -> 27
-// us, 4 x 1500 x 1600 38 -> 36), beyond it 2 do (2 x 8192 x 4096 200 -> 212 at 2.5); separate f16 ones 1.75
-// (1 x 5000 x 2048 23 -> 21, 3 x 3000 x 640 16.3 -> 15.2; bf16 loses 2 % at it).
+// Separate fp32 operands wait for their 16-byte rows longest: 2.5 waves per SIMD hide it (2 x 3000 x 960 32 -> 25 us,
+// 4 x 1500 x 1600 38 -> 36), and runs of 96 rows: 1 x 40000 x 992 128 us, with 128 rows and 2 waves 135, 1 x 56934 x 864 156 and
+// 165, 1 x 176470 x 272 163 and 198; over 39 sizes beyond the cache 4 % less time.  Rows of a multiple of 16 KB beyond it are
+// the exception: 2 x 8192 x 4096 195 us at 128 rows and 2 waves, 208 so; 2 x 4096 x 8192 195 and 205 (2048 wide, 8 KB: 222 and
+// 211).  Separate f16 operands 1.75 (1 x 5000 x 2048 23 -> 21, 3 x 3000 x 640 16.3 -> 15.2; bf16 loses 2 % at it).
 struct FwdForm { int longest; bool rag, xcd; double alone; };
 template <typename T> FwdForm fwd_form(const Dims &dm)
 {
     constexpr size_t es = sizeof(T);
     constexpr bool f16 = std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t>;
     const uint64_t row = (uint64_t)dm.d * es;
-    const bool big = 4 * (double)dm.bs * (double)dm.L * (double)row > 256.0 * 1024 * 1024, f32 = es == 4 && dm.es == 1;
-    const double alone = f32 ? big ? 2.0 : 2.5 : f16 && dm.es == 1 ? 1.75 : ALONE;
-    if (row % 8192 == 0 && !f32) return FwdForm{1024, false, false, alone};
-    if (big && !f32 && (row % 128 != 0 || (dm.es == 3 && es == 2))) return FwdForm{16, true, false, alone};
+    const bool big = 4 * (double)dm.bs * (double)dm.L * (double)row > 256.0 * 1024 * 1024;
+    if (es == 4 && dm.es == 1) return big && row % 16384 == 0 ? FwdForm{128, false, true, 2.0} : FwdForm{96, false, true, 2.5};
+    const double alone = f16 && dm.es == 1 ? 1.75 : ALONE;
+    if (row % 8192 == 0) return FwdForm{1024, false, false, alone};
+    if (big && (row % 128 != 0 || (dm.es == 3 && es == 2))) return FwdForm{16, true, false, alone};
     return FwdForm{128, false, true, alone};
 }
 
