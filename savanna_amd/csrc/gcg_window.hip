@@ -460,14 +460,18 @@ template <typename T> FwdForm fwd_form(const Dims &dm)
     return FwdForm{128, false, true, alone};
 }
 
-// the plan of a forward in its form, or in long runs where that would be more than a launch holds
+// The plan of a forward in its form, or in long runs where that would be more than a launch holds.  What hides a wave's waits is
+// the lanes in flight: rows that leave lanes of the last wave idle count that many more waves (1 x 13097 x 336 fp32, 84 lanes
+// of two waves, 23.7 -> 20.6 us, 1 x 36964 x 320 time-major 52 -> 44; over 118 sizes up to 1100 channels, of all types, 1 %).
 template <typename T> WinPlan fwd_plan(const Dims &dm, int v, FwdForm &form)
 {
+    const int64_t nvec = dm.d / v;
+    const double idle = (double)((nvec + 63) / 64 * 64) / (double)nvec;
     form = fwd_form<T>(dm);
-    WinPlan p = plan(dm, v, form.longest, form.alone, INT64_MAX);
+    WinPlan p = plan(dm, v, form.longest, form.alone * idle, INT64_MAX);
     if (!launch_holds(p.nwg, p.threads)) {
         form = FwdForm{1024, false, false, form.alone};
-        p = plan(dm, v, form.longest, form.alone, INT64_MAX);
+        p = plan(dm, v, form.longest, form.alone * idle, INT64_MAX);
     }
     p.xcd = form.xcd;
     return p;
