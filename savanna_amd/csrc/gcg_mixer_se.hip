@@ -843,7 +843,10 @@ MixPlan plan(const Dims &dm, int ch, bool backward)
     // Long runs keep the halo of up to 10 rows each side and the filter-gradient partials small (9 % of the traffic at 128
     // rows, 4 % at 512).  The backward gains nothing beyond 512 rows; the forward does (40B shape: 409 us at 512 rows, 383 at
     // 1024).  Multiples of 16 (the backward's longest ring).
-    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, 16, backward ? 512 : 1024, 9, 1.1, INT64_MAX, false);
+    // Two waves per SIMD hide the forward's waits (plan_runs): with 1.1, what the backward's one wave at a time counts, calls of
+    // 10 - 60 us took one long wave each: 3 x 2094 x 1056 planar bf16 28.7 -> 20.3 us, 2 x 1898 x 1920 26 -> 22, 3 x 6431 x 1312 f16
+    // 65 -> 58; over 120 sizes in and beyond the cache 1.1 2.5 % less time than runs of a power of two, 2 and 2.5 5 %, 3 4.5 %.
+    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, 16, backward ? 512 : 1024, 9, backward ? 1.1 : 2.0, INT64_MAX, false);
     p.ts = r.ts;
     static const char *env = tuning_env("GCG_MIXER_ROWS");      // tuning override: rows per lane, a multiple of 16
     if (env && atoi(env) >= 16 && atoi(env) % 16 == 0) p.ts = atoi(env);
