@@ -420,7 +420,10 @@ constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(floa
 // the plan, and a second round only adds its halo (2 x 4000 x 2880 f16 85 -> 78 us, 1 x 30000 x 480 72 -> 62, 2 x 1896 x 2880
 // fp32 79 -> 70; the others lose 5 - 15 % with that figure: 1 x 14000 x 272, 3 taps, f16 36 -> 42, 1 x 9000 x 1152 bf16
 // 47 -> 56).  The 4 % are for long runs, where that halo is little and two rounds are ahead (2 x 8192 x 4096 fp32 361 and 366 us).
-constexpr double ALONE = 1.3, BWD_ONE_WAVE = 1.04;
+// Interleaved fp32 operands: a lane has one channel, 12 bytes a row, and one wave's rows in flight do not keep memory busy where
+// the second would (1 x 7443 x 2944 140 -> 124 us, 4 x 1500 x 1600 70 -> 63, 3 x 218 x 3632 30 -> 27.8, 1 x 3184 x 752 30 -> 27; over
+// 104 sizes 1 % less time, and half as many that lose to runs of a power of two).
+constexpr double ALONE = 1.3, BWD_ONE_WAVE = 1.04, BWD_ONE_CHANNEL = 2.0;
 template <typename T, int HL> constexpr double bwd_alone()
 {
     return std::is_same_v<T, float> || (HL > 4 && (std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t>)) ? BWD_ONE_WAVE : ALONE;
@@ -429,6 +432,7 @@ template <typename T, int HL> constexpr double bwd_alone()
 constexpr int BWD_V = 4;   // the backward keeps four rings per lane: 4 channels is what fits
 // interleaved operands: the lane width that makes a row piece 12 contiguous bytes
 template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
+constexpr double il_bwd_alone(int v) { return v == 1 ? BWD_ONE_CHANNEL : ALONE; }
 
 // How the forward walks.  Runs of at most 128 rows in XCD-contiguous order, except:
 // - rows of a multiple of 8 KB (but separate fp32 operands): long runs in plain order (1 x 32768 x 8192 bf16 377 us, short runs
@@ -498,7 +502,7 @@ int bwd_t(const void *dy, const void *x, const void *B, const void *C, const voi
           void *dC, void *dh, void *ws, const Dims &dm, hipStream_t st)
 {
     int e = 0;
-    const WinPlan p = plan(dm, dm.es == 3 ? il_v<T>() : BWD_V, BWD_ROWS, dm.es == 3 ? ALONE : bwd_alone<T, HL>(), BWD_LANES);
+    const WinPlan p = plan(dm, dm.es == 3 ? il_v<T>() : BWD_V, BWD_ROWS, dm.es == 3 ? il_bwd_alone(il_v<T>()) : bwd_alone<T, HL>(), BWD_LANES);
     const int64_t nwg = p.nwg;
     if (nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
     if (dm.es == 3 && dm.keep_out)
@@ -577,8 +581,8 @@ size_t window_bwd_workspace(const Dims &dm)
     int64_t n = 0;
     for (int v : {1, 2, BWD_V}) {
         if (dm.d % v) continue;
-        for (double alone : {ALONE, BWD_ONE_WAVE}) {
-            if (alone != ALONE && v != BWD_V) continue;         // (separate tensors alone have the second figure)
+        // (separate tensors have 4 channels per lane and either of two figures)
+        for (double alone : {il_bwd_alone(v), v == BWD_V ? BWD_ONE_WAVE : il_bwd_alone(v)}) {
             const WinPlan p = plan(dm, v, BWD_ROWS, alone, BWD_LANES);
             if (p.nthreads > n) n = p.nthreads;
         }
