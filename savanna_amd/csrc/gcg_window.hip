@@ -436,7 +436,9 @@ constexpr double il_bwd_alone(int v) { return v == 1 ? BWD_ONE_CHANNEL : ALONE; 
 
 // How the forward walks.  Runs of at most 128 rows in XCD-contiguous order, except:
 // - rows of a multiple of 8 KB (but separate fp32 operands): long runs in plain order (1 x 32768 x 8192 bf16 377 us, short runs
-//   in XCD order 411; 2 x 8192 x 4096 fp32 interleaved 183, in XCD order 187);
+//   in XCD order 411; 2 x 8192 x 4096 fp32 interleaved 183, in XCD order 187), and beyond the last-level cache interleaved 16-bit
+//   rows whose bytes are a power of two from 2 KB on (1 x 32768 x 2048 97 us, in runs of 16 107; 2 x 65536 x 1024 198 and 204;
+//   3 KB and 6 KB rows are as fast or faster in runs of 16, 2 x 21845 x 3072 236 and 204);
 // - operands and result beyond the last-level cache, with rows off the 128-byte lines (but separate fp32 operands) or
 //   interleaved in 16 bits: 16 rows in plain order without the streaming hint, so that the neighbours of a line run at once and
 //   its parts meet in the L2 (1 x 264208 x 2032 bf16 1415 -> 850 us, 2 x 20000 x 2400 152 against 167 in the common form,
@@ -459,8 +461,9 @@ template <typename T> FwdForm fwd_form(const Dims &dm)
     const bool big = 4 * (double)dm.bs * (double)dm.L * (double)row > 256.0 * 1024 * 1024;
     if (es == 4 && dm.es == 1) return big && row % 16384 == 0 ? FwdForm{128, false, true, 2.0} : FwdForm{96, false, true, 2.5};
     const double alone = f16 && dm.es == 1 ? 1.75 : ALONE;
-    if (row % 8192 == 0) return FwdForm{1024, false, false, alone};
-    if (big && (row % 128 != 0 || (dm.es == 3 && es == 2))) return FwdForm{16, true, false, alone};
+    const bool packed = dm.es == 3 && es == 2;
+    if (row % 8192 == 0 || (big && packed && row >= 2048 && (row & (row - 1)) == 0)) return FwdForm{1024, false, false, alone};
+    if (big && (row % 128 != 0 || packed)) return FwdForm{16, true, false, alone};
     return FwdForm{128, false, true, alone};
 }
 

@@ -85,7 +85,7 @@ def test_register_window_kernels(dtype, arith, bs, L, g, wide, planar):
 # layout, tensors' and filter's type, groups, taps, sequences
 BEYOND = [("separate", "bfloat16", "bfloat16", 29, 7, 1), ("separate", "bfloat16", "float32", 29, 3, 2),
           ("separate", "float16", "float16", 27, 8, 1), ("separate", "float32", "float32", 31, 7, 1),
-          ("separate", "float32", "float32", 256, 4, 2),
+          ("separate", "float32", "float32", 256, 4, 2), ("interleaved", "float16", "float16", 64, 7, 2),
           ("extra", "bfloat16", "bfloat16", 29, 7, 2), ("extra", "float16", "float32", 27, 4, 1), ("extra", "float32", "float32", 31, 7, 1),
           ("interleaved", "float16", "float16", 61, 7, 1), ("interleaved", "bfloat16", "bfloat16", 28, 8, 2),
           ("interleaved", "float32", "float32", 30, 7, 1), ("interleaved", "float32", "float32", 31, 3, 2),
