@@ -217,7 +217,9 @@ int lane_width(int dtype, const Dims &dm)
 // Forward: the longest runs of a power of two that give two workgroups per CU (the other plan: 119 against 127 us at
 // 1 x 12000 x 12288 bf16), up to 128 rows where a row is a multiple of 8 KB (2 x 8192 x 12288 bf16 154 us, with 64 rows 165),
 // else 64, so that the rows in flight lie closer together (1 x 12000 x 12144 bf16 141 -> 134 us, 3 x 17810 x 7536 378 -> 366,
-// 1 x 6000 x 12192 fp32 127 -> 121).  Backward: plan_runs (187 -> 178 us there, 12144 channels 219 -> 210).
+// 1 x 6000 x 12192 fp32 127 -> 121).  Both sides of that line, bf16, 128 rows and 64: multiples of 8 KB, 8192 channels 161 and
+// 167 us, 12288 171 and 174; others, 8128 175 and 163, 10240 172 and 167, 14336 193 and 178, 18432 192 and 178; a multiple of 32 KB is
+// ahead with 64 (16384 channels 172 and 155).  Backward: plan_runs (187 -> 178 us there, 12144 channels 219 -> 210).
 DwPlan plan(const Dims &dm, int V, int longest, bool backward)
 {
     DwPlan p;
@@ -238,12 +240,21 @@ DwPlan plan(const Dims &dm, int V, int longest, bool backward)
     return p;
 }
 
-// Rows that start and end on odd 32-byte sectors: the forward's accesses go without the streaming hint, and the parts of a
-// shared 64 bytes meet in the L2 (followed by the operator, 3 x 17810 x 7536 bf16 645 -> 620 us, planar 8 x 3021 x 16656
-// 630 -> 590; 1 x 12000 x 12144 199 -> 204; rows of whole lines 154 -> 165 alone).  The backward keeps it: alone it gained
-// 600 -> 582 us without, behind the operator's backward, whose gradient is partly in the cache then, it lost 960 -> 971, and
-// in fp32 arithmetic at 1 x 12000 x 12144 344 -> 365.
-template <typename T> bool ragged(const Dims &dm) { return (uint64_t)dm.d * sizeof(T) % 64 != 0; }
+// Rows off the 64-byte boundaries: the forward's accesses go without the streaming hint, and the parts of a shared 64 bytes meet in
+// the L2 (2 x 9000 x 2928 bf16 58 -> 43 us, 1 x 6000 x 12144 77 -> 67; followed by the operator, 3 x 17810 x 7536 660 -> 624, planar
+// 8 x 3021 x 16656 700 -> 595; rows of whole lines 154 -> 165 alone).  Not where y is kept for the operator (keep_out) and x
+// would take its place in the last-level cache, which the two of them overflow but not by much (followed by the operator, 1 x
+// 20160 x 5520 169 us with the hint and 183 without, 1 x 152118 x 1104 301 and 321, 1 x 12000 x 12144 209 and 218, 1 x 40000 x
+// 6096 364 and 365, 1 x 6000 x 12144 109 and 108).  The backward keeps the hint: alone it gained 600 -> 582 us without, behind the
+// operator's backward, whose gradient is partly in the cache then, it lost 960 -> 971, and in fp32 arithmetic at 1 x 12000 x
+// 12144 344 -> 365.
+template <typename T> bool fwd_plain(const Dims &dm)
+{
+    constexpr double CACHE = 256.0 * 1024 * 1024;
+    const double bytes = (double)dm.bs * (double)dm.L * (double)dm.d * sizeof(T);       // of x, and of y
+    if (dm.keep_out && bytes > CACHE / 2 && bytes <= 2 * CACHE) return false;
+    return (uint64_t)dm.d * sizeof(T) % 64 != 0;
+}
 
 template <typename T, int HL, int V, bool PCF>
 int fwd_launch(const void *x, const void *w, void *y, const Dims &dm, hipStream_t st)
@@ -252,7 +263,7 @@ int fwd_launch(const void *x, const void *w, void *y, const Dims &dm, hipStream_
     DwPlan p = plan(dm, V, (uint64_t)dm.d * sizeof(T) % 8192 == 0 ? 128 : 64, false);
     if (!launch_holds(p.nwg, p.threads)) p = plan(dm, V, 128, false);
     if (p.nwg > 0x7fffffffLL) return (int)hipErrorInvalidConfiguration;
-    if (ragged<T>(dm))
+    if (fwd_plain<T>(dm))
         e = launch_plain((dwconv_fwd_kernel<T, HL, V, PCF, true, true>), dim3((unsigned)p.nwg), dim3(p.threads), st,
                            (const T *)x, (const T *)w, (T *)y, dm, p);
     else if (dm.keep_out)

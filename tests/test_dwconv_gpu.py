@@ -180,3 +180,15 @@ def test_keep_output_changes_the_cache_policy_not_the_values(gcg_lib, dtype):
     lib = _lib.load()
     p = x.data_ptr()
     assert lib.gcg_dwconv_fwd(p, p, p, 1, 64, 16, 1, 3, 0, 2, None) == -1        # unknown flag
+
+
+def test_kept_output_about_the_size_of_the_cache():
+    """Rows off the 64-byte boundaries whose output is kept: with the streaming hint between half and twice the cache, without it
+    below and above.  Same values on every path."""
+    w = torch.randn(912, 1, 3, device=DEV).to(torch.bfloat16)
+    for L in (70000, 80000, 290000, 300000):                            # 122, 139, 504 and 522 MiB
+        x = torch.empty(1, L, 912, 1, device=DEV, dtype=torch.bfloat16).normal_()
+        y = _lib.dwconv_fwd(x, w, True)
+        assert torch.equal(y, _lib.dwconv_fwd(x, w, False))
+        first = L - 3000
+        assert torch.equal(y[:, first:], _lib.dwconv_fwd(x[:, first - 2:].clone(), w)[:, 2:])
