@@ -78,8 +78,10 @@ def test_transforms_and_dual_numbers_take_the_python_functions():
         dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
         with pytest.raises(NotImplementedError, match="jvp"):
             f(dual, *xs[1:])
-    with pytest.raises(RuntimeError):
+    # (the C++ node would not refuse: vmap runs an operator without a batching rule sample by sample)
+    with pytest.raises(RuntimeError, match="setup_context"):
         torch.func.vmap(lambda t: f(t, *(p.detach() for p in xs[1:])))(x[None])
+    assert not torch.func.vmap(lambda t: t.new_full((), float(_lib.native_nodes(t))))(x[None]).any() and _lib.native_nodes(x)
 
 
 def test_refusals_are_those_of_the_python_function():
