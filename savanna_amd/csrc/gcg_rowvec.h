@@ -43,10 +43,6 @@ template <int AUX> __device__ __forceinline__ void load_piece_aux(win_t w, uint3
     const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(w, (int)off, 0, AUX);
     p[0][0] = v[0]; p[1][0] = v[1]; p[2][0] = v[2];
 }
-template <int AUX> __device__ __forceinline__ void store_piece_aux(win_t w, uint32_t off, const u32x1 (&p)[3])
-{
-    __builtin_amdgcn_raw_buffer_store_b96(u32x3{p[0][0], p[1][0], p[2][0]}, w, (int)off, 0, AUX);
-}
 template <typename R> __device__ __forceinline__ void load_piece(win_t w, uint32_t off, R (&p)[3])
 {
     constexpr int NB = sizeof(R);

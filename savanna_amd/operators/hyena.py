@@ -26,8 +26,8 @@ import torch
 import torch.nn as nn
 
 from .. import _lib
-from ..kernels.cgcg.interface import (DecayedGateConvGate, InterleavedDecayedGateConvGate,  # noqa: F401
-                                       decayed_gate_conv_gate, planar_source, two_pass_chunked_gate_conv_gate,
+from ..kernels.cgcg.interface import (InterleavedDecayedGateConvGate, decayed_gate_conv_gate, planar_source,
+                                       two_pass_chunked_gate_conv_gate,
                                        two_pass_chunked_gate_conv_gate_interleaved,
                                        two_pass_chunked_gate_conv_gate_planar)
 from ..kernels.cgcg.src.kernel_utils import BwdKernelConfigRefactor, FwdKernelConfigRefactor
