@@ -861,7 +861,7 @@ MixPlan plan(const Dims &dm, int ch, bool backward)
 
 int lane_channels(int dtype) { return dtype == GCG_F32 ? 1 : 2; }
 
-// 16-bit rows that start and end on odd 32-byte sectors are accessed without the streaming hint: the parts of a shared 64 bytes
+// 16-bit rows off the 64-byte boundaries are accessed without the streaming hint: the parts of a shared 64 bytes
 // then meet in the L2 instead of being written one by one (3 x 17810 x 2512: forward 265 -> 239 us and 297 -> 247 planar,
 // backward 438 -> 423 and 531 -> 451; rows of whole or half lines are as fast or faster with it).
 bool ragged(const Dims &dm) { return (uint64_t)dm.d * 2 % 64 != 0; }

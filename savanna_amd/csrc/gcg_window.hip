@@ -213,8 +213,7 @@ __global__ __launch_bounds__(256) void window_bwd_kernel(const T *__restrict__ d
 {
     typedef typename Vec<T, V>::raw raw_t;
     constexpr int ES = sizeof(T), IS = PK ? 3 : 1;
-    // workgroups of one XCD take adjacent channel blocks of the same rows (measured +3-5 % in the
-    // backward kernels, -3 % in the forward ones, which keep the plain order)
+    // workgroups of one XCD take adjacent channel blocks of the same rows (measured +3-5 %; the forward's order is fwd_form's)
     int64_t wg = xcd_contiguous_id(blockIdx.x, gridDim.x);
     const int cvb = (int)(wg % pl.ncvb); wg /= pl.ncvb;
     const int seg = (int)(wg % pl.nseg);
@@ -416,10 +415,12 @@ constexpr int BWD_ROWS = 1024;
 constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(float));
 
 // What a plan counts for a wave that has its SIMD to itself (plan_runs), by what that costs in each kernel.  The backward of
-// separate fp32 operands, and of f16 ones beyond four taps, holds over 256 registers: its waves run one at a time whatever
+// separate f16 operands beyond four taps, and of fp32 ones there, holds over 256 registers: its waves run one at a time whatever
 // the plan, and a second round only adds its halo (2 x 4000 x 2880 f16 85 -> 78 us, 1 x 30000 x 480 72 -> 62, 2 x 1896 x 2880
-// fp32 79 -> 70; the others lose 5 - 15 % with that figure: 1 x 14000 x 272, 3 taps, f16 36 -> 42, 1 x 9000 x 1152 bf16
-// 47 -> 56).  The 4 % are for long runs, where that halo is little and two rounds are ahead (2 x 8192 x 4096 fp32 361 and 366 us).
+// fp32 79 -> 70).  fp32 with at most four taps has room for two (184 registers), but its 16-byte rows keep memory busy from one: 3
+// taps, 2 x 3000 x 1600 65 us, with 1.3 69, 4 x 1500 x 1600 64 and 69, 2 x 4000 x 2880 137 and 147, 8 x 700 x 2048 73 and 74,
+// 2 x 8192 x 4096 357 and 356.  The others lose 5 - 15 % with that figure (1 x 14000 x 272, 3 taps, f16 36 -> 42, 1 x 9000 x 1152
+// bf16 47 -> 56).  The 4 % are for long runs, where that halo is little and two rounds are ahead (2 x 8192 x 4096 fp32 361 and 366).
 // Interleaved fp32 operands: a lane has one channel, 12 bytes a row, and one wave's rows in flight do not keep memory busy where
 // the second would (1 x 7443 x 2944 140 -> 124 us, 4 x 1500 x 1600 70 -> 63, 3 x 218 x 3632 30 -> 27.8, 1 x 3184 x 752 30 -> 27; over
 // 104 sizes 1 % less time, and half as many that lose to runs of a power of two).
