@@ -240,8 +240,8 @@ DwPlan plan(const Dims &dm, int V, int longest, bool backward)
     return p;
 }
 
-// Rows off the 64-byte boundaries: the forward's accesses go without the streaming hint, and the parts of a shared 64 bytes meet in
-// the L2 (2 x 9000 x 2928 bf16 58 -> 43 us, 1 x 6000 x 12144 77 -> 67; followed by the operator, 3 x 17810 x 7536 660 -> 624, planar
+// Rows off the 64-byte boundaries: the forward's accesses go without the streaming hint, so that a line whose other part a neighbour
+// reads is found in the L2 (3 x 17810 x 7536 bf16: 5 % fewer reads from HBM, writes the same; 2 x 9000 x 2928 bf16 58 -> 43 us, 1 x 6000 x 12144 77 -> 67; followed by the operator, 3 x 17810 x 7536 660 -> 624, planar
 // 8 x 3021 x 16656 700 -> 595; rows of whole lines 154 -> 165 alone).  Not where y is kept for the operator (keep_out) and x
 // would take its place in the last-level cache, which the two of them overflow but not by much (followed by the operator, 1 x
 // 20160 x 5520 169 us with the hint and 183 without, 1 x 152118 x 1104 301 and 321, 1 x 12000 x 12144 209 and 218, 1 x 40000 x

@@ -442,7 +442,7 @@ constexpr double il_bwd_alone(int v) { return v == 1 ? BWD_ONE_CHANNEL : ALONE; 
 //   3 KB and 6 KB rows are as fast or faster in runs of 16, 2 x 21845 x 3072 236 and 204);
 // - operands and result beyond the last-level cache, with rows off the 128-byte lines (but separate fp32 operands) or
 //   interleaved in 16 bits: 16 rows in plain order without the streaming hint, so that the neighbours of a line run at once and
-//   its parts meet in the L2 (1 x 264208 x 2032 bf16 1415 -> 850 us, 2 x 20000 x 2400 152 against 167 in the common form,
+//   its parts meet in the L2 (1 x 30000 x 2032: half as many writes of 32 bytes, for 12 % more reads, the runs' halos; 1 x 264208 x 2032 bf16 1415 -> 850 us, 2 x 20000 x 2400 152 against 167 in the common form,
 //   interleaved 149 and 168, 1 x 38836 x 3456 interleaved 197 and 213, fp32 interleaved 1 x 30000 x 2032 190 and 207,
 //   2 x 20000 x 1200 157 and 167; in the cache the common form is ahead: 2 x 9000 x 1456 47 and 49, 3 x 5000 x 1440 40 and 43,
 //   interleaved 2 x 4000 x 2880 37 and 41).  With y2 and Bx written as well 1 x 30000 x 2032 169 us, in the common form 195, in
