@@ -414,26 +414,30 @@ WinPlan plan(const Dims &dm, int v, int longest, double alone, int64_t most_lane
 constexpr int BWD_ROWS = 1024;
 constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(float));
 
-// What a plan counts for a wave that has its SIMD to itself (plan_runs), by what that costs in each kernel.  The backward of
-// separate f16 operands beyond four taps, and of fp32 ones there, holds over 256 registers: its waves run one at a time whatever
-// the plan, and a second round only adds its halo (2 x 4000 x 2880 f16 85 -> 78 us, 1 x 30000 x 480 72 -> 62, 2 x 1896 x 2880
-// fp32 79 -> 70).  fp32 with at most four taps has room for two (184 registers), but its 16-byte rows keep memory busy from one: 3
-// taps, 2 x 3000 x 1600 65 us, with 1.3 69, 4 x 1500 x 1600 64 and 69, 2 x 4000 x 2880 137 and 147, 8 x 700 x 2048 73 and 74,
-// 2 x 8192 x 4096 357 and 356.  The others lose 5 - 15 % with that figure (1 x 14000 x 272, 3 taps, f16 36 -> 42, 1 x 9000 x 1152
-// bf16 47 -> 56).  The 4 % are for long runs, where that halo is little and two rounds are ahead (2 x 8192 x 4096 fp32 361 and 366).
-// Interleaved fp32 operands: a lane has one channel, 12 bytes a row, and one wave's rows in flight do not keep memory busy where
-// the second would (1 x 7443 x 2944 140 -> 124 us, 4 x 1500 x 1600 70 -> 63, 3 x 218 x 3632 30 -> 27.8, 1 x 3184 x 752 30 -> 27; over
-// 104 sizes 1 % less time, and half as many that lose to runs of a power of two).
-constexpr double ALONE = 1.3, BWD_ONE_WAVE = 1.04, BWD_ONE_CHANNEL = 2.0;
+// What a plan counts for a wave that has its SIMD to itself (plan_runs), by what that costs in each kernel.
+// - Two waves: separate bf16 operands, and f16 ones with at most four taps (119 - 173 registers, room for two waves and more).  7 taps,
+//   1 x 17787 x 368 46 us, with 1.3 55, 3 x 3181 x 832 44 and 50, 1 x 2064 x 4128 44 and 48 (runs of a power of two 46); 4 taps,
+//   8 x 609 x 1088 f16 35 and 39, 1 x 2216 x 3952 46 and 50; over 160 sizes 2 % less time, and 2.5 is no better.
+//   Interleaved fp32 operands, whose lanes have one channel, 12 bytes a row: one wave's rows in flight do not keep memory busy where
+//   the second would (1 x 7443 x 2944 140 -> 121 us, 4 x 1500 x 1600 70 -> 63, 3 x 218 x 3632 30 -> 27.8, 1 x 3184 x 752 30 -> 27; over
+//   104 sizes 1 % less time, and half as many that lose to runs of a power of two).
+// - One: separate f16 operands beyond four taps, and fp32 ones there, hold over 256 registers: their waves run one at a time whatever
+//   the plan, and a second round only adds its halo (2 x 4000 x 2880 f16 85 -> 78 us, 1 x 30000 x 480 72 -> 62, 2 x 1896 x 2880
+//   fp32 79 -> 70).  fp32 with at most four taps has room for two (184 registers), but its 16-byte rows keep memory busy from one: 3
+//   taps, 2 x 3000 x 1600 65 us, with 1.3 69, 4 x 1500 x 1600 64 and 69, 2 x 4000 x 2880 137 and 147, 8 x 700 x 2048 73 and 74,
+//   2 x 8192 x 4096 357 and 356.  The 4 % are for long runs, where that halo is little and two rounds are ahead (2 x 8192 x 4096
+//   fp32 361 and 366).
+// - 1.3: interleaved 16-bit operands (over 72 sizes 1.3 and 1.6 alike, 2 1 % behind).
+constexpr double ALONE = 1.3, BWD_ONE_WAVE = 1.04, BWD_TWO_WAVES = 2.0;
 template <typename T, int HL> constexpr double bwd_alone()
 {
-    return std::is_same_v<T, float> || (HL > 4 && (std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t>)) ? BWD_ONE_WAVE : ALONE;
+    return std::is_same_v<T, float> || (HL > 4 && (std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t>)) ? BWD_ONE_WAVE : BWD_TWO_WAVES;
 }
 
 constexpr int BWD_V = 4;   // the backward keeps four rings per lane: 4 channels is what fits
 // interleaved operands: the lane width that makes a row piece 12 contiguous bytes
 template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
-constexpr double il_bwd_alone(int v) { return v == 1 ? BWD_ONE_CHANNEL : ALONE; }
+constexpr double il_bwd_alone(int v) { return v == 1 ? BWD_TWO_WAVES : ALONE; }
 
 // How the forward walks.  Runs of at most 128 rows in XCD-contiguous order, except:
 // - rows of a multiple of 8 KB (but separate fp32 operands): long runs in plain order (1 x 32768 x 8192 bf16 377 us, short runs
@@ -586,7 +590,7 @@ size_t window_bwd_workspace(const Dims &dm)
     for (int v : {1, 2, BWD_V}) {
         if (dm.d % v) continue;
         // (separate tensors have 4 channels per lane and either of two figures)
-        for (double alone : {il_bwd_alone(v), v == BWD_V ? BWD_ONE_WAVE : il_bwd_alone(v)}) {
+        for (double alone : {v == BWD_V ? BWD_TWO_WAVES : il_bwd_alone(v), v == BWD_V ? BWD_ONE_WAVE : il_bwd_alone(v)}) {
             const WinPlan p = plan(dm, v, BWD_ROWS, alone, BWD_LANES);
             if (p.nthreads > n) n = p.nthreads;
         }
