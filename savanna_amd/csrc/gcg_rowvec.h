@@ -113,6 +113,10 @@ template <typename T, int VV> __device__ __forceinline__ typename Vec<T, VV>::ra
 // product over the 256 CUs of four SIMDs (streams: the kernel waits for memory, and three waves on four SIMDs count as that;
 // 8192 x 16 x 768 time-major, backward, 1.5 waves of 256 rows 293 us, 3 of 128 302); fewer than `alone` waves per SIMD count as
 // that many, since nothing hides their waits (a factor on one wave alone: 3 x 3000 x 640 f16 forward 20 us, so 15 - 16).
+// by_fullest (separate operands' backward): rows of whole three-wave workgroups hide them where the fullest SIMD does, two waves at
+// 1.5 on average (8192 x 16 x 768 time-major 294 -> 289 us, 1 x 20032 x 640 bf16 73 -> 56, 3 x 2058 x 2176 66 -> 54, 4 x 2380 x 1472 71 -> 55,
+// but 8 x 429 x 3776 48 -> 52, and 4 x 43786 x 576, with a quarter of all lanes idle, 306 -> 334; over 50 sizes 1 % less
+// time).  With whole waves idle it loses 1 - 6 % (1 x 2064 x 4128 40 -> 42), in forwards 5 % (1 x 5880 x 768 f16 9.4 -> 11.3).
 // Runs are multiples of `unit` and at most `longest` rows; workgroups of four waves unless fewer leave less idle.  No more than
 // most_lanes lanes have work, unless even the longest runs need more (lanes leave partial sums behind).
 // (Against runs of a power of two that fill two workgroups per CU at least: mixer 3 x 17810 x 2512 bf16 backward 545 -> 435 us,
@@ -120,7 +124,7 @@ template <typename T, int VV> __device__ __forceinline__ typename Vec<T, VV>::ra
 // 3 x 20000 x 800 fp32 291 -> 255, 4 x 7000 x 2400 f16 240 -> 211; widths that are powers of two keep their plans.)
 struct RunPlan { int waves, ncvb, ts; };
 inline RunPlan plan_runs(int64_t bs, int64_t L, int64_t nvec, int unit, int longest, int extra, double alone,
-                         int64_t most_lanes, bool streams)
+                         int64_t most_lanes, bool streams, bool by_fullest = false)
 {
     RunPlan best{0, 0, 0};
     double least = 0;
@@ -135,8 +139,9 @@ inline RunPlan plan_runs(int64_t bs, int64_t L, int64_t nvec, int unit, int long
             const int64_t runs = (L + ts - 1) / ts;
             if (ts > longest || bs * runs * nvec > most_lanes) continue;
             const int64_t per_cu = (per * runs + 255) / 256;
-            const double per_simd = k == 3 && streams ? 0.75 * (double)per_cu : (double)((per_cu * k + 3) / 4);
-            const double cost = (per_simd < alone ? alone : per_simd) * (double)(ts + extra);
+            const double fullest = (double)((per_cu * k + 3) / 4), per_simd = k == 3 && streams ? 0.75 * (double)per_cu : fullest;
+            const double hidden = by_fullest && nw % 3 == 0 ? fullest : per_simd;
+            const double cost = (hidden < alone ? alone : per_simd) * (double)(ts + extra);
             if (best.waves == 0 || cost < least * (k == best.waves ? 1.0 : 0.97)) { best = RunPlan{k, (int)ncvb, (int)ts}; least = cost; }
             if (ts == unit) break;
         }

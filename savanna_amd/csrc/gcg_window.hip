@@ -390,12 +390,18 @@ __global__ __launch_bounds__(256) void window_bwd_kernel(const T *__restrict__ d
         if (j < hl) slot[(size_t)(hl - 1 - j) * pl.nthreads] = dha[j];
 }
 
+// the longest runs of the backward: up to 1024 rows, measured best at the 7B and 40B shapes for either operand layout (fewer
+// halo rows and filter-gradient partials).  Lanes: eight filter-gradient partials of each fill the static scratch.
+constexpr int BWD_ROWS = 1024;
+constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(float));
+constexpr int BWD_V = 4;   // the backward keeps four rings per lane: 4 channels is what fits
+
 WinPlan plan(const Dims &dm, int v, int longest, double alone, int64_t most_lanes)
 {
     WinPlan p;
     p.v = v;
     p.nvec = (int)(dm.d / v);
-    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, alone, most_lanes, true);
+    const RunPlan r = plan_runs(dm.bs, dm.L, p.nvec, RING, longest, RING, alone, most_lanes, true, most_lanes == BWD_LANES && v == BWD_V);
     p.ts = r.ts;
     static const char *env = tuning_env("GCG_WINDOW_ROWS");   // tuning override: rows per lane, a multiple of 8
     if (env && atoi(env) >= 8 && atoi(env) % 8 == 0) p.ts = atoi(env);
@@ -409,10 +415,6 @@ WinPlan plan(const Dims &dm, int v, int longest, double alone, int64_t most_lane
     p.nwg = dm.bs * p.nseg * p.ncvb;
     return p;
 }
-// the longest runs of the backward: up to 1024 rows, measured best at the 7B and 40B shapes for either operand layout (fewer
-// halo rows and filter-gradient partials).  Lanes: eight filter-gradient partials of each fill the static scratch.
-constexpr int BWD_ROWS = 1024;
-constexpr int64_t BWD_LANES = GCG_BWD_STATIC_SCRATCH_BYTES / (RING * sizeof(float));
 
 // What a plan counts for a wave that has its SIMD to itself (plan_runs), by what that costs in each kernel.
 // - Two waves: separate bf16 operands, and f16 ones with at most four taps (119 - 173 registers, room for two waves and more).  7 taps,
@@ -434,7 +436,6 @@ template <typename T, int HL> constexpr double bwd_alone()
     return std::is_same_v<T, float> || (HL > 4 && (std::is_same_v<T, f16_t> || std::is_same_v<T, f16w_t>)) ? BWD_ONE_WAVE : BWD_TWO_WAVES;
 }
 
-constexpr int BWD_V = 4;   // the backward keeps four rings per lane: 4 channels is what fits
 // interleaved operands: the lane width that makes a row piece 12 contiguous bytes
 template <typename T> constexpr int il_v() { return 4 / (int)sizeof(T); }
 constexpr double il_bwd_alone(int v) { return v == 1 ? BWD_TWO_WAVES : ALONE; }
